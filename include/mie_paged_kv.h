@@ -17,6 +17,7 @@
  *   mie_moe_route     <- fused_moe.route         src/moe_engine/fused_moe.py:274-309
  *   mie_moe_decode    <- fused_moe.decode        src/moe_engine/fused_moe.py:312-380
  *   mie_moe_decode_block <- the block's x + moe(moe_norm(x)) for one token  src/moe_engine/model.py:496-497
+ *   mie_moe_prefill   <- MoEFeedForward.forward over a prompt  src/moe_engine/model.py:443-461
  *   mie_argmax        <- Model.generate's greedy torch.argmax   src/moe_engine/model.py:603
  *   mie_lm_head       <- final_norm + output_projection (model.py:564-565) and,
  *                        optionally, the greedy argmax (:603) for one token
@@ -357,6 +358,25 @@ int32_t mie_moe_decode_block(const void* x, const void* ln_weight, const void* l
                              int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden,
                              void* router_logits, void* expert_ids, void* route_weights,
                              void* hidden_act, void* out, int32_t dtype, void* stream);
+
+/*
+ * The MoE layer over `tokens` tokens (MoEFeedForward.forward on a prompt,
+ * model.py:443-461): routing as in mie_moe_route, then for each token the sum
+ * over its top_k experts in increasing expert id of
+ * round(w * (W2_e GELU(W1_e x + b1_e) + b2_e)), with mie_moe_decode's dtypes
+ * and rounding points.  x and out [tokens, dim], the weights in canonical
+ * layouts as for mie_moe_decode, all 16-byte aligned; dim and hidden multiples
+ * of 4 (float32) or 8 (bfloat16), at most 64 experts and top_k 8.  out must
+ * not alias x.  Only experts that a token selected are read.  workspace holds
+ * mie_moe_prefill_workspace bytes (negative: the shape is not supported);
+ * nothing in it needs clearing.  Four launches per 4096 tokens.
+ */
+int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden,
+                                  int32_t dtype);
+int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* router_weight, const void* w1, const void* b1,
+                        const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim,
+                        int32_t hidden, void* out, void* workspace, int64_t workspace_bytes, int32_t dtype,
+                        void* stream);
 
 /*
  * Greedy pick (Model.generate at temperature 0, model.py:603): the index

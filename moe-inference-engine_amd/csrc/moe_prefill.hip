@@ -1,0 +1,472 @@
+// Top-k mixture-of-experts over a prompt (float32 or bfloat16): routing, the
+// selected experts' products and the weighted sum, with no host sync.
+//
+// Replaces, for several tokens, the reference's PyTorch MoE path
+// (src/moe_engine/model.py:443-461), whose per-expert torch.where makes the
+// host wait for the device once per expert:
+//
+//   logits = W_r x_t                     (float32)
+//   ids    = the top_k experts by logit  (lower id on ties), w = their softmax
+//   y_te   = W2_e GELU(W1_e x_t + b1_e) + b2_e         for the selected experts
+//   out_t  = sum over them in increasing expert id, from 0, of round(w y)
+//
+// Rounding points are the one-token kernels' (moe_decode.hip): every sum is
+// float32; in bfloat16 each Linear's output, GELU's, the route weight, the
+// product and each partial sum are rounded, as the PyTorch path stores them.
+//
+// Four launches.
+//   1. moe_prompt_route: two tokens per wave; the selected experts and weights
+//      per token, and per expert a bit mask over the tokens (one byte per
+//      workgroup of 8 tokens), so no workgroup needs another's counts.
+//   2. moe_prompt_w1: h[slot] = GELU(W1_e x_t + b1_e).  Slots are the (expert,
+//      token) pairs, expert by expert; each workgroup finds its expert and its
+//      rows in the masks by popcounts.
+//   3. moe_prompt_w2: partial sums of W2_e h over one K split.
+//   4. moe_prompt_combine: the splits' sum, bias, weight and expert-order sum.
+// The work follows the routing: top_k / E of what running every expert on
+// every token takes, at any skew, and an expert without tokens is not read.
+//
+// Bounds: at few tokens the experts' bytes (768 x 2048 x 8 float32: 101 MB),
+// at many the matrix cores (float32: 153 TFLOP/s).  A whole layer on MI355X,
+// 8 experts, top-2, before (dense-masked library products up to 512 float32
+// tokens, the per-expert PyTorch path otherwise) and with these launches:
+// 32 tokens, FFN 2048, float32: 228 -> 47 us; 1000 tokens, FFN 3072, float32:
+// 1131 -> 229 us; 512 tokens, FFN 2048, bfloat16: 1140 -> 52 us.
+#include <math.h>
+
+#include <algorithm>
+
+#include "gemm_tile.h"
+#include "mie_common.h"
+#include "moe_route.h"
+
+namespace {
+
+using namespace mie::route;
+using mie::Mem;
+using mie::gemm::f32x4;
+
+constexpr int kChunk = 4096;      // tokens per set of launches: 64 mask words per expert, one per lane
+constexpr int kRouteTokens = 8;   // tokens per routing workgroup: one mask byte per expert
+constexpr int kMaxSplits = 8;
+
+struct PromptArgs {
+  const char* x;       // T [tokens, dim]
+  const char* router;  // T [E, dim]
+  const char* w1;      // T [E, hidden, dim]
+  const char* b1;      // T [E, hidden]
+  const char* w2;      // T [E, dim, hidden]
+  const char* b2;      // T [E, dim]
+  int32_t tokens, E, top_k, dim, hidden;
+  int32_t words;              // mask words per expert: ceil(tokens / 64)
+  int32_t per_expert;         // 1: blockIdx.y is an expert; 0: the y-th row tile of all experts
+  int32_t splits, split_len;  // W2: K splits and bytes of a row per split
+  unsigned long long* masks;  // [E, words]
+  int32_t* counts;            // [E] tokens per expert
+  int32_t* ids;               // [tokens, top_k], increasing
+  float* weights;             // [tokens, top_k], the same order
+  int32_t* slots;             // [tokens, top_k], the same order
+  char* h;                    // T [tokens * top_k, hidden]
+  float* part;                // [splits, tokens * top_k, dim]
+  char* out;                  // T [tokens, dim]
+};
+
+// grid = words * 8; four waves, two tokens each.
+template <typename T>
+__global__ __launch_bounds__(256) void moe_prompt_route(PromptArgs a) {
+  __shared__ unsigned int s_mask[kMaxExperts];
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < kMaxExperts) s_mask[threadIdx.x] = 0u;
+  __syncthreads();
+  const int t0 = blockIdx.x * kRouteTokens + wave * 2;
+  if (t0 < a.tokens) {
+    const bool two = t0 + 1 < a.tokens;
+    const T* x0 = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(t0) * a.dim;
+    const T* x1 = two ? x0 + a.dim : x0;
+    const T* router = reinterpret_cast<const T*>(a.router);
+    float l0 = -INFINITY, l1 = -INFINITY;  // lane e: expert e's logit
+    // Four experts' rows at a time, so their loads and the tokens' go out together.
+    for (int e = 0; e < a.E; e += 4) {
+      float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int i = lane * 4; i < a.dim; i += 256) {
+        const f32x4_t v0 = Mem<T>::load4(x0 + i), v1 = Mem<T>::load4(x1 + i);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const f32x4_t r = Mem<T>::load4(router + static_cast<int64_t>(min(e + u, a.E - 1)) * a.dim + i);
+          s0[u] = dot4(r, v0, s0[u]);
+          s1[u] = dot4(r, v1, s1[u]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float d0 = mie::wave_sum(s0[u]), d1 = mie::wave_sum(s1[u]);
+        if (lane == e + u && e + u < a.E) {
+          l0 = d0;
+          l1 = d1;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (j == 1 && !two) break;
+      int ids[kMaxTopK];
+      float p[kMaxTopK];
+      wave_topk(j ? l1 : l0, a.top_k, a.E, lane, ids, p);
+#pragma unroll
+      for (int kk = 0; kk < kMaxTopK; ++kk) {
+        int rank = 0;  // place in increasing expert id (ids are distinct)
+#pragma unroll
+        for (int o = 0; o < kMaxTopK; ++o) rank += o < a.top_k && ids[o] < ids[kk];
+        if (kk < a.top_k && lane == kk) {
+          const int64_t at = static_cast<int64_t>(t0 + j) * a.top_k + rank;
+          a.ids[at] = ids[kk];
+          a.weights[at] = p[kk];
+          atomicOr(&s_mask[ids[kk]], 1u << (wave * 2 + j));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // Every byte of every word is written, also past the last token.
+  if (threadIdx.x < a.E)
+    reinterpret_cast<uint8_t*>(a.masks + static_cast<int64_t>(threadIdx.x) * a.words)[blockIdx.x] =
+        static_cast<uint8_t>(s_mask[threadIdx.x]);
+}
+
+__device__ __forceinline__ int wave_inclusive(int v, int lane) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(v, off);
+    v += lane >= off ? o : 0;
+  }
+  return v;
+}
+
+// The rows a workgroup works on: expert e's rows [m0, count) (only the first
+// BM of them in the row-tile form), the expert's first slot.
+struct Rows {
+  int e, m0, count, base;
+};
+
+// blockIdx.y's rows from the experts' token counts (lane e: expert e's).
+// Uniform over the workgroup; e < 0 when there are none.
+__device__ __forceinline__ Rows find_rows(const PromptArgs& a, int cnt, int bm, int lane) {
+  const int tiles = (cnt + bm - 1) / bm;
+  const int incl = wave_inclusive(cnt, lane);
+  Rows r;
+  r.m0 = 0;
+  if (a.per_expert) {
+    r.e = blockIdx.y;
+  } else {
+    const int incl_tiles = wave_inclusive(tiles, lane);
+    const unsigned long long past = __ballot(incl_tiles > static_cast<int>(blockIdx.y));
+    if (past == 0ull) return Rows{-1, 0, 0, 0};
+    r.e = __ffsll(past) - 1;
+    r.m0 = (static_cast<int>(blockIdx.y) - __shfl(incl_tiles - tiles, r.e)) * bm;
+  }
+  r.e = __builtin_amdgcn_readfirstlane(r.e);
+  r.m0 = __builtin_amdgcn_readfirstlane(r.m0);
+  r.count = __builtin_amdgcn_readlane(cnt, r.e);
+  r.base = __builtin_amdgcn_readlane(incl, r.e) - r.count;
+  if (r.m0 >= r.count) r.e = -1;
+  return r;
+}
+
+// grid = (ceil(hidden / BN), experts or row tiles).
+template <typename T, typename Tile>
+__global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
+  __shared__ __align__(16) char lds[Tile::kLds];
+  __shared__ int s_cnt[kMaxExperts];
+  __shared__ int s_rows[Tile::BM];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int e = wave; e < a.E; e += 4) {
+    const unsigned long long word = lane < a.words ? a.masks[static_cast<int64_t>(e) * a.words + lane] : 0ull;
+    const int total = wave_inclusive(__popcll(word), lane);
+    if (lane == 63) s_cnt[e] = total;
+  }
+  __syncthreads();
+  const int cnt = lane < a.E ? s_cnt[lane] : 0;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
+  const Rows r = find_rows(a, cnt, Tile::BM, lane);
+  if (r.e < 0) return;
+  const unsigned long long mask = lane < a.words ? a.masks[static_cast<int64_t>(r.e) * a.words + lane] : 0ull;
+  const int bits = __popcll(mask);
+  const int first = wave_inclusive(bits, lane) - bits;  // rank of this word's first token
+  const int64_t row_bytes = static_cast<int64_t>(a.dim) * sizeof(T);
+  const int n0 = blockIdx.x * Tile::BN;
+  const char* w = a.w1 + static_cast<int64_t>(r.e) * a.hidden * row_bytes;
+  const T* bias = reinterpret_cast<const T*>(a.b1) + static_cast<int64_t>(r.e) * a.hidden;
+  const int m_end = a.per_expert ? r.count : min(r.count, r.m0 + Tile::BM);
+  for (int m0 = r.m0; m0 < m_end; m0 += Tile::BM) {
+    // The tile's tokens, by rank.  Ranks past the expert's last repeat its
+    // first token of the tile (their results are dropped).
+    if (wave == 0) {
+      const int live = min(Tile::BM, r.count - m0);
+      unsigned long long word = mask;
+      for (int rank = first - m0; word != 0ull && rank < Tile::BM; ++rank, word &= word - 1ull) {
+        const int token = lane * 64 + __ffsll(word) - 1;
+        if (rank >= 0) s_rows[rank] = token;
+        if (rank == 0)
+          for (int i = live; i < Tile::BM; ++i) s_rows[i] = token;
+      }
+    }
+    __syncthreads();
+    f32x4 acc[Tile::NT][Tile::MT];
+#pragma unroll
+    for (int n = 0; n < Tile::NT; ++n)
+#pragma unroll
+      for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Tile::run(
+        lds, [&](int i) { return a.x + s_rows[i] * row_bytes; },
+        [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
+#pragma unroll
+    for (int n = 0; n < Tile::NT; ++n) {
+      const int c = n0 + Tile::col(n);
+      if (c >= a.hidden) continue;  // hidden is a multiple of 4: all four columns or none
+      const f32x4_t b = Mem<T>::load4(bias + c);
+#pragma unroll
+      for (int m = 0; m < Tile::MT; ++m) {
+        const int rank = m0 + Tile::row(m);
+        if (rank >= r.count) continue;
+        f32x4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float pre = Mem<T>::R(acc[n][m][i] + b[i]);  // the Linear's output
+          v[i] = 0.5f * pre * (1.f + erff(pre * 0.70710678118654752440f));
+        }
+        Mem<T>::put4(reinterpret_cast<T*>(a.h) + static_cast<int64_t>(r.base + rank) * a.hidden + c, v);
+      }
+    }
+    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < min(Tile::BM, r.count - m0)) {
+      const int token = s_rows[threadIdx.x];
+      for (int j = 0; j < a.top_k; ++j) {
+        const int64_t at = static_cast<int64_t>(token) * a.top_k + j;
+        if (a.ids[at] == r.e) a.slots[at] = r.base + m0 + threadIdx.x;
+      }
+    }
+    __syncthreads();  // s_rows is rewritten by the next tile
+  }
+}
+
+// grid = (ceil(dim / BN) * splits, experts or row tiles); blockIdx.x is
+// column tile * splits + split.
+template <typename T, typename Tile>
+__global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
+  __shared__ __align__(16) char lds[Tile::kLds];
+  const int lane = threadIdx.x & 63;
+  const Rows r = find_rows(a, lane < a.E ? a.counts[lane] : 0, Tile::BM, lane);
+  if (r.e < 0) return;
+  const int tile = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
+  const int64_t row_bytes = static_cast<int64_t>(a.hidden) * sizeof(T);
+  const int k0 = split * a.split_len;
+  const int k1 = min(static_cast<int>(row_bytes), k0 + a.split_len);
+  const int n0 = tile * Tile::BN;
+  const char* w = a.w2 + static_cast<int64_t>(r.e) * a.dim * row_bytes;
+  const char* h = a.h + r.base * row_bytes;
+  float* part = a.part + (static_cast<int64_t>(split) * a.tokens * a.top_k + r.base) * a.dim;
+  const int m_end = a.per_expert ? r.count : min(r.count, r.m0 + Tile::BM);
+  for (int m0 = r.m0; m0 < m_end; m0 += Tile::BM) {
+    f32x4 acc[Tile::NT][Tile::MT];
+#pragma unroll
+    for (int n = 0; n < Tile::NT; ++n)
+#pragma unroll
+      for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Tile::run(
+        lds, [&](int i) { return h + min(m0 + i, r.count - 1) * row_bytes; },
+        [&](int i) { return w + min(n0 + i, a.dim - 1) * row_bytes; }, k0, k1, acc);
+#pragma unroll
+    for (int n = 0; n < Tile::NT; ++n) {
+      const int c = n0 + Tile::col(n);
+      if (c >= a.dim) continue;
+#pragma unroll
+      for (int m = 0; m < Tile::MT; ++m) {
+        const int rank = m0 + Tile::row(m);
+        if (rank < r.count) *reinterpret_cast<f32x4*>(part + static_cast<int64_t>(rank) * a.dim + c) = acc[n][m];
+      }
+    }
+  }
+}
+
+// grid = ceil(tokens * dim / 4 / 256): four outputs of a token per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void moe_prompt_combine(PromptArgs a, mie::FastDiv row) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t t = row.div(i);
+  if (t >= static_cast<uint32_t>(a.tokens)) return;
+  const int c = (i - t * row.d) * 4;
+  const int64_t all = static_cast<int64_t>(a.tokens) * a.top_k * a.dim;
+  f32x4_t out = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < a.top_k; ++j) {  // increasing expert id
+    const int64_t at = static_cast<int64_t>(t) * a.top_k + j;
+    const float w = Mem<T>::R(a.weights[at]);
+    const f32x4_t b = Mem<T>::load4(reinterpret_cast<const T*>(a.b2) + static_cast<int64_t>(a.ids[at]) * a.dim + c);
+    const float* p = a.part + static_cast<int64_t>(a.slots[at]) * a.dim + c;
+    f32x4_t y = *reinterpret_cast<const f32x4_t*>(p);
+    for (int s = 1; s < a.splits; ++s) y += *reinterpret_cast<const f32x4_t*>(p + s * all);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      out[u] = Mem<T>::R(__fadd_rn(out[u], Mem<T>::R(__fmul_rn(w, Mem<T>::R(y[u] + b[u])))));
+  }
+  Mem<T>::put4(reinterpret_cast<T*>(a.out) + static_cast<int64_t>(t) * a.dim + c, out);
+}
+
+// Tiles.  Narrow: up to 32 rows per expert on average, where the launch streams
+// the experts' weights: one workgroup per (expert, column tile), 256 bytes of
+// every row in flight.  Wide: more rows.
+template <typename T> using Narrow = mie::gemm::Tile<T, 32, 64, 256, 1, 4>;
+template <typename T> using Wide = mie::gemm::Tile<T, 64, 64, 128, 2, 2>;
+
+struct Plan {
+  bool narrow;
+  int32_t rows;               // blockIdx.y extent
+  int32_t splits, split_len;  // W2
+};
+
+Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden, int elt) {
+  Plan p;
+  const int64_t slots = static_cast<int64_t>(tokens) * top_k;
+  p.narrow = slots <= 24 * static_cast<int64_t>(E);
+  const int bm = p.narrow ? 32 : 64, kb = p.narrow ? 256 : 128;
+  p.rows = p.narrow ? E : static_cast<int32_t>(slots / bm + std::min<int64_t>(E, slots));
+  // W2 has few column tiles: split its K until the launch holds about two
+  // (narrow) or four (wide) workgroups per CU.
+  const int64_t used = p.narrow ? std::min<int64_t>(E, slots) : slots / bm + E / 2;
+  const int64_t groups = static_cast<int64_t>((dim + 63) / 64) * std::max<int64_t>(1, used);
+  const int32_t steps = (hidden * elt + kb - 1) / kb;
+  const int64_t want = ((p.narrow ? 512 : 1024) + groups - 1) / groups;
+  const int32_t splits = static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>({want, kMaxSplits, steps / 2})));
+  p.split_len = (steps + splits - 1) / splits * kb;
+  p.splits = (hidden * elt + p.split_len - 1) / p.split_len;
+  return p;
+}
+
+int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
+
+// Lays the workspace out for `tokens` (at most kChunk) and returns its bytes.
+int64_t layout(PromptArgs& a, const Plan& p, int elt, char* base) {
+  const int64_t slots = static_cast<int64_t>(a.tokens) * a.top_k;
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) {
+    char* here = base + at;
+    at += align256(bytes);
+    return here;
+  };
+  a.masks = reinterpret_cast<unsigned long long*>(take(static_cast<int64_t>(a.E) * a.words * 8));
+  a.counts = reinterpret_cast<int32_t*>(take(a.E * 4));
+  a.ids = reinterpret_cast<int32_t*>(take(slots * 4));
+  a.weights = reinterpret_cast<float*>(take(slots * 4));
+  a.slots = reinterpret_cast<int32_t*>(take(slots * 4));
+  a.h = take(slots * a.hidden * elt);
+  a.part = reinterpret_cast<float*>(take(slots * a.dim * 4 * p.splits));
+  return at;
+}
+
+template <typename T>
+int32_t launch(const PromptArgs& a, const Plan& p, hipStream_t st) {
+  moe_prompt_route<T><<<a.words * 8, 256, 0, st>>>(a);
+  int32_t rc = mie::check_launch("moe_prompt_route");
+  if (rc != MIE_OK) return rc;
+  const dim3 g1((a.hidden + 63) / 64, p.rows), g2((a.dim + 63) / 64 * p.splits, p.rows);
+  if (p.narrow) {
+    moe_prompt_w1<T, Narrow<T>><<<g1, 256, 0, st>>>(a);
+  } else {
+    moe_prompt_w1<T, Wide<T>><<<g1, 256, 0, st>>>(a);
+  }
+  rc = mie::check_launch("moe_prompt_w1");
+  if (rc != MIE_OK) return rc;
+  if (p.narrow) {
+    moe_prompt_w2<T, Narrow<T>><<<g2, 256, 0, st>>>(a);
+  } else {
+    moe_prompt_w2<T, Wide<T>><<<g2, 256, 0, st>>>(a);
+  }
+  rc = mie::check_launch("moe_prompt_w2");
+  if (rc != MIE_OK) return rc;
+  const int64_t threads = static_cast<int64_t>(a.tokens) * (a.dim / 4);
+  moe_prompt_combine<T><<<static_cast<uint32_t>((threads + 255) / 256), 256, 0, st>>>(
+      a, mie::FastDiv::make(static_cast<uint32_t>(a.dim / 4)));
+  return mie::check_launch("moe_prompt_combine");
+}
+
+int32_t check(int64_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden, int32_t dtype) {
+  if (dtype != MIE_DTYPE_F32 && dtype != MIE_DTYPE_BF16)
+    return mie::fail(MIE_ERR_UNSUPPORTED, "mie_moe_prefill: float32 or bfloat16 only (dtype %d)", dtype);
+  if (tokens <= 0 || E <= 0 || E > kMaxExperts || top_k <= 0 || top_k > kMaxTopK || top_k > E)
+    return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: tokens=%lld experts=%d top_k=%d (at most %d and %d)",
+                     static_cast<long long>(tokens), E, top_k, kMaxExperts, kMaxTopK);
+  const int vec = 16 / mie::elt_size(dtype);
+  if (dim <= 0 || hidden <= 0 || dim % vec != 0 || hidden % vec != 0 || dim > (1 << 20) || hidden > (1 << 20))
+    return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: dim=%d hidden=%d must be multiples of %d up to 2^20", dim,
+                     hidden, vec);
+  return MIE_OK;
+}
+
+PromptArgs shape_args(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden) {
+  PromptArgs a{};
+  a.tokens = tokens;
+  a.E = E;
+  a.top_k = top_k;
+  a.dim = dim;
+  a.hidden = hidden;
+  a.words = (tokens + 63) / 64;
+  return a;
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+extern "C" int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts, int32_t top_k, int32_t dim,
+                                             int32_t hidden, int32_t dtype) {
+  const int32_t rc = check(tokens, num_experts, top_k, dim, hidden, dtype);
+  if (rc != MIE_OK) return -rc;
+  const int elt = mie::elt_size(dtype);
+  int64_t need = 0;
+  // The last chunk is shorter and may split K more ways.
+  for (int64_t n : {std::min<int64_t>(tokens, kChunk), tokens % kChunk}) {
+    if (n == 0) continue;
+    PromptArgs a = shape_args(static_cast<int32_t>(n), num_experts, top_k, dim, hidden);
+    need = std::max(need, layout(a, make_plan(a.tokens, num_experts, top_k, dim, hidden, elt), elt, nullptr));
+  }
+  return need;
+}
+
+extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* router_weight, const void* w1,
+                                   const void* b1, const void* w2, const void* b2, int32_t num_experts,
+                                   int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace,
+                                   int64_t workspace_bytes, int32_t dtype, void* stream) {
+  mie::clear_error();
+  int32_t rc = check(tokens, num_experts, top_k, dim, hidden, dtype);
+  if (rc != MIE_OK) return rc;
+  if (!x || !router_weight || !w1 || !b1 || !w2 || !b2 || !out || !workspace)
+    return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: null pointer");
+  for (const void* p : {x, router_weight, w1, b1, w2, b2, static_cast<const void*>(out),
+                        static_cast<const void*>(workspace)})
+    if (!aligned16(p)) return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: every pointer must be 16-byte aligned");
+  const int64_t need = mie_moe_prefill_workspace(tokens, num_experts, top_k, dim, hidden, dtype);
+  if (workspace_bytes < need)
+    return mie::fail(MIE_ERR_WORKSPACE, "mie_moe_prefill: workspace of %lld bytes, needs %lld",
+                     static_cast<long long>(workspace_bytes), static_cast<long long>(need));
+  const int elt = mie::elt_size(dtype);
+  for (int64_t t0 = 0; t0 < tokens; t0 += kChunk) {
+    PromptArgs a = shape_args(static_cast<int32_t>(std::min<int64_t>(kChunk, tokens - t0)), num_experts, top_k, dim,
+                              hidden);
+    const Plan p = make_plan(a.tokens, num_experts, top_k, dim, hidden, elt);
+    layout(a, p, elt, static_cast<char*>(workspace));
+    a.x = static_cast<const char*>(x) + t0 * dim * elt;
+    a.router = static_cast<const char*>(router_weight);
+    a.w1 = static_cast<const char*>(w1);
+    a.b1 = static_cast<const char*>(b1);
+    a.w2 = static_cast<const char*>(w2);
+    a.b2 = static_cast<const char*>(b2);
+    a.out = static_cast<char*>(out) + t0 * dim * elt;
+    a.per_expert = p.narrow;
+    a.splits = p.splits;
+    a.split_len = p.split_len;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    rc = dtype == MIE_DTYPE_F32 ? launch<float>(a, p, st) : launch<uint16_t>(a, p, st);
+    if (rc != MIE_OK) return rc;
+  }
+  return MIE_OK;
+}

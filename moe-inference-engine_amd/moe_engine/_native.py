@@ -126,6 +126,14 @@ _SIGNATURES = {
          _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,  # logits, ids, weights, hidden, out
          _i32, _c_void_p],  # dtype, stream
     ),
+    "mie_moe_prefill_workspace": (_i64, [_i64, _i32, _i32, _i32, _i32, _i32]),  # tokens, experts, top_k, dim, hidden, dtype
+    "mie_moe_prefill": (
+        _i32,
+        [_c_void_p, _i64, _c_void_p,  # x, tokens, router weight
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p,  # canonical w1, b1, w2, b2 storages
+         _i32, _i32, _i32, _i32,  # experts, top_k, dim, hidden
+         _c_void_p, _c_void_p, _i64, _i32, _c_void_p],  # out, workspace, its bytes, dtype, stream
+    ),
     "mie_argmax": (_i32, [_c_void_p, _i64, _c_void_p, _i32, _c_void_p]),  # x, n, out (int64), dtype, stream
     "mie_embed": (
         _i32,
@@ -230,6 +238,23 @@ def check(status: int, what: str) -> None:
 def is_rocm_device(t: torch.Tensor) -> bool:
     """True for tensors on a ROCm GPU (torch names the device type 'cuda')."""
     return t.is_cuda and torch.version.hip is not None
+
+
+def plain_inference(x: torch.Tensor) -> bool:
+    """True when a library call may stand in for PyTorch operations on x:
+    nothing is recorded, traced, transformed or re-dispatched (no gradients,
+    autocast, forward-mode AD, functorch transform, tracing, compilation or
+    dispatch mode), and x is a plain tensor."""
+    return (
+        not torch.is_grad_enabled()
+        and type(x) in (torch.Tensor, torch.nn.Parameter)
+        and not torch.is_autocast_enabled()
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
+        and torch._C._len_torch_dispatch_stack() == 0
+        and not torch.jit.is_tracing()
+        and not torch.compiler.is_compiling()
+    )
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

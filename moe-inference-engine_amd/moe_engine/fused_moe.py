@@ -222,3 +222,63 @@ def decode_block(x, norm_weight, norm_bias, norm_eps, router_weight, w1_base, b1
     if rc:
         _native.check(rc, "mie_moe_decode_block")
     return out.view(1, 1, dim)
+
+
+def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int) -> bool:
+    """Whether prefill() takes these tokens and weights: one dtype, float32 or
+    bfloat16, on one ROCm device, the canonical layouts of
+    has_canonical_layout, and rows of whole 16-byte vectors."""
+    dtype, device = x.dtype, x.device
+    if not HAS_HIP or not _native.is_rocm_device(x) or dtype not in DTYPES or router_weight.dim() != 2 or w1.dim() != 3:
+        return False
+    num_experts, dim = router_weight.shape
+    hidden = w1.shape[1]
+    vec = 16 // x.element_size()
+    return (
+        x.shape[-1] == dim
+        and 0 < num_experts <= MAX_EXPERTS
+        and 0 < top_k <= min(MAX_TOP_K, num_experts)
+        and dim > 0
+        and hidden > 0
+        and dim % vec == 0
+        and hidden % vec == 0
+        and all(
+            t.shape == shape and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
+            for t, shape in (
+                (router_weight, (num_experts, dim)),
+                (w1, (num_experts, hidden, dim)),
+                (b1, (num_experts, hidden)),
+                (w2, (num_experts, dim, hidden)),
+                (b2, (num_experts, dim)),
+            )
+        )
+    )
+
+
+def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int) -> torch.Tensor:
+    """The MoE layer over the tokens of x [..., hidden] (reference
+    model.py:443-461) in four launches per 4096 tokens (mie_moe_prefill), with
+    decode()'s semantics and rounding points per token; returns a new tensor
+    of x's shape."""
+    if not prefill_supported(x, router_weight, w1_base, b1_base, w2_base, b2_base, top_k):
+        raise RuntimeError("prompt MoE needs float32 or bfloat16 tokens and canonical weights on one ROCm device")
+    num_experts, dim = router_weight.shape
+    hidden = w1_base.shape[1]
+    x = x.contiguous()
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty_like(x)
+    tokens = x.numel() // dim
+    if tokens == 0:
+        return out
+    lib, code = _native.lib(), _native.dtype_code(x.dtype)
+    nbytes = lib.mie_moe_prefill_workspace(tokens, num_experts, top_k, dim, hidden, code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    rc = lib.mie_moe_prefill(
+        x.data_ptr(), tokens, router_weight.data_ptr(),
+        w1_base.data_ptr(), b1_base.data_ptr(), w2_base.data_ptr(), b2_base.data_ptr(),
+        num_experts, top_k, dim, hidden, out.data_ptr(), ws.data_ptr(), nbytes, code, _native.stream_of(x),
+    )
+    if rc:
+        _native.check(rc, "mie_moe_prefill")
+    return out

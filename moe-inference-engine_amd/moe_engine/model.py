@@ -63,6 +63,10 @@ def _tensors_replaced() -> None:
     _TENSOR_EPOCH[0] += 1
 
 
+# Hooks registered for every module: with one in place, code that stands in for
+# a module call must call the module.
+_GLOBAL_MODULE_HOOKS = (nn.modules.module._global_forward_hooks, nn.modules.module._global_forward_pre_hooks)
+
 # Plain attributes a launch plan is built from: a MoE layer's mode and a
 # norm's eps.  Changing one advances _TENSOR_EPOCH like a tensor replacement.
 _PLAN_SETTINGS = ("mode", "eps")
@@ -494,9 +498,11 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
     Mode 'reference' runs the reference's PyTorch path (model.py:443-461)
     everywhere.  In mode 'auto' or 'direct', one-token decode runs the fused
     HIP kernels (moe_engine.fused_moe) where they apply - a ROCm device, the
-    HIP library, float32 or bfloat16, one token - and a float32 prefill of up to 512
-    tokens on a ROCm device runs dense-masked (_forward_dense: the reference's
-    result without its per-expert synchronisations).  'auto' falls back to the
+    HIP library, float32 or bfloat16, one token - and prompts at inference run
+    the grouped HIP kernels (_forward_grouped: the reference's result without
+    its per-expert synchronisations).  Where those do not apply (gradients,
+    autocast, odd widths), a float32 prefill of up to 512 tokens on a ROCm
+    device runs dense-masked (_forward_dense).  'auto' falls back to the
     PyTorch path elsewhere; a forced 'direct' decode that cannot run raises
     before any cache mutation, through the model's decode preflight
     (model.py:408-441).
@@ -687,9 +693,60 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
             out = out + dense_w[:, e : e + 1] * y[e]
         return out.reshape(batch, seq_len, dim)
 
+    def _experts_are_plain(self) -> bool:
+        """Whether running the experts' modules would compute exactly what the
+        canonical storages describe: unmodified Expert modules without hooks,
+        whose parameters are the storages' slices."""
+        if any(_GLOBAL_MODULE_HOOKS):
+            return False
+        s = self._expert_storage
+        # Addresses of the next expert's parameters, and the steps between experts.
+        at = [s[name].data_ptr() for name in ("w1", "b1", "w2", "b2")]
+        step = [s[name].stride(0) * s[name].element_size() for name in ("w1", "b1", "w2", "b2")]
+        for expert in self.experts._modules.values():
+            net = expert._modules.get("net")
+            if type(expert) is not Expert or type(net) is not nn.Sequential or len(net._modules) != 3:
+                return False
+            up, act, down = net._modules.values()
+            if type(up) is not Linear or type(act) is not nn.GELU or type(down) is not Linear or act.approximate != "none":
+                return False
+            for m in (expert, net, up, act, down):
+                if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                    return False
+            for i, t in enumerate((*up._parameters.values(), *down._parameters.values())):  # weight, bias each
+                if t is None or t.data_ptr() != at[i]:
+                    return False
+                at[i] += step[i]
+        return True
+
+    def uses_grouped_prefill(self, x: torch.Tensor, *, decode: bool) -> bool:
+        """Prompts at inference take the grouped HIP kernels (fused_moe.prefill)
+        where these apply: float32 or bfloat16 on a ROCm device with the
+        canonical layout.  Gradients, autocast, forward-mode AD, functorch
+        transforms, tracing and dispatch modes keep the PyTorch paths, and so
+        do experts whose modules were changed, where those would run them
+        (_forward_dense reads the storages too)."""
+        tokens = x.shape[0] * x.shape[1]
+        s = self._expert_storage
+        return (
+            self.mode != "reference"
+            and not (decode and tokens == 1)
+            and tokens >= 1
+            and _native.plain_inference(x)
+            and fused_moe.prefill_supported(x, self.router.weight, s["w1"], s["b1"], s["w2"], s["b2"], self.top_k)
+            and s["w1"].shape[0] == self.num_experts
+            and (self.uses_dense_prefill(x, decode=decode) or self._experts_are_plain())
+        )
+
+    def _forward_grouped(self, x: torch.Tensor) -> torch.Tensor:
+        s = self._expert_storage
+        return fused_moe.prefill(x, self.router.weight, s["w1"], s["b1"], s["w2"], s["b2"], top_k=self.top_k)
+
     def forward(self, x, *, decode=False):
         if self.uses_direct(x, decode=decode):
             return self._forward_direct(x)
+        if self.uses_grouped_prefill(x, decode=decode):
+            return self._forward_grouped(x)
         if self.uses_dense_prefill(x, decode=decode):
             return self._forward_dense(x)
         return self._forward_reference(x)
