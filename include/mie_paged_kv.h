@@ -17,7 +17,10 @@
  *   mie_moe_route     <- fused_moe.route         src/moe_engine/fused_moe.py:274-309
  *   mie_moe_decode    <- fused_moe.decode        src/moe_engine/fused_moe.py:312-380
  *   mie_moe_decode_block <- the block's x + moe(moe_norm(x)) for one token  src/moe_engine/model.py:496-497
- *   mie_moe_prefill   <- MoEFeedForward.forward over a prompt  src/moe_engine/model.py:443-461
+ *   mie_moe_prefill   <- MoEFeedForward.forward over a prompt  src/moe_engine/model.py:443-461,
+ *                        optionally with the block's norm and residual (:496)
+ *   mie_attn_prefill  <- CachedAttention.forward over a prompt (model.py:226-269),
+ *                        optionally with the block's norm and residual (:495)
  *   mie_argmax        <- Model.generate's greedy torch.argmax   src/moe_engine/model.py:603
  *   mie_lm_head       <- final_norm + output_projection (model.py:564-565) and,
  *                        optionally, the greedy argmax (:603) for one token
@@ -364,7 +367,10 @@ int32_t mie_moe_decode_block(const void* x, const void* ln_weight, const void* l
  * model.py:443-461): routing as in mie_moe_route, then for each token the sum
  * over its top_k experts in increasing expert id of
  * round(w * (W2_e GELU(W1_e x + b1_e) + b2_e)), with mie_moe_decode's dtypes
- * and rounding points.  x and out [tokens, dim], the weights in canonical
+ * and rounding points.  With ln_weight the layer runs on LayerNorm(x) (as in
+ * mie_moe_decode_block) and with residual [tokens, dim] that is added to the
+ * result: together the block's MoE half, x + moe(moe_norm(x)) (model.py:496).
+ * x and out [tokens, dim], the weights in canonical
  * layouts as for mie_moe_decode, all 16-byte aligned; dim and hidden multiples
  * of 4 (float32) or 8 (bfloat16), at most 64 experts and top_k 8.  out must
  * not alias x.  Only experts that a token selected are read.  workspace holds
@@ -373,10 +379,33 @@ int32_t mie_moe_decode_block(const void* x, const void* ln_weight, const void* l
  */
 int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden,
                                   int32_t dtype);
-int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* router_weight, const void* w1, const void* b1,
-                        const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim,
-                        int32_t hidden, void* out, void* workspace, int64_t workspace_bytes, int32_t dtype,
+int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ln_weight, const void* ln_bias, float ln_eps,
+                        const void* residual, const void* router_weight, const void* w1, const void* b1,
+                        const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace, int64_t workspace_bytes, int32_t dtype,
                         void* stream);
+
+/*
+ * Attention over a prompt at position 0 (CachedAttention.forward,
+ * model.py:226-269, with cache.write :167-184): x [tokens, H * D], optionally
+ * through a LayerNorm (ln_weight non-NULL, as in mie_qkv_append), QKV
+ * projection, K and V stored at logical positions 0 .. tokens-1 of the pools
+ * (one layer, strides multiples of 8 elements, blocks reserved), causal
+ * attention over them, output projection, and the residual [tokens, H * D]
+ * when given.  float32 or bfloat16, head_dim 32, 64, 96 or 128
+ * (mie_attn_prefill_supported); every sum and the probabilities are float32,
+ * and in bfloat16 each stored tensor of the PyTorch path is rounded once.
+ * Every pointer 16-byte aligned; out may alias residual but not x; workspace
+ * holds mie_attn_prefill_workspace bytes (negative: not supported), with
+ * nothing to clear.  Three launches, four with the norm.
+ */
+int32_t mie_attn_prefill_supported(int32_t num_heads, int32_t head_dim, int32_t dtype);
+int64_t mie_attn_prefill_workspace(int32_t tokens, int32_t num_heads, int32_t head_dim, int32_t dtype);
+int32_t mie_attn_prefill(const void* x, int32_t tokens, const void* ln_weight, const void* ln_bias, float ln_eps,
+                         const void* w_in, const void* b_in, const void* w_out, const void* b_out,
+                         const void* residual, void* out, void* k_pool, void* v_pool, int64_t pool_stride_block,
+                         int64_t pool_stride_head, int32_t num_blocks, const int32_t* block_table,
+                         int32_t block_table_len, int32_t num_heads, int32_t head_dim, int32_t block_size,
+                         float scale, void* workspace, int64_t workspace_bytes, int32_t dtype, void* stream);
 
 /*
  * Greedy pick (Model.generate at temperature 0, model.py:603): the index

@@ -10,8 +10,11 @@
 //   y_te   = W2_e GELU(W1_e x_t + b1_e) + b2_e         for the selected experts
 //   out_t  = sum over them in increasing expert id, from 0, of round(w y)
 //
+// The block form adds what stands around it in a decoder block (model.py:496):
+// x_t goes through a LayerNorm first and a residual is added to out_t.
+//
 // Rounding points are the one-token kernels' (moe_decode.hip): every sum is
-// float32; in bfloat16 each Linear's output, GELU's, the route weight, the
+// float32; in bfloat16 the norm's output, each Linear's output, GELU's, the route weight, the
 // product and each partial sum are rounded, as the PyTorch path stores them.
 //
 // Four launches.
@@ -57,6 +60,11 @@ struct PromptArgs {
   const char* b1;      // T [E, hidden]
   const char* w2;      // T [E, dim, hidden]
   const char* b2;      // T [E, dim]
+  const char* ln_w;    // T [dim]; block form: the norm's weight (NULL: no norm)
+  const char* ln_b;    // T [dim] or NULL
+  const char* residual;  // T [tokens, dim]; block form: added to the output (or NULL)
+  float ln_eps;
+  char* normed;        // T [tokens, dim]: the norm's output
   int32_t tokens, E, top_k, dim, hidden;
   int32_t words;              // mask words per expert: ceil(tokens / 64)
   int32_t per_expert;         // 1: blockIdx.y is an expert; 0: the y-th row tile of all experts
@@ -71,9 +79,34 @@ struct PromptArgs {
   char* out;                  // T [tokens, dim]
 };
 
-// grid = words * 8; four waves, two tokens each.
+// LayerNorm of a row by one wave (float32, biased variance), into `out`.
+template <typename T>
+__device__ __forceinline__ void norm_row(const PromptArgs& a, const T* x, T* out, int lane) {
+  float s = 0.f;
+  for (int i = lane * 4; i < a.dim; i += 256) {
+    const f32x4_t v = Mem<T>::load4(x + i);
+    s += (v.x + v.y) + (v.z + v.w);
+  }
+  const float mean = mie::wave_sum(s) / a.dim;
+  float q = 0.f;
+  for (int i = lane * 4; i < a.dim; i += 256) {
+    const f32x4_t d = Mem<T>::load4(x + i) - mean;
+    q = dot4(d, d, q);
+  }
+  const float rstd = rsqrtf(mie::wave_sum(q) / a.dim + a.ln_eps);
+  for (int i = lane * 4; i < a.dim; i += 256) {
+    f32x4_t y = (Mem<T>::load4(x + i) - mean) * rstd * Mem<T>::load4(reinterpret_cast<const T*>(a.ln_w) + i);
+    if (a.ln_b) y += Mem<T>::load4(reinterpret_cast<const T*>(a.ln_b) + i);
+    Mem<T>::put4(out + i, y);
+  }
+}
+
+// grid = words * 8; four waves, two tokens each.  Bound by its memory rounds:
+// eight experts' rows and the tokens' go out together, in pieces of 768
+// elements (8 experts, dim 768: one round after the norm's).
 template <typename T>
 __global__ __launch_bounds__(256) void moe_prompt_route(PromptArgs a) {
+  constexpr int kPieces = 3;
   __shared__ unsigned int s_mask[kMaxExperts];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -84,22 +117,44 @@ __global__ __launch_bounds__(256) void moe_prompt_route(PromptArgs a) {
     const bool two = t0 + 1 < a.tokens;
     const T* x0 = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(t0) * a.dim;
     const T* x1 = two ? x0 + a.dim : x0;
+    if (a.ln_w) {
+      // Each lane reads back what it wrote itself.
+      T* y0 = reinterpret_cast<T*>(a.normed) + static_cast<int64_t>(t0) * a.dim;
+      norm_row(a, x0, y0, lane);
+      if (two) norm_row(a, x1, y0 + a.dim, lane);
+      x0 = y0;
+      x1 = two ? y0 + a.dim : y0;
+    }
     const T* router = reinterpret_cast<const T*>(a.router);
     float l0 = -INFINITY, l1 = -INFINITY;  // lane e: expert e's logit
-    // Four experts' rows at a time, so their loads and the tokens' go out together.
-    for (int e = 0; e < a.E; e += 4) {
-      float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int i = lane * 4; i < a.dim; i += 256) {
-        const f32x4_t v0 = Mem<T>::load4(x0 + i), v1 = Mem<T>::load4(x1 + i);
+    for (int e = 0; e < a.E; e += 8) {
+      float s0[8], s1[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const f32x4_t r = Mem<T>::load4(router + static_cast<int64_t>(min(e + u, a.E - 1)) * a.dim + i);
-          s0[u] = dot4(r, v0, s0[u]);
-          s1[u] = dot4(r, v1, s1[u]);
+      for (int u = 0; u < 8; ++u) s0[u] = s1[u] = 0.f;
+      for (int i0 = lane * 4; i0 < a.dim; i0 += 256 * kPieces) {
+        typename Mem<T>::raw4 v0[kPieces], v1[kPieces], r[8][kPieces];
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+          const int i = i0 + 256 * p < a.dim ? i0 + 256 * p : 0;  // in bounds; dropped below
+          v0[p] = Mem<T>::load_raw(x0 + i);
+          v1[p] = Mem<T>::load_raw(x1 + i);
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            r[u][p] = Mem<T>::load_raw(router + static_cast<int64_t>(min(e + u, a.E - 1)) * a.dim + i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+          if (i0 + 256 * p >= a.dim) break;
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            s0[u] = dot4(Mem<T>::widen(r[u][p]), Mem<T>::widen(v0[p]), s0[u]);
+            s1[u] = dot4(Mem<T>::widen(r[u][p]), Mem<T>::widen(v1[p]), s1[u]);
+          }
         }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < 8; ++u) {
         const float d0 = mie::wave_sum(s0[u]), d1 = mie::wave_sum(s1[u]);
         if (lane == e + u && e + u < a.E) {
           l0 = d0;
@@ -177,17 +232,24 @@ __device__ __forceinline__ Rows find_rows(const PromptArgs& a, int cnt, int bm, 
 template <typename T, typename Tile>
 __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   __shared__ __align__(16) char lds[Tile::kLds];
-  __shared__ int s_cnt[kMaxExperts];
   __shared__ int s_rows[Tile::BM];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int e = wave; e < a.E; e += 4) {
-    const unsigned long long word = lane < a.words ? a.masks[static_cast<int64_t>(e) * a.words + lane] : 0ull;
-    const int total = wave_inclusive(__popcll(word), lane);
-    if (lane == 63) s_cnt[e] = total;
+  // Every wave counts every expert's tokens: eight masks in one memory round.
+  int cnt = 0;  // lane e: expert e's
+  for (int e = 0; e < a.E; e += 8) {
+    unsigned long long word[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      word[u] = a.masks[static_cast<int64_t>(min(e + u, a.E - 1)) * a.words + min(lane, a.words - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      int c = lane < a.words ? __popcll(word[u]) : 0;
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
+      if (lane == e + u && e + u < a.E) cnt = c;
+    }
   }
-  __syncthreads();
-  const int cnt = lane < a.E ? s_cnt[lane] : 0;
   if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
   const Rows r = find_rows(a, cnt, Tile::BM, lane);
   if (r.e < 0) return;
@@ -196,6 +258,7 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   const int first = wave_inclusive(bits, lane) - bits;  // rank of this word's first token
   const int64_t row_bytes = static_cast<int64_t>(a.dim) * sizeof(T);
   const int n0 = blockIdx.x * Tile::BN;
+  const char* x = a.ln_w ? a.normed : a.x;
   const char* w = a.w1 + static_cast<int64_t>(r.e) * a.hidden * row_bytes;
   const T* bias = reinterpret_cast<const T*>(a.b1) + static_cast<int64_t>(r.e) * a.hidden;
   const int m_end = a.per_expert ? r.count : min(r.count, r.m0 + Tile::BM);
@@ -219,7 +282,7 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
 #pragma unroll
       for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     Tile::run(
-        lds, [&](int i) { return a.x + s_rows[i] * row_bytes; },
+        lds, [&](int i) { return x + s_rows[i] * row_bytes; },
         [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
 #pragma unroll
     for (int n = 0; n < Tile::NT; ++n) {
@@ -290,26 +353,58 @@ __global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
 }
 
 // grid = ceil(tokens * dim / 4 / 256): four outputs of a token per thread.
-template <typename T>
+// Two memory rounds: the token's slots, then every partial sum of KK experts.
+template <typename T, int KK>
 __global__ __launch_bounds__(256) void moe_prompt_combine(PromptArgs a, mie::FastDiv row) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   const uint32_t t = row.div(i);
   if (t >= static_cast<uint32_t>(a.tokens)) return;
   const int c = (i - t * row.d) * 4;
   const int64_t all = static_cast<int64_t>(a.tokens) * a.top_k * a.dim;
+  const int64_t here = static_cast<int64_t>(t) * a.dim + c;
+  f32x4_t res = {0.f, 0.f, 0.f, 0.f};
+  if (a.residual) res = Mem<T>::load4(reinterpret_cast<const T*>(a.residual) + here);
   f32x4_t out = {0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < a.top_k; ++j) {  // increasing expert id
-    const int64_t at = static_cast<int64_t>(t) * a.top_k + j;
-    const float w = Mem<T>::R(a.weights[at]);
-    const f32x4_t b = Mem<T>::load4(reinterpret_cast<const T*>(a.b2) + static_cast<int64_t>(a.ids[at]) * a.dim + c);
-    const float* p = a.part + static_cast<int64_t>(a.slots[at]) * a.dim + c;
-    f32x4_t y = *reinterpret_cast<const f32x4_t*>(p);
-    for (int s = 1; s < a.splits; ++s) y += *reinterpret_cast<const f32x4_t*>(p + s * all);
+  for (int j0 = 0; j0 < a.top_k; j0 += KK) {  // increasing expert id
+    int slot[KK], id[KK];
+    float w[KK];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      out[u] = Mem<T>::R(__fadd_rn(out[u], Mem<T>::R(__fmul_rn(w, Mem<T>::R(y[u] + b[u])))));
+    for (int j = 0; j < KK; ++j) {
+      const int64_t at = static_cast<int64_t>(t) * a.top_k + min(j0 + j, a.top_k - 1);
+      slot[j] = a.slots[at];
+      id[j] = a.ids[at];
+      w[j] = Mem<T>::R(a.weights[at]);
+    }
+    f32x4_t y[KK], b[KK];
+#pragma unroll
+    for (int j = 0; j < KK; ++j) {
+      b[j] = Mem<T>::load4(reinterpret_cast<const T*>(a.b2) + static_cast<int64_t>(id[j]) * a.dim + c);
+      y[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int s0 = 0; s0 < a.splits; s0 += 4) {
+      f32x4_t p[KK][4];
+#pragma unroll
+      for (int j = 0; j < KK; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          p[j][s] = *reinterpret_cast<const f32x4_t*>(a.part + min(s0 + s, a.splits - 1) * all +
+                                                      static_cast<int64_t>(slot[j]) * a.dim + c);
+#pragma unroll
+      for (int j = 0; j < KK; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          if (s0 + s < a.splits) y[j] += p[j][s];
+    }
+#pragma unroll
+    for (int j = 0; j < KK; ++j) {
+      if (j0 + j >= a.top_k) break;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        out[u] = Mem<T>::R(__fadd_rn(out[u], Mem<T>::R(__fmul_rn(w[j], Mem<T>::R(y[j][u] + b[j][u])))));
+    }
   }
-  Mem<T>::put4(reinterpret_cast<T*>(a.out) + static_cast<int64_t>(t) * a.dim + c, out);
+  if (a.residual) out += res;
+  Mem<T>::put4(reinterpret_cast<T*>(a.out) + here, out);
 }
 
 // Tiles.  Narrow: up to 32 rows per expert on average, where the launch streams
@@ -358,6 +453,7 @@ int64_t layout(PromptArgs& a, const Plan& p, int elt, char* base) {
   a.ids = reinterpret_cast<int32_t*>(take(slots * 4));
   a.weights = reinterpret_cast<float*>(take(slots * 4));
   a.slots = reinterpret_cast<int32_t*>(take(slots * 4));
+  a.normed = take(static_cast<int64_t>(a.tokens) * a.dim * elt);
   a.h = take(slots * a.hidden * elt);
   a.part = reinterpret_cast<float*>(take(slots * a.dim * 4 * p.splits));
   return at;
@@ -384,8 +480,13 @@ int32_t launch(const PromptArgs& a, const Plan& p, hipStream_t st) {
   rc = mie::check_launch("moe_prompt_w2");
   if (rc != MIE_OK) return rc;
   const int64_t threads = static_cast<int64_t>(a.tokens) * (a.dim / 4);
-  moe_prompt_combine<T><<<static_cast<uint32_t>((threads + 255) / 256), 256, 0, st>>>(
-      a, mie::FastDiv::make(static_cast<uint32_t>(a.dim / 4)));
+  const uint32_t groups = static_cast<uint32_t>((threads + 255) / 256);
+  const mie::FastDiv row = mie::FastDiv::make(static_cast<uint32_t>(a.dim / 4));
+  if (a.top_k == 1) {
+    moe_prompt_combine<T, 1><<<groups, 256, 0, st>>>(a, row);
+  } else {
+    moe_prompt_combine<T, 2><<<groups, 256, 0, st>>>(a, row);
+  }
   return mie::check_launch("moe_prompt_combine");
 }
 
@@ -432,16 +533,17 @@ extern "C" int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts
   return need;
 }
 
-extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* router_weight, const void* w1,
-                                   const void* b1, const void* w2, const void* b2, int32_t num_experts,
-                                   int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace,
+extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ln_weight, const void* ln_bias,
+                                   float ln_eps, const void* residual, const void* router_weight, const void* w1,
+                                   const void* b1, const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace,
                                    int64_t workspace_bytes, int32_t dtype, void* stream) {
   mie::clear_error();
   int32_t rc = check(tokens, num_experts, top_k, dim, hidden, dtype);
   if (rc != MIE_OK) return rc;
   if (!x || !router_weight || !w1 || !b1 || !w2 || !b2 || !out || !workspace)
     return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: null pointer");
-  for (const void* p : {x, router_weight, w1, b1, w2, b2, static_cast<const void*>(out),
+  if (!ln_weight && ln_bias) return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: a norm bias needs a weight");
+  for (const void* p : {x, ln_weight, ln_bias, residual, router_weight, w1, b1, w2, b2, static_cast<const void*>(out),
                         static_cast<const void*>(workspace)})
     if (!aligned16(p)) return mie::fail(MIE_ERR_INVALID, "mie_moe_prefill: every pointer must be 16-byte aligned");
   const int64_t need = mie_moe_prefill_workspace(tokens, num_experts, top_k, dim, hidden, dtype);
@@ -455,6 +557,10 @@ extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ro
     const Plan p = make_plan(a.tokens, num_experts, top_k, dim, hidden, elt);
     layout(a, p, elt, static_cast<char*>(workspace));
     a.x = static_cast<const char*>(x) + t0 * dim * elt;
+    a.ln_w = static_cast<const char*>(ln_weight);
+    a.ln_b = static_cast<const char*>(ln_bias);
+    a.ln_eps = ln_eps;
+    a.residual = residual ? static_cast<const char*>(residual) + t0 * dim * elt : nullptr;
     a.router = static_cast<const char*>(router_weight);
     a.w1 = static_cast<const char*>(w1);
     a.b1 = static_cast<const char*>(b1);

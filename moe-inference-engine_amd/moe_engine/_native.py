@@ -129,10 +129,21 @@ _SIGNATURES = {
     "mie_moe_prefill_workspace": (_i64, [_i64, _i32, _i32, _i32, _i32, _i32]),  # tokens, experts, top_k, dim, hidden, dtype
     "mie_moe_prefill": (
         _i32,
-        [_c_void_p, _i64, _c_void_p,  # x, tokens, router weight
+        [_c_void_p, _i64, _c_void_p, _c_void_p, _f32, _c_void_p,  # x, tokens, norm weight, norm bias, eps, residual
+         _c_void_p,  # router weight
          _c_void_p, _c_void_p, _c_void_p, _c_void_p,  # canonical w1, b1, w2, b2 storages
          _i32, _i32, _i32, _i32,  # experts, top_k, dim, hidden
          _c_void_p, _c_void_p, _i64, _i32, _c_void_p],  # out, workspace, its bytes, dtype, stream
+    ),
+    "mie_attn_prefill_supported": (_i32, [_i32, _i32, _i32]),  # heads, head_dim, dtype
+    "mie_attn_prefill_workspace": (_i64, [_i32, _i32, _i32, _i32]),  # tokens, heads, head_dim, dtype
+    "mie_attn_prefill": (
+        _i32,
+        [_c_void_p, _i32, _c_void_p, _c_void_p, _f32,  # x, tokens, norm weight, norm bias, eps
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p,  # in_proj weight, bias, out_proj weight, bias
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i32,  # residual, out, pools, strides, num_blocks
+         _c_void_p, _i32, _i32, _i32, _i32, _f32,  # block table, length, heads, head_dim, block_size, scale
+         _c_void_p, _i64, _i32, _c_void_p],  # workspace, its bytes, dtype, stream
     ),
     "mie_argmax": (_i32, [_c_void_p, _i64, _c_void_p, _i32, _c_void_p]),  # x, n, out (int64), dtype, stream
     "mie_embed": (

@@ -255,11 +255,13 @@ def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int
     )
 
 
-def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int) -> torch.Tensor:
+def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int, norm=None,
+            residual=None) -> torch.Tensor:
     """The MoE layer over the tokens of x [..., hidden] (reference
     model.py:443-461) in four launches per 4096 tokens (mie_moe_prefill), with
     decode()'s semantics and rounding points per token; returns a new tensor
-    of x's shape."""
+    of x's shape.  With `norm` (weight, bias or None, eps) the layer runs on
+    LayerNorm(x), and `residual` (x's shape, dtype and device) is added."""
     if not prefill_supported(x, router_weight, w1_base, b1_base, w2_base, b2_base, top_k):
         raise RuntimeError("prompt MoE needs float32 or bfloat16 tokens and canonical weights on one ROCm device")
     num_experts, dim = router_weight.shape
@@ -267,6 +269,17 @@ def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int)
     x = x.contiguous()
     if x.data_ptr() % 16:
         x = x.clone()
+    ln_w = ln_b = 0
+    eps = 1e-5
+    if norm is not None:
+        weight, bias, eps = norm
+        for t in (weight, bias):
+            if t is not None and (t.shape != (dim,) or not t.is_contiguous() or t.dtype != x.dtype or t.device != x.device):
+                raise ValueError(f"norm parameters must be contiguous [{dim}] vectors like x")
+        ln_w, ln_b = weight.data_ptr(), _native.ptr(bias)
+    if residual is not None and (residual.shape != x.shape or not residual.is_contiguous() or residual.dtype != x.dtype
+                                 or residual.device != x.device):
+        raise ValueError("the residual must be contiguous and like x")
     out = torch.empty_like(x)
     tokens = x.numel() // dim
     if tokens == 0:
@@ -275,7 +288,7 @@ def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int)
     nbytes = lib.mie_moe_prefill_workspace(tokens, num_experts, top_k, dim, hidden, code)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     rc = lib.mie_moe_prefill(
-        x.data_ptr(), tokens, router_weight.data_ptr(),
+        x.data_ptr(), tokens, ln_w, ln_b, float(eps), _native.ptr(residual), router_weight.data_ptr(),
         w1_base.data_ptr(), b1_base.data_ptr(), w2_base.data_ptr(), b2_base.data_ptr(),
         num_experts, top_k, dim, hidden, out.data_ptr(), ws.data_ptr(), nbytes, code, _native.stream_of(x),
     )

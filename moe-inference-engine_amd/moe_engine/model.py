@@ -67,6 +67,28 @@ def _tensors_replaced() -> None:
 # a module call must call the module.
 _GLOBAL_MODULE_HOOKS = (nn.modules.module._global_forward_hooks, nn.modules.module._global_forward_pre_hooks)
 
+# Prompts past this many tokens keep the PyTorch path (mie_attn_prefill's limit).
+_PROMPT_MAX_TOKENS = 1 << 19
+
+
+def _plain_module(module) -> bool:
+    """Whether calling the module runs its class's forward and nothing else."""
+    return not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+                or any(_GLOBAL_MODULE_HOOKS))
+
+
+def _like(t, shape, x) -> bool:
+    """A parameter the kernels can read beside x: this shape, x's dtype and
+    device, contiguous, 16-byte aligned."""
+    return (t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
+def _aligned(x):
+    x = x.contiguous()
+    return x.clone() if x.data_ptr() % 16 else x
+
+
 # Plain attributes a launch plan is built from: a MoE layer's mode and a
 # norm's eps.  Changing one advances _TENSOR_EPOCH like a tensor replacement.
 _PLAN_SETTINGS = ("mode", "eps")
@@ -448,7 +470,53 @@ class CachedAttention(_TracksReplacement, nn.Module):
             or not paged_attention.is_supported(x, self.head_dim)
         )
 
+    def prompt_supported(self, x, cache, layer_idx) -> bool:
+        """Whether a prompt x at position 0 can take the HIP prompt attention
+        (paged_attention.prefill): a paged cache on a ROCm device in a mode
+        that may run the direct kernels, one float32 or bfloat16 sequence whose
+        projections match the pools, unmodified modules, and nothing recorded
+        or transformed (_native.plain_inference)."""
+        alloc = getattr(cache, "allocator", None)
+        if (
+            alloc is None
+            or type(cache) is not PagedKVCache
+            or cache.attention_mode == "gather"
+            or cache.graph_pos is not None
+            or alloc._launch is None
+            or x.dim() != 3
+            or x.shape[0] != 1
+            or not 0 < x.shape[1] <= _PROMPT_MAX_TOKENS
+            or not _native.plain_inference(x)
+        ):
+            return False
+        pool, dim = alloc.k_pool, x.shape[2]
+        out = self._modules["out_proj"]
+        params = self._parameters
+        w_in, b_in = params["in_proj_weight"], params["in_proj_bias"]
+        return (
+            type(out) is Linear
+            and _plain_module(out)
+            and (alloc.num_heads, alloc.head_dim) == (self.num_heads, self.head_dim)
+            and self.num_heads * self.head_dim == dim
+            and 0 <= layer_idx < pool.shape[0]
+            and x.dtype == pool.dtype
+            and x.device == pool.device
+            and _like(w_in, (3 * dim, dim), x)
+            and (b_in is None or _like(b_in, (3 * dim,), x))
+            and _like(out.weight, (dim, dim), x)
+            and (out.bias is None or _like(out.bias, (dim,), x))
+            and paged_attention.prefill_supported(self.num_heads, self.head_dim, x.dtype)
+        )
+
+    def _prompt(self, x, cache, layer_idx, norm=None, residual=None):
+        out = self.out_proj
+        x = _aligned(x)
+        return paged_attention.prefill(x, cache, layer_idx, self.in_proj_weight, self.in_proj_bias, out.weight,
+                                       out.bias, norm=norm, residual=x if residual else None)
+
     def forward(self, x, cache, layer_idx, position: int):
+        if position == 0 and self.prompt_supported(x, cache, layer_idx):
+            return self._prompt(x, cache, layer_idx)
         batch, seq_len, dim = x.shape
         qkv = F.linear(x, self.in_proj_weight, self.in_proj_bias)
         # [batch, seq, 3*dim] -> three [batch, head, seq, head_dim] views
@@ -738,9 +806,10 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
             and (self.uses_dense_prefill(x, decode=decode) or self._experts_are_plain())
         )
 
-    def _forward_grouped(self, x: torch.Tensor) -> torch.Tensor:
+    def _forward_grouped(self, x: torch.Tensor, norm=None, residual=None) -> torch.Tensor:
         s = self._expert_storage
-        return fused_moe.prefill(x, self.router.weight, s["w1"], s["b1"], s["w2"], s["b2"], top_k=self.top_k)
+        return fused_moe.prefill(x, self.router.weight, s["w1"], s["b1"], s["w2"], s["b2"], top_k=self.top_k,
+                                 norm=norm, residual=residual)
 
     def forward(self, x, *, decode=False):
         if self.uses_direct(x, decode=decode):
@@ -831,6 +900,10 @@ class TransformerMoEBlock(nn.Module):
             out = self._decode_one_token(x, cache, layer_idx, position)
             if out is not None:
                 return out
+        if position == 0:
+            out = self._prompt(x, cache, layer_idx)
+            if out is not None:
+                return out
         h = self.attention.fused_decode(x, self.attn_norm, cache, layer_idx, position)
         if h is None:
             h = x + self.attention(self.attn_norm(x), cache, layer_idx, position)
@@ -839,6 +912,27 @@ class TransformerMoEBlock(nn.Module):
         if out is None:
             out = h + self.moe(self.moe_norm(h), decode=decode)
         return out
+
+    def _prompt(self, x, cache, layer_idx):
+        """The block over a prompt at position 0 in eight launches: the
+        attention half (paged_attention.prefill with the norm and the
+        residual), then the MoE half (fused_moe.prefill likewise).  None when
+        the two do not both apply or a module in between is not plain."""
+        m = self._modules
+        att, moe, an, mn = m["attention"], m["moe"], m["attn_norm"], m["moe_norm"]
+        if not (type(att) is CachedAttention and type(moe) is MoEFeedForward and _plain_module(att)
+                and _plain_module(moe) and att.prompt_supported(x, cache, layer_idx)):
+            return None
+        dim = x.shape[2]
+        for norm in (an, mn):
+            if not (type(norm) is LayerNorm and _plain_module(norm) and tuple(norm.normalized_shape) == (dim,)
+                    and norm.weight is not None and _like(norm.weight, (dim,), x)
+                    and (norm.bias is None or _like(norm.bias, (dim,), x))):
+                return None
+        if not moe.uses_grouped_prefill(x, decode=False):
+            return None
+        h = att._prompt(x, cache, layer_idx, norm=(an.weight, an.bias, an.eps), residual=True)
+        return moe._forward_grouped(h, norm=(mn.weight, mn.bias, mn.eps), residual=h)
 
     def _one_token_key(self, x, cache, layer_idx):
         """What a plan is built for besides the block's own tensors: the

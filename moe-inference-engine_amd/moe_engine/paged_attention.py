@@ -269,3 +269,44 @@ def decode_batched(
         max_context_len=max_context_len,
         **kwargs,
     )
+
+
+def prefill_supported(num_heads: int, head_dim: int, dtype: torch.dtype) -> bool:
+    """Whether mie_attn_prefill is built for these heads and this dtype."""
+    if not HAS_HIP or dtype not in SUPPORTED_DTYPES:
+        return False
+    return bool(_native.lib().mie_attn_prefill_supported(num_heads, head_dim, _native.dtype_code(dtype)))
+
+
+def prefill(x, cache, layer_idx, in_proj_weight, in_proj_bias, out_proj_weight, out_proj_bias, *, norm=None,
+            residual=None) -> torch.Tensor:
+    """The attention layer over a prompt x [1, S, H * D] at position 0
+    (reference model.py:226-269): K and V go into the cache's blocks (reserved
+    here), and the attention's output projection is returned, a new [1, S,
+    H * D] tensor.  With `norm` (weight, bias or None, eps) the layer runs on
+    LayerNorm(x), and `residual` (x's shape, contiguous) is added: the block's
+    x + attention(attn_norm(x)).  Three or four launches (mie_attn_prefill);
+    the caller has checked shapes, dtypes and devices
+    (CachedAttention.prompt_supported)."""
+    alloc = cache.allocator
+    tokens = x.shape[1]
+    cache._reserve(tokens)
+    layer_bytes, sblk, shead, code = alloc._launch
+    off = layer_idx * layer_bytes
+    lib = _native.lib()
+    nbytes = lib.mie_attn_prefill_workspace(tokens, alloc.num_heads, alloc.head_dim, code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    ln_w, ln_b, eps = norm if norm is not None else (None, None, 1e-5)
+    table = cache.block_table_device
+    rc = lib.mie_attn_prefill(
+        x.data_ptr(), tokens, _native.ptr(ln_w), _native.ptr(ln_b), float(eps),
+        in_proj_weight.data_ptr(), _native.ptr(in_proj_bias), out_proj_weight.data_ptr(), _native.ptr(out_proj_bias),
+        _native.ptr(residual), out.data_ptr(),
+        alloc.k_pool.data_ptr() + off, alloc.v_pool.data_ptr() + off, sblk, shead, alloc.num_blocks,
+        table.data_ptr(), table.numel(), alloc.num_heads, alloc.head_dim, alloc.block_size,
+        1.0 / math.sqrt(alloc.head_dim), ws.data_ptr(), nbytes, code, _native.stream_of(x),
+    )
+    if rc:
+        _native.check(rc, "mie_attn_prefill")
+    return out

@@ -8,7 +8,7 @@ from moe_engine.model import MoEFeedForward
 
 INVALID, UNSUPPORTED, WORKSPACE = 1, 2, 3
 F32, BF16, F64 = 0, 1, 3
-GOOD = dict(x=1 << 24, tokens=33, router=2 << 24, w1=3 << 24, b1=4 << 24, w2=5 << 24, b2=6 << 24, experts=8, top_k=2,
+GOOD = dict(x=1 << 24, tokens=33, ln_w=None, ln_b=None, eps=1e-5, residual=None, router=2 << 24, w1=3 << 24, b1=4 << 24, w2=5 << 24, b2=6 << 24, experts=8, top_k=2,
             dim=64, hidden=128, out=7 << 24, ws=8 << 24, ws_bytes=1 << 40, dtype=F32, stream=None)
 
 
@@ -19,6 +19,7 @@ GOOD = dict(x=1 << 24, tokens=33, router=2 << 24, w1=3 << 24, b1=4 << 24, w2=5 <
         (dict(experts=1, top_k=2), INVALID), (dict(dim=66), INVALID), (dict(hidden=0), INVALID),
         (dict(dim=68, dtype=BF16), INVALID), (dict(dtype=F64), UNSUPPORTED), (dict(x=0), INVALID),
         (dict(w2=(5 << 24) + 8), INVALID), (dict(out=(7 << 24) + 4), INVALID), (dict(ws_bytes=64), WORKSPACE),
+        (dict(ln_b=9 << 24), INVALID),
     ],
 )
 def test_bad_arguments_fail_before_launch(change, status):
