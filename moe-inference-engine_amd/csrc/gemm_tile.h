@@ -2,9 +2,7 @@
 // both K-contiguous ("NT"), float32 or bfloat16, accumulated in float32.
 //
 // 256 threads, four waves as WM x WN over a BM x BN tile, each wave MT x NT
-// blocks of 16 x 16; with WK > 1, WK waves share a block and each takes every
-// WK-th 64 bytes of K (their sums meet in LDS at the end): small tiles that
-// spread few rows over more workgroups.  One 16-byte LDS read per lane is one fragment: four
+// blocks of 16 x 16.  One 16-byte LDS read per lane is one fragment: four
 // v_mfma_f32_16x16x4_f32 steps of float32, or one v_mfma_f32_16x16x32_bf16.
 // A lane's fragment holds consecutive K of one row, so a float32 step j
 // multiplies K = 4 g + j of lane group g: a permutation of the contraction,
@@ -51,9 +49,9 @@ __device__ __forceinline__ f32x4 mfma_fragment<uint16_t>(u32x4 a, u32x4 b, f32x4
                                                  0, 0);
 }
 
-template <typename T, int BM_, int BN_, int KB_, int WM_, int WN_, int WK_ = 1>
+template <typename T, int BM_, int BN_, int KB_, int WM_, int WN_>
 struct Tile {
-  static constexpr int BM = BM_, BN = BN_, KB = KB_, WM = WM_, WN = WN_, WK = WK_;
+  static constexpr int BM = BM_, BN = BN_, KB = KB_, WM = WM_, WN = WN_;
   static constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
   static constexpr int kStride = KB + 16;         // LDS bytes per row
   static constexpr int kVec = KB / 16;            // 16-byte vectors per row and step
@@ -61,8 +59,7 @@ struct Tile {
   static constexpr int kA = BM / kRows, kW = BN / kRows;  // passes over the A and W rows
   static constexpr int kBuffer = (BM + BN) * kStride;
   static constexpr int kLds = 2 * kBuffer;  // bytes of LDS
-  static_assert(WM * WN * WK == 4 && KB % (64 * WK) == 0 && MT >= 1 && NT >= 1 && kA >= 1 && kW >= 1, "tile does not fit four waves");
-  static_assert(WK == 1 || 4 * NT * MT * 1024 <= 2 * (BM + BN) * (KB + 16), "sums do not fit the buffers");
+  static_assert(WM * WN == 4 && MT >= 1 && NT >= 1 && kA >= 1 && kW >= 1, "tile does not fit four waves");
   static_assert(BM % kRows == 0 && BN % kRows == 0 && KB % 64 == 0, "tile does not divide into passes");
 
   // acc[n][m] += the tile's product over row bytes [k0, k1): a_row(r) and
@@ -76,7 +73,7 @@ struct Tile {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+    const int wm = wave % WM, wn = wave / WM;
     const int vr = tid / kVec, vc = (tid % kVec) * 16;
     const char* ap[kA];
     const char* wp[kW];
@@ -109,8 +106,7 @@ struct Tile {
     const int w_frag = (BM + wn * NT * 16) * kStride + frag;
     auto multiply = [&](const char* buf) {
 #pragma unroll
-      for (int u = 0; u < KB; u += 64 * WK) {
-        const int c = u + wk * 64;
+      for (int c = 0; c < KB; c += 64) {
         u32x4 a[MT], w[NT];
 #pragma unroll
         for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const u32x4*>(buf + a_frag + m * 16 * kStride + c);
@@ -137,31 +133,6 @@ struct Tile {
       }
       lds_barrier();
     }
-    if constexpr (WK > 1) {
-      // The tile's buffers are free: the other waves' sums go there.
-      f32x4* sums = reinterpret_cast<f32x4*>(lds) + lane;
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) sums[(wave * NT * MT + n * MT + m) * 64] = acc[n][m];
-      lds_barrier();
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          acc[n][m] = sums[(wave % (WM * WN) * NT * MT + n * MT + m) * 64];
-#pragma unroll
-          for (int k = 1; k < WK; ++k)
-            acc[n][m] += sums[((wave % (WM * WN) + k * WM * WN) * NT * MT + n * MT + m) * 64];
-        }
-      lds_barrier();
-    }
-  }
-
-  // Whether this wave's results are its own to store (with WK > 1 the WK waves
-  // of a block hold the same sums).
-  static __device__ __forceinline__ bool owner() {
-    return WK == 1 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < WM * WN;
   }
 
   // Tile row and first column of the four results a lane holds in acc[n][m].
@@ -169,7 +140,7 @@ struct Tile {
     return ((__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % WM) * MT + m) * 16 + (threadIdx.x & 15);
   }
   static __device__ __forceinline__ int col(int n) {
-    return ((__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / WM % WN) * NT + n) * 16 + ((threadIdx.x & 63) >> 4) * 4;
+    return ((__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / WM) * NT + n) * 16 + ((threadIdx.x & 63) >> 4) * 4;
   }
 };
 

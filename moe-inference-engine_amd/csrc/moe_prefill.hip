@@ -39,9 +39,11 @@
 
 #include <algorithm>
 
+#include "gemm_direct.h"
 #include "gemm_tile.h"
 #include "mie_common.h"
 #include "moe_route.h"
+#include "row_norm.h"
 
 namespace {
 
@@ -79,34 +81,13 @@ struct PromptArgs {
   char* out;                  // T [tokens, dim]
 };
 
-// LayerNorm of a row by one wave (float32, biased variance), into `out`.
-template <typename T>
-__device__ __forceinline__ void norm_row(const PromptArgs& a, const T* x, T* out, int lane) {
-  float s = 0.f;
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    const f32x4_t v = Mem<T>::load4(x + i);
-    s += (v.x + v.y) + (v.z + v.w);
-  }
-  const float mean = mie::wave_sum(s) / a.dim;
-  float q = 0.f;
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    const f32x4_t d = Mem<T>::load4(x + i) - mean;
-    q = dot4(d, d, q);
-  }
-  const float rstd = rsqrtf(mie::wave_sum(q) / a.dim + a.ln_eps);
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    f32x4_t y = (Mem<T>::load4(x + i) - mean) * rstd * Mem<T>::load4(reinterpret_cast<const T*>(a.ln_w) + i);
-    if (a.ln_b) y += Mem<T>::load4(reinterpret_cast<const T*>(a.ln_b) + i);
-    Mem<T>::put4(out + i, y);
-  }
-}
-
-// grid = words * 8; four waves, two tokens each.  Bound by its memory rounds:
-// eight experts' rows and the tokens' go out together, in pieces of 768
-// elements (8 experts, dim 768: one round after the norm's).
-template <typename T>
+// grid = words * 8; four waves, two tokens each.  Bound by its memory rounds.
+// P > 0 (dim <= 256 P): the tokens' rows stay in registers, and up to
+// kRouteRows / P experts' router rows go out with them in one round.  P = 0:
+// any dim.
+constexpr int kRouteRows = 24;
+template <typename T, int P, int K>
 __global__ __launch_bounds__(256) void moe_prompt_route(PromptArgs a) {
-  constexpr int kPieces = 3;
   __shared__ unsigned int s_mask[kMaxExperts];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -117,62 +98,98 @@ __global__ __launch_bounds__(256) void moe_prompt_route(PromptArgs a) {
     const bool two = t0 + 1 < a.tokens;
     const T* x0 = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(t0) * a.dim;
     const T* x1 = two ? x0 + a.dim : x0;
-    if (a.ln_w) {
-      // Each lane reads back what it wrote itself.
-      T* y0 = reinterpret_cast<T*>(a.normed) + static_cast<int64_t>(t0) * a.dim;
-      norm_row(a, x0, y0, lane);
-      if (two) norm_row(a, x1, y0 + a.dim, lane);
-      x0 = y0;
-      x1 = two ? y0 + a.dim : y0;
-    }
+    const T* ln_w = reinterpret_cast<const T*>(a.ln_w);
+    const T* ln_b = reinterpret_cast<const T*>(a.ln_b);
+    // Without a second token its norm goes where the first's goes (the same row).
+    T* y0 = reinterpret_cast<T*>(a.normed) + static_cast<int64_t>(t0) * a.dim;
+    T* y1 = two ? y0 + a.dim : y0;
     const T* router = reinterpret_cast<const T*>(a.router);
     float l0 = -INFINITY, l1 = -INFINITY;  // lane e: expert e's logit
-    for (int e = 0; e < a.E; e += 8) {
-      float s0[8], s1[8];
+    if constexpr (P > 0) {
+      constexpr int G = kRouteRows / P;
+      typename Mem<T>::raw4 r[G][P];
+      auto load_rows = [&](int e) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s0[u] = s1[u] = 0.f;
-      for (int i0 = lane * 4; i0 < a.dim; i0 += 256 * kPieces) {
-        typename Mem<T>::raw4 v0[kPieces], v1[kPieces], r[8][kPieces];
+        for (int u = 0; u < G; ++u)
 #pragma unroll
-        for (int p = 0; p < kPieces; ++p) {
-          const int i = i0 + 256 * p < a.dim ? i0 + 256 * p : 0;  // in bounds; dropped below
-          v0[p] = Mem<T>::load_raw(x0 + i);
-          v1[p] = Mem<T>::load_raw(x1 + i);
-#pragma unroll
-          for (int u = 0; u < 8; ++u)
+          for (int p = 0; p < P; ++p) {
+            const int i = p * 256 + lane * 4 < a.dim ? p * 256 + lane * 4 : 0;  // in bounds; met by zeros
             r[u][p] = Mem<T>::load_raw(router + static_cast<int64_t>(min(e + u, a.E - 1)) * a.dim + i);
+          }
+      };
+      f32x4_t v0[P], v1[P];
+      if (a.ln_w) {
+        load_rows(0);
+        mie::norm_row<T, P>(x0, ln_w, ln_b, y0, a.dim, a.ln_eps, lane, v0);
+        mie::norm_row<T, P>(x1, ln_w, ln_b, y1, a.dim, a.ln_eps, lane, v1);
+      } else {
+        typename Mem<T>::raw4 w0[P], w1[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int i = p * 256 + lane * 4 < a.dim ? p * 256 + lane * 4 : 0;
+          w0[p] = Mem<T>::load_raw(x0 + i);
+          w1[p] = Mem<T>::load_raw(x1 + i);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        load_rows(0);
 #pragma unroll
-        for (int p = 0; p < kPieces; ++p) {
-          if (i0 + 256 * p >= a.dim) break;
+        for (int p = 0; p < P; ++p) {
+          const bool live = p * 256 + lane * 4 < a.dim;
+          v0[p] = live ? Mem<T>::widen(w0[p]) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+          v1[p] = live ? Mem<T>::widen(w1[p]) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      for (int e = 0; e < a.E; e += G) {
+        if (e > 0) load_rows(e);
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            s0[u] = dot4(Mem<T>::widen(r[u][p]), Mem<T>::widen(v0[p]), s0[u]);
-            s1[u] = dot4(Mem<T>::widen(r[u][p]), Mem<T>::widen(v1[p]), s1[u]);
+        for (int u = 0; u < G; ++u) {
+          float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            if (p * 256 + lane * 4 >= a.dim) continue;
+            s0 = dot4(Mem<T>::widen(r[u][p]), v0[p], s0);
+            s1 = dot4(Mem<T>::widen(r[u][p]), v1[p], s1);
+          }
+          s0 = mie::wave_sum(s0);
+          s1 = mie::wave_sum(s1);
+          if (lane == e + u && e + u < a.E) {
+            l0 = s0;
+            l1 = s1;
           }
         }
       }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float d0 = mie::wave_sum(s0[u]), d1 = mie::wave_sum(s1[u]);
-        if (lane == e + u && e + u < a.E) {
-          l0 = d0;
-          l1 = d1;
+    } else {
+      if (a.ln_w) {  // each lane reads back what it wrote itself
+        mie::norm_row<T, 0>(x0, ln_w, ln_b, y0, a.dim, a.ln_eps, lane);
+        mie::norm_row<T, 0>(x1, ln_w, ln_b, y1, a.dim, a.ln_eps, lane);
+        x0 = y0;
+        x1 = y1;
+      }
+      for (int e = 0; e < a.E; ++e) {
+        float s0 = 0.f, s1 = 0.f;
+        for (int i = lane * 4; i < a.dim; i += 256) {
+          const f32x4_t r = Mem<T>::load4(router + static_cast<int64_t>(e) * a.dim + i);
+          s0 = dot4(r, Mem<T>::load4(x0 + i), s0);
+          s1 = dot4(r, Mem<T>::load4(x1 + i), s1);
+        }
+        s0 = mie::wave_sum(s0);
+        s1 = mie::wave_sum(s1);
+        if (lane == e) {
+          l0 = s0;
+          l1 = s1;
         }
       }
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if (j == 1 && !two) break;
-      int ids[kMaxTopK];
-      float p[kMaxTopK];
-      wave_topk(j ? l1 : l0, a.top_k, a.E, lane, ids, p);
+      int ids[K];
+      float p[K];
+      wave_topk<K>(j ? l1 : l0, a.top_k, a.E, lane, ids, p);
 #pragma unroll
-      for (int kk = 0; kk < kMaxTopK; ++kk) {
+      for (int kk = 0; kk < K; ++kk) {
         int rank = 0;  // place in increasing expert id (ids are distinct)
 #pragma unroll
-        for (int o = 0; o < kMaxTopK; ++o) rank += o < a.top_k && ids[o] < ids[kk];
+        for (int o = 0; o < K; ++o) rank += o < a.top_k && ids[o] < ids[kk];
         if (kk < a.top_k && lane == kk) {
           const int64_t at = static_cast<int64_t>(t0 + j) * a.top_k + rank;
           a.ids[at] = ids[kk];
@@ -198,8 +215,8 @@ __device__ __forceinline__ int wave_inclusive(int v, int lane) {
   return v;
 }
 
-// The rows a workgroup works on: expert e's rows [m0, count) (only the first
-// BM of them in the row-tile form), the expert's first slot.
+// The rows a workgroup works on: expert e's rows from m0 (of `count`: up to
+// one tile of them, or all in the few-rows form), the expert's first slot.
 struct Rows {
   int e, m0, count, base;
 };
@@ -228,7 +245,45 @@ __device__ __forceinline__ Rows find_rows(const PromptArgs& a, int cnt, int bm, 
   return r;
 }
 
-// grid = (ceil(hidden / BN), experts or row tiles).
+// Token counts of the eight experts from e0 (their mask words `word`, one per
+// lane) into lanes e0 .. e0 + 7 of cnt.
+__device__ __forceinline__ int count_tokens(const PromptArgs& a, const unsigned long long (&word)[8], int e0, int lane,
+                                            int cnt) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    int c = lane < a.words ? __popcll(word[u]) : 0;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
+    cnt = lane == e0 + u && e0 + u < a.E ? c : cnt;
+  }
+  return cnt;
+}
+
+// One wave lists an expert's tokens of ranks m0 .. m0 + BM - 1 (its mask, and
+// the rank of each word's first token); entries past the expert's last token
+// repeat the first listed one (their results are dropped).
+template <int BM>
+__device__ __forceinline__ void list_rows(unsigned long long mask, int first, int m0, int count, int lane, int* rows) {
+  unsigned long long word = mask;
+  for (int rank = first - m0; word != 0ull && rank < BM; ++rank, word &= word - 1ull) {
+    const int token = lane * 64 + __ffsll(word) - 1;
+    if (rank >= 0) rows[rank] = token;
+    if (rank == 0)
+      for (int i = min(BM, count - m0); i < BM; ++i) rows[i] = token;
+  }
+}
+
+// Records where token's output of expert e is, for the combining launch.
+__device__ __forceinline__ void keep_slot(const PromptArgs& a, int token, int e, int slot) {
+  for (int j = 0; j < a.top_k; ++j) {
+    const int64_t at = static_cast<int64_t>(token) * a.top_k + j;
+    if (a.ids[at] == e) a.slots[at] = slot;
+  }
+}
+
+__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752440f)); }
+
+// grid = (ceil(hidden / BN), row tiles).
 template <typename T, typename Tile>
 __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   __shared__ __align__(16) char lds[Tile::kLds];
@@ -237,18 +292,12 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Every wave counts every expert's tokens: eight masks in one memory round.
   int cnt = 0;  // lane e: expert e's
-  for (int e = 0; e < a.E; e += 8) {
+  for (int e0 = 0; e0 < a.E; e0 += 8) {
     unsigned long long word[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      word[u] = a.masks[static_cast<int64_t>(min(e + u, a.E - 1)) * a.words + min(lane, a.words - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      int c = lane < a.words ? __popcll(word[u]) : 0;
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
-      if (lane == e + u && e + u < a.E) cnt = c;
-    }
+      word[u] = a.masks[static_cast<int64_t>(min(e0 + u, a.E - 1)) * a.words + min(lane, a.words - 1)];
+    cnt = count_tokens(a, word, e0, lane, cnt);
   }
   if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
   const Rows r = find_rows(a, cnt, Tile::BM, lane);
@@ -261,59 +310,36 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   const char* x = a.ln_w ? a.normed : a.x;
   const char* w = a.w1 + static_cast<int64_t>(r.e) * a.hidden * row_bytes;
   const T* bias = reinterpret_cast<const T*>(a.b1) + static_cast<int64_t>(r.e) * a.hidden;
-  const int m_end = a.per_expert ? r.count : min(r.count, r.m0 + Tile::BM);
-  for (int m0 = r.m0; m0 < m_end; m0 += Tile::BM) {
-    // The tile's tokens, by rank.  Ranks past the expert's last repeat its
-    // first token of the tile (their results are dropped).
-    if (wave == 0) {
-      const int live = min(Tile::BM, r.count - m0);
-      unsigned long long word = mask;
-      for (int rank = first - m0; word != 0ull && rank < Tile::BM; ++rank, word &= word - 1ull) {
-        const int token = lane * 64 + __ffsll(word) - 1;
-        if (rank >= 0) s_rows[rank] = token;
-        if (rank == 0)
-          for (int i = live; i < Tile::BM; ++i) s_rows[i] = token;
-      }
+  if (wave == 0) list_rows<Tile::BM>(mask, first, r.m0, r.count, lane, s_rows);
+  __syncthreads();
+  f32x4 acc[Tile::NT][Tile::MT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n)
+#pragma unroll
+    for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Tile::run(
+      lds, [&](int i) { return x + s_rows[i] * row_bytes; },
+      [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n) {
+    const int c = n0 + Tile::col(n);
+    if (c >= a.hidden) continue;  // hidden is a multiple of 4: all four columns or none
+    const f32x4_t b = Mem<T>::load4(bias + c);
+#pragma unroll
+    for (int m = 0; m < Tile::MT; ++m) {
+      const int rank = r.m0 + Tile::row(m);
+      if (rank >= r.count) continue;
+      f32x4_t v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = gelu(Mem<T>::R(acc[n][m][i] + b[i]));  // of the Linear's output
+      Mem<T>::put4(reinterpret_cast<T*>(a.h) + static_cast<int64_t>(r.base + rank) * a.hidden + c, v);
     }
-    __syncthreads();
-    f32x4 acc[Tile::NT][Tile::MT];
-#pragma unroll
-    for (int n = 0; n < Tile::NT; ++n)
-#pragma unroll
-      for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Tile::run(
-        lds, [&](int i) { return x + s_rows[i] * row_bytes; },
-        [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
-#pragma unroll
-    for (int n = 0; n < Tile::NT; ++n) {
-      const int c = n0 + Tile::col(n);
-      if (c >= a.hidden) continue;  // hidden is a multiple of 4: all four columns or none
-      const f32x4_t b = Mem<T>::load4(bias + c);
-#pragma unroll
-      for (int m = 0; m < Tile::MT; ++m) {
-        const int rank = m0 + Tile::row(m);
-        if (rank >= r.count) continue;
-        f32x4_t v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pre = Mem<T>::R(acc[n][m][i] + b[i]);  // the Linear's output
-          v[i] = 0.5f * pre * (1.f + erff(pre * 0.70710678118654752440f));
-        }
-        Mem<T>::put4(reinterpret_cast<T*>(a.h) + static_cast<int64_t>(r.base + rank) * a.hidden + c, v);
-      }
-    }
-    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < min(Tile::BM, r.count - m0)) {
-      const int token = s_rows[threadIdx.x];
-      for (int j = 0; j < a.top_k; ++j) {
-        const int64_t at = static_cast<int64_t>(token) * a.top_k + j;
-        if (a.ids[at] == r.e) a.slots[at] = r.base + m0 + threadIdx.x;
-      }
-    }
-    __syncthreads();  // s_rows is rewritten by the next tile
   }
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < min(Tile::BM, r.count - r.m0))
+    keep_slot(a, s_rows[threadIdx.x], r.e, r.base + r.m0 + threadIdx.x);
 }
 
-// grid = (ceil(dim / BN) * splits, experts or row tiles); blockIdx.x is
+// grid = (ceil(dim / BN) * splits, row tiles); blockIdx.x is
 // column tile * splits + split.
 template <typename T, typename Tile>
 __global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
@@ -329,25 +355,22 @@ __global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
   const char* w = a.w2 + static_cast<int64_t>(r.e) * a.dim * row_bytes;
   const char* h = a.h + r.base * row_bytes;
   float* part = a.part + (static_cast<int64_t>(split) * a.tokens * a.top_k + r.base) * a.dim;
-  const int m_end = a.per_expert ? r.count : min(r.count, r.m0 + Tile::BM);
-  for (int m0 = r.m0; m0 < m_end; m0 += Tile::BM) {
-    f32x4 acc[Tile::NT][Tile::MT];
+  f32x4 acc[Tile::NT][Tile::MT];
 #pragma unroll
-    for (int n = 0; n < Tile::NT; ++n)
+  for (int n = 0; n < Tile::NT; ++n)
 #pragma unroll
-      for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Tile::run(
-        lds, [&](int i) { return h + min(m0 + i, r.count - 1) * row_bytes; },
-        [&](int i) { return w + min(n0 + i, a.dim - 1) * row_bytes; }, k0, k1, acc);
+    for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Tile::run(
+      lds, [&](int i) { return h + min(r.m0 + i, r.count - 1) * row_bytes; },
+      [&](int i) { return w + min(n0 + i, a.dim - 1) * row_bytes; }, k0, k1, acc);
 #pragma unroll
-    for (int n = 0; n < Tile::NT; ++n) {
-      const int c = n0 + Tile::col(n);
-      if (c >= a.dim) continue;
+  for (int n = 0; n < Tile::NT; ++n) {
+    const int c = n0 + Tile::col(n);
+    if (c >= a.dim) continue;
 #pragma unroll
-      for (int m = 0; m < Tile::MT; ++m) {
-        const int rank = m0 + Tile::row(m);
-        if (rank < r.count) *reinterpret_cast<f32x4*>(part + static_cast<int64_t>(rank) * a.dim + c) = acc[n][m];
-      }
+    for (int m = 0; m < Tile::MT; ++m) {
+      const int rank = r.m0 + Tile::row(m);
+      if (rank < r.count) *reinterpret_cast<f32x4*>(part + static_cast<int64_t>(rank) * a.dim + c) = acc[n][m];
     }
   }
 }
@@ -407,30 +430,146 @@ __global__ __launch_bounds__(256) void moe_prompt_combine(PromptArgs a, mie::Fas
   Mem<T>::put4(reinterpret_cast<T*>(a.out) + here, out);
 }
 
-// Tiles.  Narrow: up to 32 rows per expert on average, where the launch streams
-// the experts' weights: one workgroup per (expert, column tile), 256 bytes of
-// every row in flight.  Wide: more rows.
-template <typename T> using Narrow = mie::gemm::Tile<T, 32, 64, 256, 1, 4>;
+// ---- few rows per expert -----------------------------------------------------
+// The two products where the launch streams the experts' weights: one
+// workgroup per (expert, 32 columns), direct tiles (gemm_direct.h), 32 or 16
+// rows at a time.  The expert is known from blockIdx, so two windows of its
+// weights (2048 bytes of each row) are in flight before the routing is read.
+template <typename T> using Few = mie::gemm::Direct<T, 2, 4>;
+
+// grid = (ceil(hidden / 32), E).
+template <typename T>
+__global__ __launch_bounds__(256, 2) void moe_prompt_w1_few(PromptArgs a) {
+  using Tile = Few<T>;
+  __shared__ __align__(16) char lds[Tile::template kLds<2>];
+  __shared__ int s_rows[32];
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = blockIdx.y, n0 = blockIdx.x * Tile::BN;
+  const int row_bytes = a.dim * static_cast<int>(sizeof(T));
+  const unsigned long long mask = lane < a.words ? a.masks[static_cast<int64_t>(e) * a.words + lane] : 0ull;
+  unsigned long long word[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    word[u] = a.masks[static_cast<int64_t>(min(u, a.E - 1)) * a.words + min(lane, a.words - 1)];
+  const char* wp[Tile::NT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n)
+    wp[n] = a.w1 + (static_cast<int64_t>(e) * a.hidden + min(n0 + n * 16 + i, a.hidden - 1)) * row_bytes;
+  typename Tile::template Set<Tile::NT> ws[2];
+  Tile::prefetch(ws, wp, 0, row_bytes);
+  __builtin_amdgcn_sched_barrier(0);
+  int cnt = count_tokens(a, word, 0, lane, 0);
+  for (int e0 = 8; e0 < a.E; e0 += 8) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      word[u] = a.masks[static_cast<int64_t>(min(e0 + u, a.E - 1)) * a.words + min(lane, a.words - 1)];
+    cnt = count_tokens(a, word, e0, lane, cnt);
+  }
+  if (blockIdx.x == 0 && e == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
+  const Rows r = find_rows(a, cnt, 32, lane);
+  if (r.e < 0) return;
+  const int bits = __popcll(mask);
+  const int rank0 = wave_inclusive(bits, lane) - bits;
+  const char* x = a.ln_w ? a.normed : a.x;
+  f32x4_t bias[Tile::NT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n)
+    bias[n] = Mem<T>::load4(reinterpret_cast<const T*>(a.b1) + static_cast<int64_t>(e) * a.hidden +
+                            min(n0 + n * 16 + g * 4, a.hidden - 4));
+  for (int m0 = 0; m0 < r.count; m0 += 32) {
+    if (m0 > 0) {
+      __syncthreads();  // the last tile's rows and sums are read
+      Tile::prefetch(ws, wp, 0, row_bytes);
+    }
+    if (wave == 0) list_rows<32>(mask, rank0, m0, r.count, lane, s_rows);
+    mie::gemm::lds_barrier();
+    auto store = [&](int n, int m, f32x4 sum) {
+      const int c = n0 + n * 16 + g * 4, rank = m0 + m * 16 + i;
+      if (c >= a.hidden || rank >= r.count) return;
+      f32x4_t v;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = gelu(Mem<T>::R(sum[u] + bias[n][u]));
+      Mem<T>::put4(reinterpret_cast<T*>(a.h) + static_cast<int64_t>(r.base + rank) * a.hidden + c, v);
+    };
+    if (r.count - m0 > 16) {
+      const char* ap[2] = {x + static_cast<int64_t>(s_rows[i]) * row_bytes,
+                           x + static_cast<int64_t>(s_rows[16 + i]) * row_bytes};
+      Tile::template run<2>(lds, ws, ap, wp, 0, row_bytes, store);
+    } else {
+      const char* ap[1] = {x + static_cast<int64_t>(s_rows[i]) * row_bytes};
+      Tile::template run<1>(lds, ws, ap, wp, 0, row_bytes, store);
+    }
+    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < min(32, r.count - m0))
+      keep_slot(a, s_rows[threadIdx.x], e, r.base + m0 + threadIdx.x);
+  }
+}
+
+// grid = (ceil(dim / 32) * splits, E); blockIdx.x is column tile * splits + split.
+template <typename T>
+__global__ __launch_bounds__(256, 2) void moe_prompt_w2_few(PromptArgs a) {
+  using Tile = Few<T>;
+  __shared__ __align__(16) char lds[Tile::template kLds<2>];
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int e = blockIdx.y, n0 = blockIdx.x / a.splits * Tile::BN, split = blockIdx.x % a.splits;
+  const int row_bytes = a.hidden * static_cast<int>(sizeof(T));
+  const int k0 = split * a.split_len, k1 = min(row_bytes, k0 + a.split_len);
+  const int cnt = a.counts[min(lane, a.E - 1)];
+  const char* wp[Tile::NT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n)
+    wp[n] = a.w2 + (static_cast<int64_t>(e) * a.dim + min(n0 + n * 16 + i, a.dim - 1)) * row_bytes;
+  typename Tile::template Set<Tile::NT> ws[2];
+  Tile::prefetch(ws, wp, k0, k1);
+  __builtin_amdgcn_sched_barrier(0);
+  const Rows r = find_rows(a, lane < a.E ? cnt : 0, 32, lane);
+  if (r.e < 0) return;
+  const char* h = a.h + static_cast<int64_t>(r.base) * row_bytes;
+  float* part = a.part + (static_cast<int64_t>(split) * a.tokens * a.top_k + r.base) * a.dim;
+  for (int m0 = 0; m0 < r.count; m0 += 32) {
+    if (m0 > 0) {
+      __syncthreads();
+      Tile::prefetch(ws, wp, k0, k1);
+    }
+    auto store = [&](int n, int m, f32x4 sum) {
+      const int c = n0 + n * 16 + g * 4, rank = m0 + m * 16 + i;
+      if (c < a.dim && rank < r.count) *reinterpret_cast<f32x4*>(part + static_cast<int64_t>(rank) * a.dim + c) = sum;
+    };
+    const char* ap[2] = {h + static_cast<int64_t>(min(m0 + i, r.count - 1)) * row_bytes,
+                         h + static_cast<int64_t>(min(m0 + 16 + i, r.count - 1)) * row_bytes};
+    if (r.count - m0 > 16) {
+      Tile::template run<2>(lds, ws, ap, wp, k0, k1, store);
+    } else {
+      const char* one[1] = {ap[0]};
+      Tile::template run<1>(lds, ws, one, wp, k0, k1, store);
+    }
+  }
+}
+
+// More rows: LDS-staged tiles of 64 x 64.
 template <typename T> using Wide = mie::gemm::Tile<T, 64, 64, 128, 2, 2>;
 
 struct Plan {
-  bool narrow;
+  bool few;
   int32_t rows;               // blockIdx.y extent
   int32_t splits, split_len;  // W2
 };
 
+// Few rows: up to 20 per expert on average.  At 16 (62 tokens, 8 experts,
+// top-2, float32) both forms take 36-38 us for the two products, at 8 the
+// direct tiles 29 against 35 us, at 32 the staged ones 50 against 62 us.
 Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden, int elt) {
   Plan p;
   const int64_t slots = static_cast<int64_t>(tokens) * top_k;
-  p.narrow = slots <= 24 * static_cast<int64_t>(E);
-  const int bm = p.narrow ? 32 : 64, kb = p.narrow ? 256 : 128;
-  p.rows = p.narrow ? E : static_cast<int32_t>(slots / bm + std::min<int64_t>(E, slots));
+  p.few = slots <= 20 * static_cast<int64_t>(E);
+  const int bn = p.few ? 32 : 64, kb = p.few ? 1024 : 128;
+  p.rows = p.few ? E : static_cast<int32_t>(slots / 64 + std::min<int64_t>(E, slots));
   // W2 has few column tiles: split its K until the launch holds about two
-  // (narrow) or four (wide) workgroups per CU.
-  const int64_t used = p.narrow ? std::min<int64_t>(E, slots) : slots / bm + E / 2;
-  const int64_t groups = static_cast<int64_t>((dim + 63) / 64) * std::max<int64_t>(1, used);
+  // (few rows) or four workgroups per CU.
+  const int64_t used = p.few ? std::min<int64_t>(E, slots) : slots / 64 + E / 2;
+  const int64_t groups = static_cast<int64_t>((dim + bn - 1) / bn) * std::max<int64_t>(1, used);
   const int32_t steps = (hidden * elt + kb - 1) / kb;
-  const int64_t want = ((p.narrow ? 512 : 1024) + groups - 1) / groups;
+  const int64_t want = ((p.few ? 512 : 1024) + groups - 1) / groups;
   const int32_t splits = static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>({want, kMaxSplits, steps / 2})));
   p.split_len = (steps + splits - 1) / splits * kb;
   p.splits = (hidden * elt + p.split_len - 1) / p.split_len;
@@ -459,21 +598,34 @@ int64_t layout(PromptArgs& a, const Plan& p, int elt, char* base) {
   return at;
 }
 
+template <typename T, int K>
+void launch_route(const PromptArgs& a, hipStream_t st) {
+  const int groups = a.words * 8;
+  if (a.dim <= 768) {
+    moe_prompt_route<T, 3, K><<<groups, 256, 0, st>>>(a);
+  } else if (a.dim <= 1024) {
+    moe_prompt_route<T, 4, K><<<groups, 256, 0, st>>>(a);
+  } else {
+    moe_prompt_route<T, 0, K><<<groups, 256, 0, st>>>(a);
+  }
+}
+
 template <typename T>
 int32_t launch(const PromptArgs& a, const Plan& p, hipStream_t st) {
-  moe_prompt_route<T><<<a.words * 8, 256, 0, st>>>(a);
+  a.top_k <= 2 ? launch_route<T, 2>(a, st) : launch_route<T, kMaxTopK>(a, st);
   int32_t rc = mie::check_launch("moe_prompt_route");
   if (rc != MIE_OK) return rc;
-  const dim3 g1((a.hidden + 63) / 64, p.rows), g2((a.dim + 63) / 64 * p.splits, p.rows);
-  if (p.narrow) {
-    moe_prompt_w1<T, Narrow<T>><<<g1, 256, 0, st>>>(a);
+  const int bn = p.few ? 32 : 64;
+  const dim3 g1((a.hidden + bn - 1) / bn, p.rows), g2((a.dim + bn - 1) / bn * p.splits, p.rows);
+  if (p.few) {
+    moe_prompt_w1_few<T><<<g1, 256, 0, st>>>(a);
   } else {
     moe_prompt_w1<T, Wide<T>><<<g1, 256, 0, st>>>(a);
   }
   rc = mie::check_launch("moe_prompt_w1");
   if (rc != MIE_OK) return rc;
-  if (p.narrow) {
-    moe_prompt_w2<T, Narrow<T>><<<g2, 256, 0, st>>>(a);
+  if (p.few) {
+    moe_prompt_w2_few<T><<<g2, 256, 0, st>>>(a);
   } else {
     moe_prompt_w2<T, Wide<T>><<<g2, 256, 0, st>>>(a);
   }
@@ -567,7 +719,7 @@ extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ln
     a.w2 = static_cast<const char*>(w2);
     a.b2 = static_cast<const char*>(b2);
     a.out = static_cast<char*>(out) + t0 * dim * elt;
-    a.per_expert = p.narrow;
+    a.per_expert = p.few;
     a.splits = p.splits;
     a.split_len = p.split_len;
     const hipStream_t st = static_cast<hipStream_t>(stream);

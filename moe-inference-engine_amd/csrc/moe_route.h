@@ -53,13 +53,14 @@ __device__ __forceinline__ void topk_dpp(float& v, int& i) {
 // Top-k over a wave: lane e holds expert e's logit (-inf for lanes >= E).
 // Round kk takes the largest logit not yet taken, the lower expert id on ties;
 // ids and weights (the softmax of the selected logits) come out uniform across
-// the wave.  Fixed-size loops keep both arrays in registers.
+// the wave.  Fixed-size loops keep both arrays in registers; top_k <= K.
+template <int K = kMaxTopK>
 __device__ __forceinline__ void wave_topk(float logit, int top_k, int num_experts, int lane, int* ids,
                                           float* weights) {
   bool taken = false;
-  float vals[kMaxTopK];
+  float vals[K];
 #pragma unroll
-  for (int kk = 0; kk < kMaxTopK; ++kk) {
+  for (int kk = 0; kk < K; ++kk) {
     ids[kk] = 0;
     vals[kk] = 0.f;
     if (kk < top_k) {
@@ -86,12 +87,12 @@ __device__ __forceinline__ void wave_topk(float logit, int top_k, int num_expert
   // softmax over the selected logits; vals[0] is their maximum
   float sum = 0.f;
 #pragma unroll
-  for (int kk = 0; kk < kMaxTopK; ++kk) {
+  for (int kk = 0; kk < K; ++kk) {
     weights[kk] = kk < top_k ? expf(vals[kk] - vals[0]) : 0.f;
     sum += weights[kk];
   }
 #pragma unroll
-  for (int kk = 0; kk < kMaxTopK; ++kk) weights[kk] /= sum;
+  for (int kk = 0; kk < K; ++kk) weights[kk] /= sum;
 }
 
 }  // namespace route

@@ -19,7 +19,7 @@
 // tokens bfloat16 85 -> 25 us; with the MoE half, 62 tokens float32 through 12
 // blocks and the head 4.1 -> 1.1 ms.
 //
-// Attention.  One workgroup per (head, 16 * QT queries); its four waves take
+// Attention.  One workgroup per (head, 16 queries); its four waves take
 // every fourth block of 32 keys and merge their softmax states in LDS once.
 // Nothing else is shared, so there is no barrier in the loop.  Scores are
 // computed transposed, S^T = K Q^T, so a lane holds four consecutive keys of
@@ -31,12 +31,15 @@
 
 #include <algorithm>
 
+#include "gemm_direct.h"
 #include "gemm_tile.h"
 #include "mie_common.h"
+#include "row_norm.h"
 
 namespace {
 
 using mie::Mem;
+using mie::gemm::Direct;
 using mie::gemm::f32x4;
 using mie::gemm::Tile;
 using mie::gemm::u32x4;
@@ -54,31 +57,16 @@ struct NormArgs {
   float eps;
 };
 
-// grid = ceil(rows / 4): one wave per row (float32, biased variance).
-template <typename T>
+// grid = ceil(rows / 4): one wave per row (float32, biased variance), the row
+// and the parameters in registers (one memory round), P pieces of 256 elements.
+template <typename T, int P>
 __global__ __launch_bounds__(256) void prompt_norm_kernel(NormArgs a) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= a.rows) return;
   const T* x = reinterpret_cast<const T*>(a.x) + static_cast<int64_t>(row) * a.dim;
-  T* out = reinterpret_cast<T*>(a.out) + static_cast<int64_t>(row) * a.dim;
-  float s = 0.f;
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    const f32x4 v = Mem<T>::load4(x + i);
-    s += (v.x + v.y) + (v.z + v.w);
-  }
-  const float mean = mie::wave_sum(s) / a.dim;
-  float q = 0.f;
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    const f32x4 d = Mem<T>::load4(x + i) - mean;
-    q += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
-  }
-  const float rstd = rsqrtf(mie::wave_sum(q) / a.dim + a.eps);
-  for (int i = lane * 4; i < a.dim; i += 256) {
-    f32x4 y = (Mem<T>::load4(x + i) - mean) * rstd * Mem<T>::load4(reinterpret_cast<const T*>(a.w) + i);
-    if (a.b) y += Mem<T>::load4(reinterpret_cast<const T*>(a.b) + i);
-    Mem<T>::put4(out + i, y);
-  }
+  mie::norm_row<T, P>(x, reinterpret_cast<const T*>(a.w), reinterpret_cast<const T*>(a.b),
+                      reinterpret_cast<T*>(a.out) + static_cast<int64_t>(row) * a.dim, a.dim, a.eps, lane);
 }
 
 struct LinearArgs {
@@ -98,6 +86,38 @@ struct LinearArgs {
   mie::FastDiv block, head;  // block size, head_dim
 };
 
+// The pool block of row r (token r) in the QKV form; -1 when it is not stored.
+__device__ __forceinline__ int32_t block_of(const LinearArgs& a, int r) {
+  if (!a.k_pool) return -1;
+  const int32_t id = a.table[a.block.div(min(r, a.rows - 1))];
+  return id < a.num_blocks ? id : -1;
+}
+
+// Stores four consecutive results of row r, columns c .. c + 3 (before bias);
+// blk is block_of(r).
+template <typename T>
+__device__ __forceinline__ void store_linear(const LinearArgs& a, int r, int c, f32x4 sum, f32x4 bias, int32_t blk) {
+  f32x4 v = Mem<T>::R4(sum + bias);
+  const int64_t at = static_cast<int64_t>(r) * a.n + c;
+  if (a.residual) v = Mem<T>::load4(reinterpret_cast<const T*>(a.residual) + at) + v;
+  Mem<T>::put4(reinterpret_cast<T*>(a.out) + at, v);
+  if (blk >= 0 && c >= a.dim) {
+    const int d = c < 2 * a.dim ? c - a.dim : c - 2 * a.dim;
+    char* pool = c < 2 * a.dim ? a.k_pool : a.v_pool;
+    const uint32_t h = a.head.div(d), slot = r - a.block.div(r) * a.block.d;
+    Mem<T>::put4(reinterpret_cast<T*>(pool) + blk * a.sblk + h * a.shead + static_cast<int64_t>(slot) * a.head_dim +
+                     (d - h * a.head_dim),
+                 v);
+  }
+}
+
+// Bias of columns c .. c + 3 (zeros without a bias or past the edge).
+template <typename T>
+__device__ __forceinline__ f32x4 bias_of(const LinearArgs& a, int c) {
+  if (!a.bias || c >= a.n) return f32x4{0.f, 0.f, 0.f, 0.f};
+  return Mem<T>::load4(reinterpret_cast<const T*>(a.bias) + c);
+}
+
 // grid = (ceil(n / BN), ceil(rows / BM)).
 template <typename T, typename Tile>
 __global__ __launch_bounds__(256) void prompt_linear_kernel(LinearArgs a) {
@@ -112,33 +132,47 @@ __global__ __launch_bounds__(256) void prompt_linear_kernel(LinearArgs a) {
   Tile::run(
       lds, [&](int i) { return a.x + min(m0 + i, a.rows - 1) * row_bytes; },
       [&](int i) { return a.w + min(n0 + i, a.n - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
-  if (!Tile::owner()) return;
+  int32_t blk[Tile::MT];
+#pragma unroll
+  for (int m = 0; m < Tile::MT; ++m) blk[m] = block_of(a, m0 + Tile::row(m));
 #pragma unroll
   for (int n = 0; n < Tile::NT; ++n) {
     const int c = n0 + Tile::col(n);
     if (c >= a.n) continue;  // n is a multiple of 4
-    f32x4 b = {0.f, 0.f, 0.f, 0.f};
-    if (a.bias) b = Mem<T>::load4(reinterpret_cast<const T*>(a.bias) + c);
+    const f32x4 b = bias_of<T>(a, c);
 #pragma unroll
     for (int m = 0; m < Tile::MT; ++m) {
       const int r = m0 + Tile::row(m);
-      if (r >= a.rows) continue;
-      f32x4 v = Mem<T>::R4(acc[n][m] + b);
-      const int64_t at = static_cast<int64_t>(r) * a.n + c;
-      if (a.residual) v = Mem<T>::load4(reinterpret_cast<const T*>(a.residual) + at) + v;
-      Mem<T>::put4(reinterpret_cast<T*>(a.out) + at, v);
-      if (a.k_pool && c >= a.dim) {
-        const int d = c < 2 * a.dim ? c - a.dim : c - 2 * a.dim;
-        char* pool = c < 2 * a.dim ? a.k_pool : a.v_pool;
-        const uint32_t blk = a.block.div(r), h = a.head.div(d);
-        const int32_t id = a.table[blk];
-        if (id >= 0 && id < a.num_blocks)
-          Mem<T>::put4(reinterpret_cast<T*>(pool) + id * a.sblk + h * a.shead +
-                           static_cast<int64_t>(r - blk * a.block.d) * a.head_dim + (d - h * a.head_dim),
-                       v);
-      }
+      if (r < a.rows) store_linear<T>(a, r, c, acc[n][m], b, blk[m]);
     }
   }
+}
+
+// grid = (ceil(n / BN), ceil(rows / (16 MT))): few rows.
+template <typename T, typename Tile, int MT>
+__global__ __launch_bounds__(256, 2) void prompt_linear_direct_kernel(LinearArgs a) {
+  __shared__ __align__(16) char lds[Tile::template kLds<MT>];
+  const int n0 = blockIdx.x * Tile::BN, m0 = blockIdx.y * MT * 16;
+  const int row_bytes = a.k * static_cast<int>(sizeof(T));
+  const int i = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  const char *ap[MT], *wp[Tile::NT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n) wp[n] = a.w + static_cast<int64_t>(min(n0 + n * 16 + i, a.n - 1)) * row_bytes;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) ap[m] = a.x + static_cast<int64_t>(min(m0 + m * 16 + i, a.rows - 1)) * row_bytes;
+  typename Tile::template Set<Tile::NT> ws[2];
+  Tile::prefetch(ws, wp, 0, row_bytes);
+  // What the epilogue needs goes out with the operands.
+  f32x4 bias[Tile::NT];
+  int32_t blk[MT];
+#pragma unroll
+  for (int n = 0; n < Tile::NT; ++n) bias[n] = bias_of<T>(a, n0 + n * 16 + g * 4);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) blk[m] = block_of(a, m0 + m * 16 + i);
+  Tile::template run<MT>(lds, ws, ap, wp, 0, row_bytes, [&](int n, int m, f32x4 sum) {
+    const int c = n0 + n * 16 + g * 4, r = m0 + m * 16 + i;
+    if (c < a.n && r < a.rows) store_linear<T>(a, r, c, sum, bias[n], blk[m]);  // n is a multiple of 4
+  });
 }
 
 struct AttnArgs {
@@ -210,143 +244,150 @@ template <int VEC> struct ValueGroup<uint16_t, VEC> {
   }
 };
 
-// grid = (heads, ceil(rows / (16 QT))); the tiles with the most keys first.
-template <typename T, int D, int QT>
-__global__ __launch_bounds__(256) void prompt_attention_kernel(AttnArgs a) {
+// grid = (heads, ceil(rows / 16)).  Sixteen queries per workgroup rather than
+// 32: 1000 tokens x 12 heads make 756 workgroups instead of 384 (28.8 against
+// 33.6 us, float32).  Tiles with more keys take longer, and that many
+// workgroups are resident at once, dealt to the CUs in order: the first third
+// of the grid takes the longest tiles, longest first, the second third the
+// shortest, shortest first, so a CU's workgroups add up to about the same
+// (27.4 against 30.0 us longest first throughout).
+template <typename T, int D>
+__global__ __launch_bounds__(256, D <= 64 ? 3 : 2) void prompt_attention_kernel(AttnArgs a) {
   constexpr int NCH = D * static_cast<int>(sizeof(T)) / 64;  // 64-byte pieces of a row
   constexpr int G4 = D / 64, G2 = D % 64 / 32;               // 64- and 32-dim groups
   constexpr int NO = G4 * 4 + G2 * 2;                        // 16-dim blocks
-  constexpr int Q = 16 * QT;
+  constexpr int Q = 16;
   __shared__ float s_max[4][Q], s_sum[4][Q];
   __shared__ __align__(16) float s_out[4][Q][D + 4];
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = blockIdx.x;
-  const int q0 = (gridDim.y - 1 - blockIdx.y) * Q;
-  const int64_t stride = static_cast<int64_t>(3) * a.dim;
-  const T* base = reinterpret_cast<const T*>(a.qkv) + h * D;
+  const int tiles = gridDim.y, third = (tiles + 2) / 3, y = blockIdx.y;
+  const int q0 = (y < third ? tiles - 1 - y : y - third) * Q;
+  const uint32_t stride = 3u * a.dim * sizeof(T);  // bytes
+  const char* base = a.qkv + static_cast<int64_t>(h) * D * sizeof(T);
   const int last = a.rows - 1;
   const int keys = min(q0 + Q, a.rows);  // this tile's last query sees [0, keys)
 
-  u32x4 q[QT][NCH];
+  u32x4 q[NCH];
 #pragma unroll
-  for (int t = 0; t < QT; ++t)
+  for (int c = 0; c < NCH; ++c)
+    q[c] = *reinterpret_cast<const u32x4*>(base + static_cast<int64_t>(min(q0 + i, last)) * stride + c * 64 + g * 16);
+  f32x4 o[NO];
+  float m = -INFINITY, l = 0.f;
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
-      q[t][c] = *reinterpret_cast<const u32x4*>(
-          reinterpret_cast<const char*>(base + min(q0 + t * 16 + i, last) * stride) + c * 64 + g * 16);
-  f32x4 o[QT][NO];
-  float m[QT], l[QT];
-#pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    m[t] = -INFINITY;
-    l[t] = 0.f;
-#pragma unroll
-    for (int n = 0; n < NO; ++n) o[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int n = 0; n < NO; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // A block's rows as offsets from its first one (a wave-uniform address): the
+  // offsets change only where rows past the last token repeat it (masked).
+  uint32_t k_off[2], v_off[2][4];
+  auto offsets = [&](int top) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      k_off[t] = min(t * 16 + i, top) * stride + a.dim * sizeof(T) + g * 16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v_off[t][r] = min(t * 16 + g * 4 + r, top) * stride + 2u * a.dim * sizeof(T);
+    }
+  };
+  offsets(31);
   u32x4 kf[2][NCH];
-  auto load_keys = [&](int k0) {  // rows past the last token read it (masked below)
+  auto load_keys = [&](int k0) {
+    const char* rows = base + static_cast<int64_t>(k0) * stride;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int c = 0; c < NCH; ++c)
-        kf[t][c] = *reinterpret_cast<const u32x4*>(
-            reinterpret_cast<const char*>(base + a.dim + min(k0 + t * 16 + i, last) * stride) + c * 64 + g * 16);
+      for (int c = 0; c < NCH; ++c) kf[t][c] = *reinterpret_cast<const u32x4*>(rows + k_off[t] + c * 64);
   };
-  if (wave * 32 < keys) load_keys(wave * 32);
-  for (int k0 = wave * 32; k0 < keys; k0 += 128) {
+  int k0 = wave * 32;
+  if (k0 < keys) {
+    if (k0 + 31 > last) offsets(last - k0);
+    load_keys(k0);
+  }
+  for (; k0 < keys; k0 += 128) {
     ValueGroup<T, 4> v4[G4 > 0 ? G4 : 1];
     ValueGroup<T, 2> v2[G2 > 0 ? G2 : 1];
+    const char* rows = base + static_cast<int64_t>(k0) * stride;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const T* v = base + 2 * a.dim + min(k0 + t * 16 + g * 4 + r, last) * stride;
+        const T* v = reinterpret_cast<const T*>(rows + v_off[t][r]);
 #pragma unroll
         for (int n = 0; n < G4; ++n) v4[n].load(t, r, v + n * 64 + i * 4);
 #pragma unroll
         for (int n = 0; n < G2; ++n) v2[n].load(t, r, v + G4 * 64 + n * 32 + i * 2);
       }
-    f32x4 s[QT][2];
+    f32x4 s[2];
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
+    for (int u = 0; u < 2; ++u) {
+      s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        s[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) s[t][u] = mie::gemm::mfma_fragment<T>(kf[u][c], q[t][c], s[t][u]);
-      }
-    if (k0 + 128 < keys) load_keys(k0 + 128);
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const int query = q0 + t * 16 + i;
-      float p[2][4];
-      float top = m[t];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          p[u][r] = k0 + u * 16 + g * 4 + r <= query ? s[t][u][r] * a.scale : -INFINITY;
-          top = fmaxf(top, p[u][r]);
-        }
-      top = across_groups<true>(top);
-      const float ref = top == -INFINITY ? 0.f : top;
-      const float alpha = mie::fast_exp2(m[t] - ref);
-      m[t] = top;
-      float sum = 0.f;
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          p[u][r] = mie::fast_exp2(p[u][r] - ref);
-          sum += p[u][r];
-        }
-      l[t] = l[t] * alpha + sum;
-#pragma unroll
-      for (int n = 0; n < NO; ++n) o[t][n] *= alpha;
-#pragma unroll
-      for (int n = 0; n < G4; ++n) v4[n].multiply(p, &o[t][n * 4]);
-#pragma unroll
-      for (int n = 0; n < G2; ++n) v2[n].multiply(p, &o[t][G4 * 4 + n * 2]);
+      for (int c = 0; c < NCH; ++c) s[u] = mie::gemm::mfma_fragment<T>(kf[u][c], q[c], s[u]);
     }
+    if (k0 + 128 < keys) {
+      if (k0 + 128 + 31 > last) offsets(last - k0 - 128);
+      load_keys(k0 + 128);
+    }
+    float p[2][4];
+    float top = m;
+    const bool diagonal = k0 + 31 > q0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[u][r] = s[u][r] * a.scale;
+        if (diagonal) p[u][r] = k0 + u * 16 + g * 4 + r <= q0 + i ? p[u][r] : -INFINITY;
+        top = fmaxf(top, p[u][r]);
+      }
+    top = across_groups<true>(top);
+    const float ref = top == -INFINITY ? 0.f : top;
+    if (__any(top > m)) {  // a later maximum: the sums so far shrink
+      const float alpha = mie::fast_exp2(m - ref);
+      l *= alpha;
+#pragma unroll
+      for (int n = 0; n < NO; ++n) o[n] *= alpha;
+    }
+    m = top;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[u][r] = mie::fast_exp2(p[u][r] - ref);
+        l += p[u][r];
+      }
+#pragma unroll
+    for (int n = 0; n < G4; ++n) v4[n].multiply(p, &o[n * 4]);
+#pragma unroll
+    for (int n = 0; n < G2; ++n) v2[n].multiply(p, &o[G4 * 4 + n * 2]);
   }
 
   // Merge the waves: the largest maximum, then the rescaled sums and outputs.
-#pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    l[t] = across_groups<false>(l[t]);
-    if (g == 0) {
-      s_max[wave][t * 16 + i] = m[t];
-      s_sum[wave][t * 16 + i] = l[t];
-    }
+  l = across_groups<false>(l);
+  if (g == 0) {
+    s_max[wave][i] = m;
+    s_sum[wave][i] = l;
   }
   __syncthreads();
+  const float top = fmaxf(fmaxf(s_max[0][i], s_max[1][i]), fmaxf(s_max[2][i], s_max[3][i]));
+  const float f = m == -INFINITY ? 0.f : mie::fast_exp2(m - top);
+  // Lane (i, g) holds, of a 64-dim group, dims 16 g + 4 r + j in o[j][r]; of a
+  // 32-dim group, dims 8 g + 2 r + j.
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    const int at = t * 16 + i;
-    const float top = fmaxf(fmaxf(s_max[0][at], s_max[1][at]), fmaxf(s_max[2][at], s_max[3][at]));
-    const float f = m[t] == -INFINITY ? 0.f : mie::fast_exp2(m[t] - top);
-    // Lane (i, g) holds, of a 64-dim group, dims 16 g + 4 r + j in o[j][r]; of a
-    // 32-dim group, dims 8 g + 2 r + j.
+  for (int n = 0; n < G4; ++n)
 #pragma unroll
-    for (int n = 0; n < G4; ++n)
+    for (int r = 0; r < 4; ++r) {
+      const f32x4* u = &o[n * 4];
+      *reinterpret_cast<f32x4*>(&s_out[wave][i][n * 64 + g * 16 + r * 4]) = f32x4{u[0][r], u[1][r], u[2][r], u[3][r]} * f;
+    }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const f32x4* u = &o[t][n * 4];
-        *reinterpret_cast<f32x4*>(&s_out[wave][at][n * 64 + g * 16 + r * 4]) =
-            f32x4{u[0][r], u[1][r], u[2][r], u[3][r]} * f;
-      }
+  for (int n = 0; n < G2; ++n)
 #pragma unroll
-    for (int n = 0; n < G2; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const f32x4* u = &o[t][G4 * 4 + n * 2];
-        float* dst = &s_out[wave][at][G4 * 64 + n * 32 + g * 8 + r * 2];
-        dst[0] = u[0][r] * f;
-        dst[1] = u[1][r] * f;
-      }
-  }
+    for (int r = 0; r < 4; ++r) {
+      const f32x4* u = &o[G4 * 4 + n * 2];
+      float* dst = &s_out[wave][i][G4 * 64 + n * 32 + g * 8 + r * 2];
+      dst[0] = u[0][r] * f;
+      dst[1] = u[1][r] * f;
+    }
   __syncthreads();
   for (int e = threadIdx.x; e < Q * (D / 4); e += 256) {
     const int row = e / (D / 4), c = e % (D / 4) * 4;
@@ -374,28 +415,46 @@ void launch_tile(const LinearArgs& a, hipStream_t st) {
       <<<dim3((a.n + Tile::BN - 1) / Tile::BN, (a.rows + Tile::BM - 1) / Tile::BM), 256, 0, st>>>(a);
 }
 
+template <typename T, typename Tile, int MT>
+void launch_direct(const LinearArgs& a, hipStream_t st) {
+  prompt_linear_direct_kernel<T, Tile, MT>
+      <<<dim3((a.n + Tile::BN - 1) / Tile::BN, (a.rows + 16 * MT - 1) / (16 * MT)), 256, 0, st>>>(a);
+}
+
+// Fewer than 128 tiles of 32 x 32 (few rows): direct tiles, the larger that
+// still makes 128 workgroups.  Otherwise the staged tile whose last round of
+// workgroups over the 256 CUs wastes least - rounds x tile area; on a tie the
+// smallest tile while it makes at most 512 workgroups (more of them hide each
+// other's waits), the largest beyond (less operand traffic).  Measured on
+// MI355X, float32, K 768, 64x48 / 32x64 / 32x32 / 64x64: 1000 x 2304 44.1 /
+// 45.8 / - / 50.3 us, 1000 x 768 18.7 / 21.6 / - / 22.0, 512 x 768 17.5 / 14.4
+// / 12.8 / -, 200 x 2304 - / 16.5 / 15.0 / -; 62 x 2304 9.7 us with 32x32 and
+// 10.6 with direct tiles, 62 x 768 8.8 and 5.6.
 template <typename T>
 int32_t launch_linear(const LinearArgs& a, hipStream_t st) {
   auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((a.rows + bm - 1) / bm) * ((a.n + bn - 1) / bn); };
-  if (tiles(64, 64) >= 192) {
-    launch_tile<T, Tile<T, 64, 64, 128, 2, 2>>(a, st);
-  } else if (tiles(32, 32) >= 192) {
+  auto cost = [&](int bm, int bn) { return (tiles(bm, bn) + 255) / 256 * bm * bn; };
+  const int64_t big = cost(64, 48), mid = cost(32, 64), small = cost(32, 32);
+  const bool favour_small = tiles(32, 32) <= 512;
+  if (tiles(32, 32) < 128) {
+    if (tiles(32, 16) >= 128) {
+      launch_direct<T, Direct<T, 1, 6>, 2>(a, st);
+    } else {
+      launch_direct<T, Direct<T, 1, 6>, 1>(a, st);
+    }
+  } else if (favour_small ? small <= mid && small <= big : small < mid && small < big) {
     launch_tile<T, Tile<T, 32, 32, 256, 2, 2>>(a, st);
-  } else if (tiles(16, 32) >= 192) {
-    launch_tile<T, Tile<T, 16, 32, 256, 1, 1, 4>>(a, st);
+  } else if (mid < big) {
+    launch_tile<T, Tile<T, 32, 64, 128, 2, 2>>(a, st);
   } else {
-    launch_tile<T, Tile<T, 16, 16, 256, 1, 1, 4>>(a, st);
+    launch_tile<T, Tile<T, 64, 48, 256, 4, 1>>(a, st);
   }
   return mie::check_launch("prompt_linear_kernel");
 }
 
 template <typename T, int D>
 void launch_heads(const AttnArgs& a, int32_t heads, hipStream_t st) {
-  if (D <= 64 && a.rows > 256) {
-    prompt_attention_kernel<T, D, D <= 64 ? 2 : 1><<<dim3(heads, (a.rows + 31) / 32), 256, 0, st>>>(a);
-  } else {
-    prompt_attention_kernel<T, D, 1><<<dim3(heads, (a.rows + 15) / 16), 256, 0, st>>>(a);
-  }
+  prompt_attention_kernel<T, D><<<dim3(heads, (a.rows + 15) / 16), 256, 0, st>>>(a);
 }
 
 template <typename T>
@@ -475,10 +534,13 @@ extern "C" int32_t mie_attn_prefill(const void* x, int32_t tokens, const void* l
   if (ln_weight) {
     const NormArgs n{in, static_cast<const char*>(ln_weight), static_cast<const char*>(ln_bias), normed, tokens, dim,
                      ln_eps};
-    if (f32) {
-      prompt_norm_kernel<float><<<(tokens + 3) / 4, 256, 0, st>>>(n);
+    const int groups = (tokens + 3) / 4;
+    if (dim <= 1024) {
+      f32 ? prompt_norm_kernel<float, 4><<<groups, 256, 0, st>>>(n)
+          : prompt_norm_kernel<uint16_t, 4><<<groups, 256, 0, st>>>(n);
     } else {
-      prompt_norm_kernel<uint16_t><<<(tokens + 3) / 4, 256, 0, st>>>(n);
+      f32 ? prompt_norm_kernel<float, 0><<<groups, 256, 0, st>>>(n)
+          : prompt_norm_kernel<uint16_t, 0><<<groups, 256, 0, st>>>(n);
     }
     rc = mie::check_launch("prompt_norm_kernel");
     if (rc != MIE_OK) return rc;
