@@ -20,6 +20,21 @@ template <> struct Raw<8> { using T = uint2; };
 template <> struct Raw<4> { using T = uint32_t; };
 template <> struct Raw<2> { using T = uint16_t; };
 
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+
+// Streaming load of data read exactly once (global_load ... nt).
+template <typename T>
+__device__ __forceinline__ T load_once(const char* p) {
+  if constexpr (sizeof(T) == 16) {
+    return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+  } else if constexpr (sizeof(T) == 8) {
+    return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p)));
+  } else {
+    return __builtin_nontemporal_load(reinterpret_cast<const T*>(p));
+  }
+}
+
 struct AppendArgs {
   char* k_pool;
   char* v_pool;
@@ -89,27 +104,58 @@ struct GatherArgs {
   mie::FastDiv bs;
 };
 
-// grid = (ceil(length * vecs_per_row / kCopyThreads), num_heads, 2 [K, V]).
-template <int VB>
+// grid = (ceil(length * vecs_per_row / (PER * kCopyThreads)), num_heads, 2 [K, V]).
+// A thread moves PER vectors, kCopyThreads apart, all their table reads and
+// then all their loads in flight together: with one vector a wave spends its
+// life in one dependent chain (table, load, store).  The pool is read once
+// (non-temporal); the output is for the attention that follows and is stored
+// through the caches.  8192 tokens x 12 heads x 64 bf16 (50 MB moved) on
+// MI355X: 12.95 -> 11.66 us.
+template <int VB, int PER>
 __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
   using T = typename Raw<VB>::T;
-  const uint32_t i = blockIdx.x * kCopyThreads + threadIdx.x;
-  const uint32_t t = a.vecs_per_row.div(i);
-  if (t >= static_cast<uint32_t>(a.length)) return;
-  const uint32_t vec = i - t * a.vecs_per_row.d;
   const int h = blockIdx.y;
   const bool is_v = blockIdx.z != 0;
+  const char* pool = (is_v ? a.v_pool : a.k_pool) + h * a.pool_shead;
+  char* out = (is_v ? a.v_out : a.k_out) + h * a.out_sh;
+  const uint32_t i0 = blockIdx.x * (PER * kCopyThreads) + threadIdx.x;
+  int32_t phys[PER];
+  uint32_t tok[PER];
+  T v[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    tok[p] = a.vecs_per_row.div(i0 + p * kCopyThreads);
+    const uint32_t t = min(tok[p], static_cast<uint32_t>(a.length) - 1u);  // in bounds; not stored
+    phys[p] = a.block_table[a.bs.div(t)];
+  }
+  // Loads are unconditional, so they go out together: a vector past the end
+  // reads the last token's row, an id outside the pool block 0; neither is
+  // stored.
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const uint32_t vec = i0 + p * kCopyThreads - tok[p] * a.vecs_per_row.d;
+    const uint32_t t = min(tok[p], static_cast<uint32_t>(a.length) - 1u);
+    const uint32_t slot = t - a.bs.div(t) * a.bs.d;
+    const bool ok = phys[p] >= 0 && phys[p] < a.num_blocks;
+    v[p] = load_once<T>(pool + (ok ? phys[p] : 0) * a.pool_sblk + static_cast<int64_t>(slot) * a.row_bytes +
+                        static_cast<int64_t>(vec) * VB);
+    if (!ok) tok[p] = 0xffffffffu;
+  }
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    if (tok[p] >= static_cast<uint32_t>(a.length)) continue;
+    const uint32_t vec = i0 + p * kCopyThreads - tok[p] * a.vecs_per_row.d;
+    *reinterpret_cast<T*>(out + static_cast<int64_t>(tok[p]) * a.out_st + static_cast<int64_t>(vec) * VB) = v[p];
+  }
+}
 
-  const uint32_t blk = a.bs.div(t);
-  const uint32_t slot = t - blk * a.bs.d;
-  const int32_t phys = a.block_table[blk];
-  if (phys < 0 || phys >= a.num_blocks) return;
-
-  const char* src = (is_v ? a.v_pool : a.k_pool) + phys * a.pool_sblk + h * a.pool_shead +
-                    static_cast<int64_t>(slot) * a.row_bytes + static_cast<int64_t>(vec) * VB;
-  char* dst = (is_v ? a.v_out : a.k_out) + h * a.out_sh + static_cast<int64_t>(t) * a.out_st +
-              static_cast<int64_t>(vec) * VB;
-  *reinterpret_cast<T*>(dst) = *reinterpret_cast<const T*>(src);
+template <int VB>
+void launch_gather(const GatherArgs& a, dim3 grid, bool four, hipStream_t st) {
+  if (four) {
+    kv_gather_kernel<VB, 4><<<grid, kCopyThreads, 0, st>>>(a);
+  } else {
+    kv_gather_kernel<VB, 1><<<grid, kCopyThreads, 0, st>>>(a);
+  }
 }
 
 // Widest vector that divides the row and every byte stride the kernel adds to
@@ -253,14 +299,17 @@ extern "C" int32_t mie_kv_gather(const void* k_pool, const void* v_pool, int64_t
   if (total >= (int64_t{1} << 31))
     return mie::fail(MIE_ERR_INVALID, "mie_kv_gather: length * row vectors exceeds 2^31");
 
-  const int threads = kCopyThreads;
-  dim3 grid(static_cast<uint32_t>((total + threads - 1) / threads), num_heads, 2);
+  // Four vectors per thread where that still makes 1024 workgroups (four per
+  // CU); the last workgroup's indices stay in FastDiv's range.
+  const int64_t wide = (total + 4 * kCopyThreads - 1) / (4 * kCopyThreads);
+  const bool four = wide * num_heads * 2 >= 1024 && total < (int64_t{1} << 31) - 4 * kCopyThreads;
+  const dim3 grid(static_cast<uint32_t>(four ? wide : (total + kCopyThreads - 1) / kCopyThreads), num_heads, 2);
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (vb) {
-    case 16: kv_gather_kernel<16><<<grid, threads, 0, st>>>(a); break;
-    case 8: kv_gather_kernel<8><<<grid, threads, 0, st>>>(a); break;
-    case 4: kv_gather_kernel<4><<<grid, threads, 0, st>>>(a); break;
-    default: kv_gather_kernel<2><<<grid, threads, 0, st>>>(a); break;
+    case 16: launch_gather<16>(a, grid, four, st); break;
+    case 8: launch_gather<8>(a, grid, four, st); break;
+    case 4: launch_gather<4>(a, grid, four, st); break;
+    default: launch_gather<2>(a, grid, four, st); break;
   }
   return mie::check_launch("mie_kv_gather");
 }

@@ -1,0 +1,77 @@
+"""The append fused into the partition form of the paged decode: against the
+append launch followed by the plain decode, on the sequence lengths where a
+partition ends, begins with the new token alone, or is the only one.
+
+The new token's score and value come from registers instead of the pool, with
+the same arithmetic; it joins its wave's softmax state last instead of in its
+tile, so outputs may differ by float32 rounding of the merge: 2^-22 of the
+largest value times a few operations, below 4e-6 for N(0, 1) values.  Pools
+must be equal bit for bit.
+"""
+
+import pytest
+import torch
+
+from conftest import print_case
+from moe_engine import kv_ops, paged_attention
+from moe_engine.workloads import make_workload, take_last_tokens
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,head_dim,block_size", [(12, 64, 16), (8, 96, 16), (3, 128, 32), (5, 64, 12), (2, 4, 8)])
+def test_fused_append_equals_append_then_decode(heads, head_dim, block_size, dtype):
+    # 256-token partitions whatever the tile (head_dim 4 has the largest).
+    lens = [1, 2, 31, 32, 33, 255, 256, 257, 258, 512, 513, 1000, 0]
+    part = 1024 if head_dim == 4 else 256
+    w = make_workload(lens, num_heads=heads, head_dim=head_dim, block_size=block_size, dtype=dtype, seed=3)
+    k_new, v_new = take_last_tokens(w)
+    pools = [t.clone() for t in (w.k_pool, w.v_pool)]
+    print_case("append in partitions", heads, head_dim, block_size, dtype)
+    got = paged_attention.decode_batched(
+        w.q, w.k_pool, w.v_pool, 0, w.block_tables, w.context_lens, w.max_len, partition_tokens=part,
+        context_lens_host=w.lens, k_new=k_new, v_new=v_new, out_dtype=torch.float32)
+    kv_ops.append(*pools, 0, k_new[:, :, None], v_new[:, :, None], w.block_tables,
+                  positions=(w.context_lens - 1).contiguous())
+    want = paged_attention.decode_batched(
+        w.q, *pools, 0, w.block_tables, w.context_lens, w.max_len, partition_tokens=part, context_lens_host=w.lens,
+        out_dtype=torch.float32)
+    assert torch.equal(w.k_pool, pools[0]) and torch.equal(w.v_pool, pools[1])
+    assert (got - want).abs().max().item() <= 4e-6
+    # A launch bound instead of the exact list, and a bad block id for one sequence.
+    again = paged_attention.decode_batched(
+        w.q, w.k_pool, w.v_pool, 0, w.block_tables, w.context_lens, w.max_len, partition_tokens=part, k_new=k_new,
+        v_new=v_new, out_dtype=torch.float32)
+    assert torch.equal(again, got)
+    tables = w.block_tables.clone()
+    last = (w.lens[8] - 1) // block_size
+    tables[8, last] = -1
+    before = w.k_pool.clone()
+    bad = paged_attention.decode_batched(
+        w.q, w.k_pool, w.v_pool, 0, tables, w.context_lens, w.max_len, partition_tokens=part, context_lens_host=w.lens,
+        k_new=k_new, v_new=v_new, out_dtype=torch.float32)
+    assert bad[8].isnan().all() and torch.equal(w.k_pool, before)
+    rest = [b for b in range(len(lens)) if b != 8]
+    assert torch.equal(bad[rest], got[rest])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16, torch.float64])
+@pytest.mark.parametrize("heads,head_dim,block_size,length", [(12, 64, 16, 8192), (12, 64, 16, 4097), (40, 24, 7, 3001),
+                                                              (12, 64, 16, 1)])
+def test_gather_with_several_vectors_per_thread(heads, head_dim, block_size, length, dtype):
+    """Lengths on both sides of the switch to four vectors per thread, with a
+    tail, against the indexed rebuild; rows of a bad block id stay unwritten."""
+    blocks = -(-length // block_size) + 3
+    pools = [torch.randn(1, blocks, heads, block_size, head_dim, device="cuda").to(dtype) for _ in range(2)]
+    table = torch.randperm(blocks)[: -(-length // block_size)].to(torch.int32).to("cuda")
+    print_case("gather", heads, head_dim, block_size, length, dtype)
+    want = [p[0, table.long()].transpose(0, 1).reshape(heads, -1, head_dim)[:, :length] for p in pools]
+    got = kv_ops.gather(*pools, 0, table, length)
+    assert all(torch.equal(g[0], w) for g, w in zip(got, want))
+    table[-1] = blocks
+    out = [torch.full((1, heads, length, head_dim), 7, dtype=dtype, device="cuda") for _ in range(2)]
+    kv_ops.gather(*pools, 0, table, length, *out)
+    start = (len(table) - 1) * block_size
+    for o, w in zip(out, want):
+        assert torch.equal(o[0, :, :start], w[:, :start]) and (o[0, :, start:] == 7).all()
