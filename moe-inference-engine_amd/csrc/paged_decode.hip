@@ -76,10 +76,18 @@ constexpr int kMinWaves = 4;
 constexpr int kFlatMaxBatch = 512;
 // Workgroup form: one workgroup of kSplitWaves waves per (sequence, head).
 // Each wave reads its slice as a serial chain of tiles (~2 us per tile when
-// latency-bound), so the automatic plan takes this form for at most
-// kWgMaxRows (sequence, head) rows when every slice is short (max_ctx <=
-// kWgShortCtx: at most 64 tokens per wave) or when there are enough rows to
-// fill the GPU with workgroups (rows >= kWgMinRows, max_ctx <= kWgMaxCtx).
+// latency-bound) and a row's K and V come in at one CU's rate, so the automatic
+// plan takes this form for at most kWgMaxRows (sequence, head) rows when a row
+// is short (max_ctx <= kWgShortCtx: at most 64 tokens per wave, and at most
+// kWgRowBytes of K and V) or when there are enough rows to fill the GPU with
+// workgroups (rows >= kWgMinRows, max_ctx <= kWgMaxCtx).  The line in bytes,
+// workgroup form against 32-token partitions and their merge (us per call,
+// graph replays): 256 KB rows 5.9 / 7.2 (1 x 512, f32 12 x 64), 7.9 / 6.9 (1 x
+// 1000, bf16 12 x 64), 8.8 / 8.2 (5 x 1000, bf16), 7.4 / 8.7 (1 x 256, f32 6 x
+// 128); 375 KB rows 11.0 / 7.8 (1 x 1000, bf16 8 x 96), 10.2 / 9.4 (5 x 512,
+// f32 8 x 96); 500 KB and more 11.6 / 7.6 (1 x 1000, f32 12 x 64), 17.1 / 11.0
+// (5 x 1000, f32 8 x 96), 20.4 / 11.5 (5 x 1000, f32 6 x 128).  From kWgMinRows
+// rows on the rows fill the CUs: 20.5 / 24.5 (21 x 1000, f32 12 x 64).
 // Measured on MI355X (per call, graph replays), workgroup form vs the
 // partition plan: 1 x 96 tokens 3.9 vs 6.8 us, 1 x 512 5.4 vs 7.0, 21 x 1000
 // 13.6 vs 16.3, 16 x 4096 33.5 vs 35.3, 64 x 2048 68.7 vs 73.3, 64 x 4096
@@ -96,6 +104,7 @@ constexpr int kSplitWaves = 16;
 constexpr int kWgTileWords = 8;
 constexpr int kWgOrderMax = 1024;  // batches the workgroup form can dispatch longest first
 constexpr int kWgShortCtx = 1024;
+constexpr int64_t kWgRowBytes = 320 << 10;
 constexpr int kWgMinRows = 128;
 constexpr int kWgMaxRows = 1024;
 constexpr int kWgMaxCtx = 8192;
@@ -187,8 +196,8 @@ struct DecodeArgs {
   float* ws_acc;  // [B, H, max_parts, D]
   int32_t max_parts;
   int32_t part_shift;  // partition = 1 << part_shift tokens
-  // Fused append (workgroup form): the new token's K/V rows [B, H, D]; NULL
-  // for a plain decode.  The token is the sequence's last (position ctx - 1).
+  // Fused append (workgroup and flat forms): the new token's K/V rows [B, H,
+  // D]; NULL for a plain decode.  The token is the sequence's last (position ctx - 1).
   const char* k_new;
   const char* v_new;
   int64_t new_sb, new_sh;  // elements
@@ -429,18 +438,105 @@ __device__ __forceinline__ void attend_range(const DecodeArgs& a, int b, int h, 
   if constexpr (YIELD) __builtin_amdgcn_s_setprio(0);
 }
 
+// Element i of packed words.
+template <int DT, int NW>
+__device__ __forceinline__ float element(const Words<NW>& x, int i) {
+  if constexpr (DT == MIE_DTYPE_BF16) return i % 2 ? mie::bf16_hi(x.w[i / 2]) : mie::bf16_lo(x.w[i / 2]);
+  else return __uint_as_float(x.w[i]);
+}
+
+// A fused append's new token of (sequence b, head h), at position ctx - 1: the
+// lanes of each token group hold its K, V slices; group 0 stores them into the
+// pool (bounds-checked like the append kernel).  `dot` is the token's score,
+// computed as the pool path computes one (consume()), in every lane, and vw
+// the V slice as stored (see element()).  Returns whether the block id was
+// valid.
+template <int DT, int D, typename G>
+__device__ __forceinline__ bool append_token(const DecodeArgs& a, int b, int h, int ctx, int lane, Words<G::NW>& vw,
+                                             float& dot) {
+  constexpr int VEC = G::VEC, NW = G::NW, LPT = G::LPT, ELT = G::ELT;
+  const int g = lane / LPT;
+  const int jl = lane % LPT;
+  const bool jv = jl < G::NV;
+  const int64_t row = (b * a.new_sb + h * a.new_sh + jl * VEC) * ELT;
+  Words<NW> kw, qw;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) kw.w[w] = vw.w[w] = qw.w[w] = 0u;
+  if (jv) {
+    kw = load_words<NW>(a.k_new + row);
+    vw = load_words<NW>(a.v_new + row);
+    qw = load_words<NW>(a.q + (b * a.q_sb + h * a.q_sh + jl * VEC) * ELT);
+  }
+  const uint32_t p = static_cast<uint32_t>(ctx - 1);
+  const uint32_t lb = a.bs.div(p);
+  const int32_t phys = lb < a.bt_cap ? a.bt[b * a.bt_stride + lb] : -1;
+  const bool ok = phys >= 0 && phys < a.num_blocks;
+  if (ok && g == 0 && jv) {
+    const int64_t off = (phys * a.kv_sblk + h * a.kv_sh + static_cast<int64_t>(p - lb * a.bs.d) * D + jl * VEC) * ELT;
+    if constexpr (NW == 4) {
+      *reinterpret_cast<u32x4_t*>(const_cast<char*>(a.k) + off) = u32x4_t{kw.w[0], kw.w[1], kw.w[2], kw.w[3]};
+      *reinterpret_cast<u32x4_t*>(const_cast<char*>(a.v) + off) = u32x4_t{vw.w[0], vw.w[1], vw.w[2], vw.w[3]};
+    } else {
+      *reinterpret_cast<u32x2_t*>(const_cast<char*>(a.k) + off) = u32x2_t{kw.w[0], kw.w[1]};
+      *reinterpret_cast<u32x2_t*>(const_cast<char*>(a.v) + off) = u32x2_t{vw.w[0], vw.w[1]};
+    }
+  }
+  dot = 0.f;
+  if constexpr (DT == MIE_DTYPE_BF16) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+      dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, kw.w[w]), __builtin_bit_cast(bf16x2_t, qw.w[w]),
+                                            dot, false);
+    dot = mie::group_sum<LPT>(dot) * a.qk_scale;
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) dot = fmaf(__uint_as_float(kw.w[i]), __uint_as_float(qw.w[i]) * a.qk_scale, dot);
+    dot = mie::group_sum<LPT>(dot);
+  }
+  return ok;
+}
+
 // One work item: sequence b (ctx tokens, ctx > 0), head h, partition `part`,
-// computed by one full wavefront.
-template <int DT, int D, bool FAST>
+// computed by one full wavefront.  APPEND: the sequence's last token comes
+// from the caller's new rows, not the pool; the last partition's wave stores
+// them and adds the token's state to its own.
+template <int DT, int D, bool FAST, bool APPEND = false>
 __device__ __forceinline__ void decode_item(const DecodeArgs& a, int b, int h, int part, int ctx, int lane) {
   using G = Geometry<DT, D>;
   constexpr int VEC = G::VEC;
   const int nparts = (ctx + (1 << a.part_shift) - 1) >> a.part_shift;
   const int t_begin = part << a.part_shift;
-  const int t_end = min(ctx, t_begin + (1 << a.part_shift));
+  const int t_end = min(APPEND ? ctx - 1 : ctx, t_begin + (1 << a.part_shift));
   float m, l, acc[VEC];
   bool bad;
-  attend_range<DT, D, FAST>(a, b, h, t_begin, t_end, lane, m, l, acc, bad);
+  if constexpr (APPEND) {
+    const bool last = part == nparts - 1;
+    Words<G::NW> v_new;
+    float dot = 0.f;
+    bool stored = true;
+    if (last) stored = append_token<DT, D, G>(a, b, h, ctx, lane, v_new, dot);
+    if (t_begin < t_end) {
+      attend_range<DT, D, FAST>(a, b, h, t_begin, t_end, lane, m, l, acc, bad);
+    } else {  // the partition holds the new token alone
+      m = -INFINITY;
+      l = 0.f;
+      bad = false;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
+    }
+    if (last) {
+      const float mn = fmaxf(m, dot);
+      const float mr = mn == -INFINITY ? 0.f : mn;
+      const float ca = mie::fast_exp2(m - mr), cb = mie::fast_exp2(dot - mr);
+      l = l * ca + cb;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) acc[i] = acc[i] * ca + element<DT>(v_new, i) * cb;
+      m = mn;
+      bad = bad || !stored;
+    }
+  } else {
+    attend_range<DT, D, FAST>(a, b, h, t_begin, t_end, lane, m, l, acc, bad);
+  }
 
   const int g = lane / G::LPT;
   const int jl = lane % G::LPT;
@@ -504,7 +600,7 @@ void paged_decode_grid_kernel(DecodeArgs a) {
 // 64 sequences per step, so no workgroup exists for a partition past a
 // sequence's end.  When the launch is an upper bound rather than the exact
 // count, the surplus workgroups find no item and exit.
-template <int DT, int D, bool FAST>
+template <int DT, int D, bool FAST, bool APPEND>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kMinWaves, 8)))
 void paged_decode_flat_kernel(DecodeArgs a, int batch, int head_groups) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -548,7 +644,7 @@ void paged_decode_flat_kernel(DecodeArgs a, int batch, int head_groups) {
     zero_item<DT, D>(a, b, h, lane);
     return;
   }
-  decode_item<DT, D, FAST>(a, b, h, part, seq_ctx_len, lane);
+  decode_item<DT, D, FAST, APPEND>(a, b, h, part, seq_ctx_len, lane);
 }
 
 // Workgroup form: grid = (H, batch), one workgroup of kSplitWaves waves per
@@ -573,7 +669,7 @@ template <int DT, int D, bool FAST>
 __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(kMinWaves, 8)))
 void paged_decode_wg_kernel(DecodeArgs a, WgOrder order) {
   using G = Geometry<DT, D, kWgTileWords>;
-  constexpr int VEC = G::VEC, NW = G::NW, LPT = G::LPT, ELT = G::ELT;
+  constexpr int VEC = G::VEC, LPT = G::LPT;
   constexpr int kStates = kSplitWaves + 1;  // the waves' slices, then a fused append's new token
   __shared__ float s_m[kStates], s_l[kStates];
   __shared__ float s_acc[kStates][D];
@@ -624,43 +720,9 @@ void paged_decode_wg_kernel(DecodeArgs a, WgOrder order) {
     for (int i = 0; i < VEC; ++i) s_acc[wave][jl * VEC + i] = acc[i];
   }
   if (append && wave == kSplitWaves - 1) {
-    const int64_t row = (b * a.new_sb + h * a.new_sh + jl * VEC) * ELT;
-    Words<NW> kw, vw, qw;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) kw.w[w] = vw.w[w] = qw.w[w] = 0u;
-    if (jv) {
-      kw = load_words<NW>(a.k_new + row);
-      vw = load_words<NW>(a.v_new + row);
-      qw = load_words<NW>(a.q + (b * a.q_sb + h * a.q_sh + jl * VEC) * ELT);
-    }
-    // Store the rows at position ctx - 1 (bounds-checked like the append kernel).
-    const uint32_t p = static_cast<uint32_t>(ctx - 1);
-    const uint32_t lb = a.bs.div(p);
-    const int32_t phys = lb < a.bt_cap ? a.bt[b * a.bt_stride + lb] : -1;
-    const bool ok = phys >= 0 && phys < a.num_blocks;
-    if (ok && g == 0 && jv) {
-      const int64_t off = (phys * a.kv_sblk + h * a.kv_sh + static_cast<int64_t>(p - lb * a.bs.d) * D + jl * VEC) * ELT;
-      if constexpr (NW == 4) {
-        *reinterpret_cast<u32x4_t*>(const_cast<char*>(a.k) + off) = u32x4_t{kw.w[0], kw.w[1], kw.w[2], kw.w[3]};
-        *reinterpret_cast<u32x4_t*>(const_cast<char*>(a.v) + off) = u32x4_t{vw.w[0], vw.w[1], vw.w[2], vw.w[3]};
-      } else {
-        *reinterpret_cast<u32x2_t*>(const_cast<char*>(a.k) + off) = u32x2_t{kw.w[0], kw.w[1]};
-        *reinterpret_cast<u32x2_t*>(const_cast<char*>(a.v) + off) = u32x2_t{vw.w[0], vw.w[1]};
-      }
-    }
-    // The token's score, computed as the pool path computes one (consume()).
-    float dot = 0.f;
-    if constexpr (DT == MIE_DTYPE_BF16) {
-#pragma unroll
-      for (int w = 0; w < NW; ++w)
-        dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, kw.w[w]), __builtin_bit_cast(bf16x2_t, qw.w[w]),
-                                              dot, false);
-      dot = mie::group_sum<LPT>(dot) * a.qk_scale;
-    } else {
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) dot = fmaf(__uint_as_float(kw.w[i]), __uint_as_float(qw.w[i]) * a.qk_scale, dot);
-      dot = mie::group_sum<LPT>(dot);
-    }
+    Words<G::NW> v;
+    float dot;
+    const bool ok = append_token<DT, D, G>(a, b, h, ctx, lane, v, dot);
     if (lane == 0) {
       s_m[kSplitWaves] = dot;
       s_l[kSplitWaves] = 1.f;
@@ -668,14 +730,7 @@ void paged_decode_wg_kernel(DecodeArgs a, WgOrder order) {
     }
     if (g == 0 && jv) {
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        if constexpr (DT == MIE_DTYPE_BF16) {
-          s_acc[kSplitWaves][jl * VEC + 2 * w] = mie::bf16_lo(vw.w[w]);
-          s_acc[kSplitWaves][jl * VEC + 2 * w + 1] = mie::bf16_hi(vw.w[w]);
-        } else {
-          s_acc[kSplitWaves][jl * VEC + w] = __uint_as_float(vw.w[w]);
-        }
-      }
+      for (int i = 0; i < VEC; ++i) s_acc[kSplitWaves][jl * VEC + i] = element<DT>(v, i);
     }
   }
   __syncthreads();
@@ -866,9 +921,11 @@ int32_t plan(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_s
   const bool fast_blocks = is_pow2(block_size) && block_size % ks.tpl == 0;
   const int64_t fast_cap = static_cast<int64_t>(kWindow) * block_size;  // FAST: <= kWindow blocks
   const int64_t rows = static_cast<int64_t>(batch) * num_heads;
+  const int64_t row_bytes = static_cast<int64_t>(max_ctx) * head_dim * 2 * mie::elt_size(dtype);
   const bool wg = requested == -1 ||
                   (requested == 0 && rows <= kWgMaxRows &&
-                   (max_ctx <= kWgShortCtx || (rows >= kWgMinRows && max_ctx <= kWgMaxCtx)));
+                   ((max_ctx <= kWgShortCtx && row_bytes <= kWgRowBytes) ||
+                    (rows >= kWgMinRows && max_ctx <= kWgMaxCtx)));
   if (requested < -1)
     return mie::fail(MIE_ERR_INVALID, "mie_paged_decode: partition_tokens %d (0 = automatic, -1 = workgroup form)",
                      requested);
@@ -931,10 +988,13 @@ int32_t launch(DecodeArgs& a, int batch, bool fast, bool wg, const WgOrder& orde
   }
   if (flat_items > 0) {
     const dim3 grid(static_cast<uint32_t>(flat_items));
-    if (fast) {
-      paged_decode_flat_kernel<DT, D, true><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups);
+    if (a.k_new) {
+      fast ? paged_decode_flat_kernel<DT, D, true, true><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups)
+           : paged_decode_flat_kernel<DT, D, false, true><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups);
+    } else if (fast) {
+      paged_decode_flat_kernel<DT, D, true, false><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups);
     } else {
-      paged_decode_flat_kernel<DT, D, false><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups);
+      paged_decode_flat_kernel<DT, D, false, false><<<grid, 64 * kWaves, 0, st>>>(a, batch, head_groups);
     }
   } else {
     const dim3 grid(a.max_parts, head_groups, batch);
@@ -1111,14 +1171,15 @@ int32_t decode_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h, const
     if (blocks <= kWindow) a.win_blocks = static_cast<int32_t>(blocks);
   }
   if (k_new) {
-    if (p.wg) {
-      // The decode kernel stores the rows and attends to the new token itself.
+    if (p.wg || flat_items > 0) {
+      // The decode kernel stores the rows and attends to the new token itself
+      // (1 x 2048 bf16: two launches instead of three).
       a.k_new = static_cast<const char*>(k_new);
       a.v_new = static_cast<const char*>(v_new);
       a.new_sb = new_stride_b;
       a.new_sh = new_stride_h;
     } else {
-      // Partition form: append each sequence's last token first (same stream).
+      // Grid form: append each sequence's last token first (same stream).
       const int32_t rc = mie::kv_append_impl(const_cast<void*>(k_pool), const_cast<void*>(v_pool), pool_stride_block,
                                              pool_stride_head, num_blocks, k_new, v_new, new_stride_b, new_stride_h, 0,
                                              block_tables, block_table_stride, ctx_lens, ctx_len, -1, batch, 1,
