@@ -69,7 +69,7 @@ struct PromptArgs {
   char* normed;        // T [tokens, dim]: the norm's output
   int32_t tokens, E, top_k, dim, hidden;
   int32_t words;              // mask words per expert: ceil(tokens / 64)
-  int32_t per_expert;         // 1: blockIdx.y is an expert; 0: the y-th row tile of all experts
+  int32_t per_expert;         // 1: the few-rows form (a workgroup per expert); 0: row tiles of all experts
   int32_t splits, split_len;  // W2: K splits and bytes of a row per split
   unsigned long long* masks;  // [E, words]
   int32_t* counts;            // [E] tokens per expert
@@ -221,21 +221,22 @@ struct Rows {
   int e, m0, count, base;
 };
 
-// blockIdx.y's rows from the experts' token counts (lane e: expert e's).
+// Rows of expert y or of row tile y from the experts' token counts (lane e:
+// expert e's).
 // Uniform over the workgroup; e < 0 when there are none.
-__device__ __forceinline__ Rows find_rows(const PromptArgs& a, int cnt, int bm, int lane) {
+__device__ __forceinline__ Rows find_rows(const PromptArgs& a, int cnt, int bm, int lane, int y) {
   const int tiles = (cnt + bm - 1) / bm;
   const int incl = wave_inclusive(cnt, lane);
   Rows r;
   r.m0 = 0;
   if (a.per_expert) {
-    r.e = blockIdx.y;
+    r.e = y;
   } else {
     const int incl_tiles = wave_inclusive(tiles, lane);
-    const unsigned long long past = __ballot(incl_tiles > static_cast<int>(blockIdx.y));
+    const unsigned long long past = __ballot(incl_tiles > y);
     if (past == 0ull) return Rows{-1, 0, 0, 0};
     r.e = __ffsll(past) - 1;
-    r.m0 = (static_cast<int>(blockIdx.y) - __shfl(incl_tiles - tiles, r.e)) * bm;
+    r.m0 = (y - __shfl(incl_tiles - tiles, r.e)) * bm;
   }
   r.e = __builtin_amdgcn_readfirstlane(r.e);
   r.m0 = __builtin_amdgcn_readfirstlane(r.m0);
@@ -259,18 +260,23 @@ __device__ __forceinline__ int count_tokens(const PromptArgs& a, const unsigned 
   return cnt;
 }
 
-// One wave lists an expert's tokens of ranks m0 .. m0 + BM - 1 (its mask, and
-// the rank of each word's first token); entries past the expert's last token
-// repeat the first listed one (their results are dropped).
+// The workgroup lists an expert's tokens of ranks m0 .. m0 + BM - 1: lane w
+// holds word w of its mask and the rank of that word's first token; wave v
+// takes words v, v + 4, ..., a token per lane.  Entries past the expert's last
+// token name token 0 (their results are dropped).
 template <int BM>
-__device__ __forceinline__ void list_rows(unsigned long long mask, int first, int m0, int count, int lane, int* rows) {
-  unsigned long long word = mask;
-  for (int rank = first - m0; word != 0ull && rank < BM; ++rank, word &= word - 1ull) {
-    const int token = lane * 64 + __ffsll(word) - 1;
-    if (rank >= 0) rows[rank] = token;
-    if (rank == 0)
-      for (int i = min(BM, count - m0); i < BM; ++i) rows[i] = token;
+__device__ __forceinline__ void list_rows(unsigned long long mask, int first, int m0, int count, int words, int lane,
+                                          int wave, int* rows) {
+  const int lo = static_cast<int>(mask), hi = static_cast<int>(mask >> 32);
+  for (int w = wave; w < words; w += 4) {
+    const unsigned int wl = __builtin_amdgcn_readlane(lo, w), wh = __builtin_amdgcn_readlane(hi, w);
+    const int rank = __builtin_amdgcn_readlane(first, w) +
+                     static_cast<int>(__builtin_amdgcn_mbcnt_hi(wh, __builtin_amdgcn_mbcnt_lo(wl, 0u))) - m0;
+    const bool in = (((static_cast<unsigned long long>(wh) << 32) | wl) >> lane) & 1ull;
+    if (in && rank >= 0 && rank < BM) rows[rank] = w * 64 + lane;
   }
+  const int i = wave * 64 + lane;
+  if (i < BM && i >= count - m0) rows[i] = 0;
 }
 
 // Records where token's output of expert e is, for the combining launch.
@@ -300,7 +306,7 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
     cnt = count_tokens(a, word, e0, lane, cnt);
   }
   if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
-  const Rows r = find_rows(a, cnt, Tile::BM, lane);
+  const Rows r = find_rows(a, cnt, Tile::BM, lane, static_cast<int>(blockIdx.y));
   if (r.e < 0) return;
   const unsigned long long mask = lane < a.words ? a.masks[static_cast<int64_t>(r.e) * a.words + lane] : 0ull;
   const int bits = __popcll(mask);
@@ -310,7 +316,7 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   const char* x = a.ln_w ? a.normed : a.x;
   const char* w = a.w1 + static_cast<int64_t>(r.e) * a.hidden * row_bytes;
   const T* bias = reinterpret_cast<const T*>(a.b1) + static_cast<int64_t>(r.e) * a.hidden;
-  if (wave == 0) list_rows<Tile::BM>(mask, first, r.m0, r.count, lane, s_rows);
+  list_rows<Tile::BM>(mask, first, r.m0, r.count, a.words, lane, wave, s_rows);
   __syncthreads();
   f32x4 acc[Tile::NT][Tile::MT];
 #pragma unroll
@@ -339,13 +345,13 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
     keep_slot(a, s_rows[threadIdx.x], r.e, r.base + r.m0 + threadIdx.x);
 }
 
-// grid = (ceil(dim / BN) * splits, row tiles); blockIdx.x is
-// column tile * splits + split.
+// grid = (ceil(dim / BN) * splits, row tiles); blockIdx.x is column tile *
+// splits + split.
 template <typename T, typename Tile>
 __global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
   __shared__ __align__(16) char lds[Tile::kLds];
   const int lane = threadIdx.x & 63;
-  const Rows r = find_rows(a, lane < a.E ? a.counts[lane] : 0, Tile::BM, lane);
+  const Rows r = find_rows(a, lane < a.E ? a.counts[lane] : 0, Tile::BM, lane, static_cast<int>(blockIdx.y));
   if (r.e < 0) return;
   const int tile = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
   const int64_t row_bytes = static_cast<int64_t>(a.hidden) * sizeof(T);
@@ -467,7 +473,7 @@ __global__ __launch_bounds__(256, 2) void moe_prompt_w1_few(PromptArgs a) {
     cnt = count_tokens(a, word, e0, lane, cnt);
   }
   if (blockIdx.x == 0 && e == 0 && wave == 0 && lane < a.E) a.counts[lane] = cnt;
-  const Rows r = find_rows(a, cnt, 32, lane);
+  const Rows r = find_rows(a, cnt, 32, lane, e);
   if (r.e < 0) return;
   const int bits = __popcll(mask);
   const int rank0 = wave_inclusive(bits, lane) - bits;
@@ -482,7 +488,7 @@ __global__ __launch_bounds__(256, 2) void moe_prompt_w1_few(PromptArgs a) {
       __syncthreads();  // the last tile's rows and sums are read
       Tile::prefetch(ws, wp, 0, row_bytes);
     }
-    if (wave == 0) list_rows<32>(mask, rank0, m0, r.count, lane, s_rows);
+    list_rows<32>(mask, rank0, m0, r.count, a.words, lane, wave, s_rows);
     mie::gemm::lds_barrier();
     auto store = [&](int n, int m, f32x4 sum) {
       const int c = n0 + n * 16 + g * 4, rank = m0 + m * 16 + i;
@@ -522,7 +528,7 @@ __global__ __launch_bounds__(256, 2) void moe_prompt_w2_few(PromptArgs a) {
   typename Tile::template Set<Tile::NT> ws[2];
   Tile::prefetch(ws, wp, k0, k1);
   __builtin_amdgcn_sched_barrier(0);
-  const Rows r = find_rows(a, lane < a.E ? cnt : 0, 32, lane);
+  const Rows r = find_rows(a, lane < a.E ? cnt : 0, 32, lane, e);
   if (r.e < 0) return;
   const char* h = a.h + static_cast<int64_t>(r.base) * row_bytes;
   float* part = a.part + (static_cast<int64_t>(split) * a.tokens * a.top_k + r.base) * a.dim;
@@ -564,13 +570,37 @@ Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hi
   p.few = slots <= 20 * static_cast<int64_t>(E);
   const int bn = p.few ? 32 : 64, kb = p.few ? 1024 : 128;
   p.rows = p.few ? E : static_cast<int32_t>(slots / 64 + std::min<int64_t>(E, slots));
-  // W2 has few column tiles: split its K until the launch holds about two
-  // (few rows) or four workgroups per CU.
+  // W2 has few column tiles, so its K is split.  bfloat16 and few rows wait on
+  // memory: until the launch holds two workgroups per CU, and, where that can
+  // be had, with a multiple of 8 column tiles x splits - workgroups are dealt
+  // to the 8 XCDs in turn, so each column tile is then read through one XCD's
+  // L2.  float32 tiles fill the matrix cores: the split with the least rounds
+  // over the 256 CUs per split (a round more costs a tile, a third of one is
+  // lost once) and partial sums (8 bytes each way per value and split, against
+  // a tile's time).  Measured, us for 1, 2, 3, 4, 5, 6, 8 splits: float32 128
+  // tokens, FFN 2048: 50, 29, 32, 26, 22, 26, 21; 300 tokens 53, 46, 35, 37,
+  // 38, 34, 37; 1000 tokens, FFN 3072: 130, 126, 114, 116, 121, 114, 118;
+  // bfloat16 512 tokens 20, 15, 18, 15, 20, 16, 17.
   const int64_t used = p.few ? std::min<int64_t>(E, slots) : slots / 64 + E / 2;
-  const int64_t groups = static_cast<int64_t>((dim + bn - 1) / bn) * std::max<int64_t>(1, used);
+  const int64_t columns = (dim + bn - 1) / bn;
+  const int64_t groups = columns * std::max<int64_t>(1, used);
   const int32_t steps = (hidden * elt + kb - 1) / kb;
-  const int64_t want = ((p.few ? 512 : 1024) + groups - 1) / groups;
-  const int32_t splits = static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>({want, kMaxSplits, steps / 2})));
+  const int32_t most = std::max<int32_t>(1, std::min<int32_t>(kMaxSplits, steps / 2));
+  int32_t splits = 1;
+  if (p.few || elt == 2) {
+    splits = static_cast<int32_t>(std::min<int64_t>(most, (511 + groups) / groups));
+    if (!p.few)
+      for (int32_t s = splits; s <= most; ++s)
+        if (columns * s % 8 == 0) {
+          splits = s;
+          break;
+        }
+  } else {
+    const double partials = 0.82 * static_cast<double>(slots) * dim / hidden;
+    auto cost = [&](int32_t s) { return (static_cast<double>((groups * s + 255) / 256) * 100 + 35) / s + partials / 100 * s; };
+    for (int32_t s = 2; s <= most; ++s)
+      if (cost(s) < cost(splits)) splits = s;
+  }
   p.split_len = (steps + splits - 1) / splits * kb;
   p.splits = (hidden * elt + p.split_len - 1) / p.split_len;
   return p;
