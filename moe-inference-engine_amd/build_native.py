@@ -3,7 +3,8 @@
     python moe-inference-engine_amd/build_native.py
 
 compiles each csrc/*.hip with hipcc (in parallel, one object per source) and
-links the objects into moe_engine/libmie_paged.so.  The library is written to
+links the objects into moe_engine/libmie_paged.so, and compiles the host side
+of the short calls (csrc/host_calls.cpp) into moe_engine/_host_calls.so.  The library is written to
 a temporary name first and renamed, so a process that already mapped the old
 file keeps a consistent copy.
 """
@@ -12,6 +13,7 @@ import os
 import shlex
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -21,6 +23,7 @@ REPO_ROOT = PKG_ROOT.parent
 CSRC = PKG_ROOT / "csrc"
 INCLUDE = REPO_ROOT / "include"
 OUTPUT = PKG_ROOT / "moe_engine" / "libmie_paged.so"
+HOST_OUTPUT = PKG_ROOT / "moe_engine" / "_host_calls.so"
 ARCH = os.environ.get("MIE_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops: keep the compiler from emitting v_pk_{add,mul,fma}_f32.
@@ -49,8 +52,32 @@ def _run(cmd, verbose):
 
 
 def build(verbose: bool = True) -> Path:
-    _link(sorted(CSRC.glob("*.hip")), OUTPUT, verbose)
+    with ThreadPoolExecutor(1) as pool:
+        host = pool.submit(_build_host, verbose)
+        _link(sorted(CSRC.glob("*.hip")), OUTPUT, verbose)
+        host.result()
     return OUTPUT
+
+
+def _build_host(verbose: bool) -> None:
+    """moe_engine/_host_calls.so: a Python module over torch's C++ tensors, no
+    device code (g++)."""
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = HOST_OUTPUT.with_name(HOST_OUTPUT.name + f".tmp{os.getpid()}")
+    rc, err = _run(
+        [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+         *(f"-isystem{p}" for p in cpp_extension.include_paths()), f"-I{sysconfig.get_paths()['include']}",
+         str(CSRC / "host_calls.cpp"), "-o", str(tmp),
+         *(f"-L{p}" for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10"],
+        verbose,
+    )
+    if rc != 0:
+        tmp.unlink(missing_ok=True)
+        raise RuntimeError(f"building {HOST_OUTPUT.name} failed ({rc}):\n{err}")
+    os.replace(tmp, HOST_OUTPUT)
 
 
 def _link(sources, output: Path, verbose: bool, extra=()) -> None:

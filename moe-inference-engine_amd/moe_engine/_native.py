@@ -229,6 +229,24 @@ except OSError as exc:  # reported by lib(); there is no substitute implementati
 HAS_HIP = _LIB is not None
 
 
+def _open_host():
+    """The compiled host side of the short calls (csrc/host_calls.cpp), bound
+    to the loaded library's entry points; None without it, and the same calls
+    then go through Python."""
+    if _LIB is None:
+        return None
+    try:
+        from moe_engine import _host_calls
+    except ImportError:
+        return None
+    entry_points = (_LIB.mie_paged_decode, _LIB.mie_paged_decode_append, _LIB.mie_paged_decode_plan, _LIB.mie_kv_gather)
+    _host_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in entry_points))
+    return _host_calls
+
+
+HOST = _open_host()
+
+
 def lib():
     """The loaded library; raises when it is missing or unloadable."""
     if _LIB is None:

@@ -391,6 +391,14 @@ class PagedKVCache:
         """Contiguous K, V [1, H, length, D] of logical positions 0..length-1."""
         alloc = self.allocator
         if alloc.on_device:
+            if _native.HOST is not None:
+                # The usual form in one compiled call; None for any other.
+                kv = _native.HOST.gather(alloc.k_pool, alloc.v_pool, layer_idx, self.block_table_device, length,
+                                         _native.stream_of(alloc.k_pool))
+                if type(kv) is int:
+                    _native.check(kv, "mie_kv_gather")
+                if kv is not None:
+                    return kv
             return kv_ops.gather(alloc.k_pool, alloc.v_pool, layer_idx, self.block_table_device, length)
         ids = self.block_table[: -(-length // alloc.block_size)]
 

@@ -245,6 +245,10 @@ def decode(q: torch.Tensor, cache, layer_idx: int, context_len: int) -> torch.Te
     return out.view(1, num_heads, 1, head_dim)
 
 
+# decode_batched's options that the compiled call takes.
+_HOST_KEYWORDS = {"context_lens_host", "scale", "partition_tokens", "k_new", "v_new"}
+
+
 def decode_batched(
     q: torch.Tensor,
     k_pool: torch.Tensor,
@@ -260,6 +264,19 @@ def decode_batched(
     q [B, H, D]; pools [L, NB, H, BS, D]; block_tables int32 [B, max_blocks];
     context_lens int32 [B] on the device; max_context_len a host bound.
     """
+    host = _native.HOST
+    if host is not None and kwargs.keys() <= _HOST_KEYWORDS and q.is_cuda:
+        # The usual form in one compiled call; None for any other, which the
+        # checks below take (or refuse).
+        out = host.decode(
+            q, k_pool, v_pool, layer_idx, block_tables, context_lens, max_context_len,
+            kwargs.get("context_lens_host"), kwargs.get("scale"), kwargs.get("partition_tokens", 0),
+            kwargs.get("k_new"), kwargs.get("v_new"), _native.stream_of(q),
+        )
+        if type(out) is int:
+            _native.check(out, "mie_paged_decode")
+        if out is not None:
+            return out
     return decode_layer(
         q,
         k_pool[layer_idx],
