@@ -30,16 +30,19 @@
 // every token takes, at any skew, and an expert without tokens is not read.
 //
 // Bounds: at few tokens the experts' bytes (768 x 2048 x 8 float32: 101 MB),
-// at many the matrix cores (float32: 153 TFLOP/s).  A whole layer on MI355X,
+// at many the matrix cores (float32 instructions: 153 TFLOP/s; the split form
+// also by the vector instructions that make the parts).  A whole layer on MI355X,
 // 8 experts, top-2, before (dense-masked library products up to 512 float32
 // tokens, the per-expert PyTorch path otherwise) and with these launches:
-// 32 tokens, FFN 2048, float32: 228 -> 47 us; 1000 tokens, FFN 3072, float32:
-// 1131 -> 229 us; 512 tokens, FFN 2048, bfloat16: 1140 -> 52 us.
+// 32 tokens, FFN 2048, float32: 228 -> 40 us; 1000 tokens, FFN 3072, float32:
+// 1131 -> 186 us; 512 tokens, FFN 2048, bfloat16: 1140 -> 43 us.
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_direct.h"
+#include "gemm_split.h"
 #include "gemm_tile.h"
 #include "mie_common.h"
 #include "moe_route.h"
@@ -289,9 +292,35 @@ __device__ __forceinline__ void keep_slot(const PromptArgs& a, int token, int e,
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752440f)); }
 
+template <typename Tile> struct Waves {
+  static constexpr int value = 1;
+};
+template <int MT, int NT> struct Waves<mie::gemm::SplitTile<MT, NT>> {
+  static constexpr int value = mie::gemm::SplitTile<MT, NT>::kWaves;
+};
+
+// Tile's product over its first `rows` rows.
+template <typename Tile, typename ARow, typename WRow>
+__device__ __forceinline__ void run_tile(char* lds, ARow a_row, WRow w_row, int k0, int k1, int rows,
+                                         f32x4 (&acc)[Tile::NT][Tile::MT]) {
+  if constexpr (std::is_same_v<Tile, mie::gemm::SplitTile<4, 1>>) {
+    if (rows > 48) {
+      Tile::template run<4>(lds, a_row, w_row, k0, k1, acc);
+    } else if (rows > 32) {
+      Tile::template run<3>(lds, a_row, w_row, k0, k1, acc);
+    } else if (rows > 16) {
+      Tile::template run<2>(lds, a_row, w_row, k0, k1, acc);
+    } else {
+      Tile::template run<1>(lds, a_row, w_row, k0, k1, acc);
+    }
+  } else {
+    Tile::run(lds, a_row, w_row, k0, k1, acc);
+  }
+}
+
 // grid = (ceil(hidden / BN), row tiles).
 template <typename T, typename Tile>
-__global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
+__global__ __launch_bounds__(256, Waves<Tile>::value) void moe_prompt_w1(PromptArgs a) {
   __shared__ __align__(16) char lds[Tile::kLds];
   __shared__ int s_rows[Tile::BM];
   const int lane = threadIdx.x & 63;
@@ -323,9 +352,10 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
   for (int n = 0; n < Tile::NT; ++n)
 #pragma unroll
     for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Tile::run(
+  run_tile<Tile>(
       lds, [&](int i) { return x + s_rows[i] * row_bytes; },
-      [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes), acc);
+      [&](int i) { return w + min(n0 + i, a.hidden - 1) * row_bytes; }, 0, static_cast<int>(row_bytes),
+      r.count - r.m0, acc);
 #pragma unroll
   for (int n = 0; n < Tile::NT; ++n) {
     const int c = n0 + Tile::col(n);
@@ -348,7 +378,7 @@ __global__ __launch_bounds__(256) void moe_prompt_w1(PromptArgs a) {
 // grid = (ceil(dim / BN) * splits, row tiles); blockIdx.x is column tile *
 // splits + split.
 template <typename T, typename Tile>
-__global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
+__global__ __launch_bounds__(256, Waves<Tile>::value) void moe_prompt_w2(PromptArgs a) {
   __shared__ __align__(16) char lds[Tile::kLds];
   const int lane = threadIdx.x & 63;
   const Rows r = find_rows(a, lane < a.E ? a.counts[lane] : 0, Tile::BM, lane, static_cast<int>(blockIdx.y));
@@ -366,9 +396,9 @@ __global__ __launch_bounds__(256) void moe_prompt_w2(PromptArgs a) {
   for (int n = 0; n < Tile::NT; ++n)
 #pragma unroll
     for (int m = 0; m < Tile::MT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Tile::run(
+  run_tile<Tile>(
       lds, [&](int i) { return h + min(r.m0 + i, r.count - 1) * row_bytes; },
-      [&](int i) { return w + min(n0 + i, a.dim - 1) * row_bytes; }, k0, k1, acc);
+      [&](int i) { return w + min(n0 + i, a.dim - 1) * row_bytes; }, k0, k1, r.count - r.m0, acc);
 #pragma unroll
   for (int n = 0; n < Tile::NT; ++n) {
     const int c = n0 + Tile::col(n);
@@ -552,8 +582,16 @@ __global__ __launch_bounds__(256, 2) void moe_prompt_w2_few(PromptArgs a) {
   }
 }
 
-// More rows: LDS-staged tiles of 64 x 64.
-template <typename T> using Wide = mie::gemm::Tile<T, 64, 64, 128, 2, 2>;
+// More rows: LDS-staged tiles of 64 x 64, for float32 on the bfloat16 matrix
+// cores (gemm_split.h) and over the rows a tile has, 16 to 64 (1000 tokens,
+// top-2 of 8, FFN 3072: W1 127 -> 98 us, W2 116 -> 89).
+template <typename T> struct WideTile {
+  using type = mie::gemm::Tile<T, 64, 64, 128, 2, 2>;
+};
+template <> struct WideTile<float> {
+  using type = mie::gemm::SplitTile<4, 1>;
+};
+template <typename T> using Wide = typename WideTile<T>::type;
 
 struct Plan {
   bool few;
@@ -563,7 +601,7 @@ struct Plan {
 
 // Few rows: up to 20 per expert on average.  At 16 (62 tokens, 8 experts,
 // top-2, float32) both forms take 36-38 us for the two products, at 8 the
-// direct tiles 29 against 35 us, at 32 the staged ones 50 against 62 us.
+// direct tiles 29 against 35 us, at 32 the staged ones 50 against 62 us (in float32 instructions).
 Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden, int elt) {
   Plan p;
   const int64_t slots = static_cast<int64_t>(tokens) * top_k;
@@ -577,10 +615,9 @@ Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hi
   // L2.  float32 tiles fill the matrix cores: the split with the least rounds
   // over the 256 CUs per split (a round more costs a tile, a third of one is
   // lost once) and partial sums (8 bytes each way per value and split, against
-  // a tile's time).  Measured, us for 1, 2, 3, 4, 5, 6, 8 splits: float32 128
-  // tokens, FFN 2048: 50, 29, 32, 26, 22, 26, 21; 300 tokens 53, 46, 35, 37,
-  // 38, 34, 37; 1000 tokens, FFN 3072: 130, 126, 114, 116, 121, 114, 118;
-  // bfloat16 512 tokens 20, 15, 18, 15, 20, 16, 17.
+  // a tile's time).  Measured, us for 1, 2, 3, 4, 5, 6, 8 splits: float32 1000
+  // tokens, FFN 3072, whole layer: 188, 197, 183, 181, 187, 183, 189; bfloat16
+  // 512 tokens 20, 15, 18, 15, 20, 16, 17.
   const int64_t used = p.few ? std::min<int64_t>(E, slots) : slots / 64 + E / 2;
   const int64_t columns = (dim + bn - 1) / bn;
   const int64_t groups = columns * std::max<int64_t>(1, used);
@@ -596,8 +633,8 @@ Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hi
           break;
         }
   } else {
-    const double partials = 0.82 * static_cast<double>(slots) * dim / hidden;
-    auto cost = [&](int32_t s) { return (static_cast<double>((groups * s + 255) / 256) * 100 + 35) / s + partials / 100 * s; };
+    const double partials = 1.25 * static_cast<double>(slots) * dim / hidden;
+    auto cost = [&](int32_t s) { return (static_cast<double>((groups * s + 255) / 256) * 100 + 53) / s + partials / 100 * s; };
     for (int32_t s = 2; s <= most; ++s)
       if (cost(s) < cost(splits)) splits = s;
   }

@@ -15,9 +15,9 @@
 // Launches: norm (block form), QKV, attention, output projection.  Few tokens
 // are bound by the launches and the weights, many by the matrix cores.  A
 // layer on MI355X, 12 heads x 64, against library products, PyTorch's
-// attention and the append launch: 1000 tokens float32 126 -> 102 us, 333
+// attention and the append launch: 1000 tokens float32 126 -> 77 us, 333
 // tokens bfloat16 85 -> 25 us; with the MoE half, 62 tokens float32 through 12
-// blocks and the head 4.1 -> 1.1 ms.
+// blocks and the head 4.1 -> 0.95 ms.
 //
 // Attention.  One workgroup per (head, 16 queries); its four waves take
 // every fourth block of 32 keys and merge their softmax states in LDS once.
@@ -32,6 +32,7 @@
 #include <algorithm>
 
 #include "gemm_direct.h"
+#include "gemm_split.h"
 #include "gemm_tile.h"
 #include "mie_common.h"
 #include "row_norm.h"
@@ -118,10 +119,8 @@ __device__ __forceinline__ f32x4 bias_of(const LinearArgs& a, int c) {
   return Mem<T>::load4(reinterpret_cast<const T*>(a.bias) + c);
 }
 
-// grid = (ceil(n / BN), ceil(rows / BM)).
 template <typename T, typename Tile>
-__global__ __launch_bounds__(256) void prompt_linear_kernel(LinearArgs a) {
-  __shared__ __align__(16) char lds[Tile::kLds];
+__device__ __forceinline__ void linear_tile(const LinearArgs& a, char* lds) {
   const int n0 = blockIdx.x * Tile::BN, m0 = blockIdx.y * Tile::BM;
   const int64_t row_bytes = static_cast<int64_t>(a.k) * sizeof(T);
   f32x4 acc[Tile::NT][Tile::MT];
@@ -146,6 +145,20 @@ __global__ __launch_bounds__(256) void prompt_linear_kernel(LinearArgs a) {
       if (r < a.rows) store_linear<T>(a, r, c, acc[n][m], b, blk[m]);
     }
   }
+}
+
+// grid = (ceil(n / BN), ceil(rows / BM)).
+template <typename T, typename Tile>
+__global__ __launch_bounds__(256) void prompt_linear_kernel(LinearArgs a) {
+  __shared__ __align__(16) char lds[Tile::kLds];
+  linear_tile<T, Tile>(a, lds);
+}
+
+// The same on gemm_split.h's tiles.
+template <typename Tile>
+__global__ __launch_bounds__(256, Tile::kWaves) void prompt_linear_split_kernel(LinearArgs a) {
+  __shared__ __align__(16) char lds[Tile::kLds];
+  linear_tile<float, Tile>(a, lds);
 }
 
 // grid = (ceil(n / BN), ceil(rows / (16 MT))): few rows.
@@ -415,6 +428,13 @@ void launch_tile(const LinearArgs& a, hipStream_t st) {
       <<<dim3((a.n + Tile::BN - 1) / Tile::BN, (a.rows + Tile::BM - 1) / Tile::BM), 256, 0, st>>>(a);
 }
 
+template <int MT, int NT>
+void launch_split(const LinearArgs& a, hipStream_t st) {
+  using Tile = mie::gemm::SplitTile<MT, NT>;
+  prompt_linear_split_kernel<Tile>
+      <<<dim3((a.n + Tile::BN - 1) / Tile::BN, (a.rows + Tile::BM - 1) / Tile::BM), 256, 0, st>>>(a);
+}
+
 template <typename T, typename Tile, int MT>
 void launch_direct(const LinearArgs& a, hipStream_t st) {
   prompt_linear_direct_kernel<T, Tile, MT>
@@ -422,32 +442,64 @@ void launch_direct(const LinearArgs& a, hipStream_t st) {
 }
 
 // Fewer than 128 tiles of 32 x 32 (few rows): direct tiles, the larger that
-// still makes 128 workgroups.  Otherwise the staged tile whose last round of
-// workgroups over the 256 CUs wastes least - rounds x tile area; on a tie the
-// smallest tile while it makes at most 512 workgroups (more of them hide each
-// other's waits), the largest beyond (less operand traffic).  Measured on
-// MI355X, float32, K 768, 64x48 / 32x64 / 32x32 / 64x64: 1000 x 2304 44.1 /
-// 45.8 / - / 50.3 us, 1000 x 768 18.7 / 21.6 / - / 22.0, 512 x 768 17.5 / 14.4
-// / 12.8 / -, 200 x 2304 - / 16.5 / 15.0 / -; 62 x 2304 9.7 us with 32x32 and
-// 10.6 with direct tiles, 62 x 768 8.8 and 5.6.
+// still makes 128 workgroups.
+//
+// float32 beyond: the tile of the least estimated time.  A first round of
+// workgroups over the 256 CUs takes `first`, each further one, overlapping,
+// `more` (us at K 768 with the epilogue; every tile scales with K alike).  Split tiles
+// win from about 320 x 2304 on; below, the small tile's rounds are few and the
+// shortest (300 tokens: a layer in 35 us with it, 37 with 48x64 split).  Measured on MI355X, us, 32x32 / 64x48 in float32
+// instructions, then split 32x64 / 48x64 / 64x64 / 64x128, products alone: 1000 x 2304 44 / 42
+// - 40 / 31 / 33 / 39; 1000 x 768 16 / 16 - 16 / 17 / 18 / 25; 333 x 2304 20 / 26
+// - 16 / 17 / 17 / 27; 2048 x 3072 103 / 99 - 86 / 77 / 63 / 60; 62 x 2304 8 / 16
+// - 13 / 16 / 17 / 24.
+//
+// bfloat16: the staged tile whose last round wastes least - rounds x tile area;
+// on a tie the smallest tile while it makes at most 512 workgroups (more of
+// them hide each other's waits), the largest beyond (less operand traffic).
 template <typename T>
 int32_t launch_linear(const LinearArgs& a, hipStream_t st) {
   auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((a.rows + bm - 1) / bm) * ((a.n + bn - 1) / bn); };
-  auto cost = [&](int bm, int bn) { return (tiles(bm, bn) + 255) / 256 * bm * bn; };
-  const int64_t big = cost(64, 48), mid = cost(32, 64), small = cost(32, 32);
-  const bool favour_small = tiles(32, 32) <= 512;
+  auto rounds = [&](int bm, int bn) { return (tiles(bm, bn) + 255) / 256; };
   if (tiles(32, 32) < 128) {
     if (tiles(32, 16) >= 128) {
       launch_direct<T, Direct<T, 1, 6>, 2>(a, st);
     } else {
       launch_direct<T, Direct<T, 1, 6>, 1>(a, st);
     }
-  } else if (favour_small ? small <= mid && small <= big : small < mid && small < big) {
-    launch_tile<T, Tile<T, 32, 32, 256, 2, 2>>(a, st);
-  } else if (mid < big) {
-    launch_tile<T, Tile<T, 32, 64, 128, 2, 2>>(a, st);
+  } else if constexpr (sizeof(T) == 4) {
+    struct Form {
+      int bm, bn;
+      float first, more;
+      void (*launch)(const LinearArgs&, hipStream_t);
+    };
+    static constexpr Form kForms[] = {
+        {32, 32, 8.0f, 4.6f, launch_tile<T, Tile<T, 32, 32, 256, 2, 2>>},
+        {32, 64, 13.9f, 6.6f, launch_split<2, 1>},
+        {48, 64, 17.7f, 7.3f, launch_split<3, 1>},
+        {64, 64, 18.5f, 8.6f, launch_split<4, 1>},
+        {64, 128, 26.0f, 16.5f, launch_split<4, 2>},
+    };
+    const Form* best = nullptr;
+    float least = 0.f;
+    for (const Form& f : kForms) {
+      const float cost = f.first + f.more * static_cast<float>(rounds(f.bm, f.bn) - 1);
+      if (!best || cost < least) {
+        best = &f;
+        least = cost;
+      }
+    }
+    best->launch(a, st);
   } else {
-    launch_tile<T, Tile<T, 64, 48, 256, 4, 1>>(a, st);
+    auto cost = [&](int bm, int bn) { return rounds(bm, bn) * bm * bn; };
+    const int64_t big = cost(64, 48), mid = cost(32, 64), small = cost(32, 32);
+    if (tiles(32, 32) <= 512 ? small <= mid && small <= big : small < mid && small < big) {
+      launch_tile<T, Tile<T, 32, 32, 256, 2, 2>>(a, st);
+    } else if (mid < big) {
+      launch_tile<T, Tile<T, 32, 64, 128, 2, 2>>(a, st);
+    } else {
+      launch_tile<T, Tile<T, 64, 48, 256, 4, 1>>(a, st);
+    }
   }
   return mie::check_launch("prompt_linear_kernel");
 }
