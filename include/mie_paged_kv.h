@@ -208,11 +208,11 @@ int32_t mie_paged_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,
  * new_stride_h, inner axis contiguous, `dtype`) are stored at position
  * ctx_b - 1 through the block table, exactly as mie_kv_append stores them,
  * and the output is mie_paged_decode's over tokens [0, ctx_b) with that token
- * included.  The pools are written.  When the plan takes the workgroup form
- * this is ONE launch: the decode kernel stores the rows and takes the new
- * token's score and value from the rows it loaded, without reading them back;
- * otherwise the append runs as its own launch before the decode, on the same
- * stream.  A sequence with ctx_b = 0 gets no append and a zero output; a new
+ * included.  The pools are written.  When the plan takes the workgroup form,
+ * or partitions of one sequence, the decode kernel stores the rows and takes
+ * the new token's score and value from the rows it loaded, without reading
+ * them back; otherwise the append runs as its own launch before the decode, on
+ * the same stream.  A sequence with ctx_b = 0 gets no append and a zero output; a new
  * token whose block id is outside the pool is not stored and its output is
  * NaN.  Other arguments and limits as mie_paged_decode.
  */

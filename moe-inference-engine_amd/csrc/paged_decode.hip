@@ -1171,15 +1171,18 @@ int32_t decode_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h, const
     if (blocks <= kWindow) a.win_blocks = static_cast<int32_t>(blocks);
   }
   if (k_new) {
-    if (p.wg || flat_items > 0) {
+    if (p.wg || (flat_items > 0 && batch == 1)) {
       // The decode kernel stores the rows and attends to the new token itself
-      // (1 x 2048 bf16: two launches instead of three).
+      // (1 x 2048 bf16: two launches instead of three).  In partitions for one
+      // sequence only: several may name the same blocks (the last tokens of one
+      // sequence at several lengths), and each must then see what the others
+      // append.
       a.k_new = static_cast<const char*>(k_new);
       a.v_new = static_cast<const char*>(v_new);
       a.new_sb = new_stride_b;
       a.new_sh = new_stride_h;
     } else {
-      // Grid form: append each sequence's last token first (same stream).
+      // Append each sequence's last token first (same stream).
       const int32_t rc = mie::kv_append_impl(const_cast<void*>(k_pool), const_cast<void*>(v_pool), pool_stride_block,
                                              pool_stride_head, num_blocks, k_new, v_new, new_stride_b, new_stride_h, 0,
                                              block_tables, block_table_stride, ctx_lens, ctx_len, -1, batch, 1,

@@ -76,7 +76,7 @@ def decode_layer(
     With k_new / v_new ([B, H, D], the pools' dtype) the step's append is
     fused in: each sequence's new token is its last context token, stored at
     position ctx_b - 1 through the table and attended to (mie_paged_decode_append;
-    one launch when the plan takes the workgroup form).
+    no launch of its own in the workgroup form or for one sequence).
     """
     lib = _native.lib()
     if q.dim() != 3:

@@ -39,6 +39,19 @@ def test_fused_append_equals_append_then_decode(heads, head_dim, block_size, dty
         out_dtype=torch.float32)
     assert torch.equal(w.k_pool, pools[0]) and torch.equal(w.v_pool, pools[1])
     assert (got - want).abs().max().item() <= 4e-6
+    # Each sequence alone (the fused form), from pools without the new rows.
+    for b, n in enumerate(lens):
+        w1 = make_workload(lens, num_heads=heads, head_dim=head_dim, block_size=block_size, dtype=dtype, seed=3)
+        take_last_tokens(w1)
+        alone = paged_attention.decode_batched(
+            w1.q[b : b + 1], w1.k_pool, w1.v_pool, 0, w1.block_tables[b : b + 1], w1.context_lens[b : b + 1], max(n, 1),
+            partition_tokens=part, context_lens_host=[n], k_new=k_new[b : b + 1], v_new=v_new[b : b + 1],
+            out_dtype=torch.float32)
+        assert (alone[0] - want[b]).abs().max().item() <= 4e-6
+        if n > 0:
+            at = w.block_tables[b, (n - 1) // block_size], (n - 1) % block_size
+            for mine, theirs in ((w1.k_pool, pools[0]), (w1.v_pool, pools[1])):
+                assert torch.equal(mine[0, at[0], :, at[1]], theirs[0, at[0], :, at[1]])
     # A launch bound instead of the exact list, and a bad block id for one sequence.
     again = paged_attention.decode_batched(
         w.q, w.k_pool, w.v_pool, 0, w.block_tables, w.context_lens, w.max_len, partition_tokens=part, k_new=k_new,
@@ -54,6 +67,26 @@ def test_fused_append_equals_append_then_decode(heads, head_dim, block_size, dty
     assert bad[8].isnan().all() and torch.equal(w.k_pool, before)
     rest = [b for b in range(len(lens)) if b != 8]
     assert torch.equal(bad[rest], got[rest])
+
+
+def test_rows_of_one_sequence_see_each_others_tokens():
+    """Three rows share one block table at lengths n, n + 1, n + 2: each
+    attends to the tokens the shorter ones append in the same call."""
+    w = make_workload([700], num_heads=12, head_dim=64, block_size=16, dtype=torch.float32, seed=5)
+    lens = [698, 699, 700]
+    tables = w.block_tables.expand(3, -1).contiguous()
+    q, k_new, v_new = (torch.randn(3, 12, 64, device="cuda") for _ in range(3))
+    context = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    print_case("shared table")
+    got = paged_attention.decode_batched(q, w.k_pool, w.v_pool, 0, tables, context, 700, partition_tokens=256,
+                                         context_lens_host=lens, k_new=k_new, v_new=v_new)
+    want = paged_attention.decode_batched(q, w.k_pool, w.v_pool, 0, tables, context, 700, partition_tokens=256,
+                                          context_lens_host=lens)
+    assert torch.equal(got, want)
+    ids = tables[0].long()
+    for pool, new in ((w.k_pool, k_new), (w.v_pool, v_new)):
+        rows = pool[0, ids].transpose(0, 1).reshape(12, -1, 64)[:, 697:700]
+        assert torch.equal(rows, new.transpose(0, 1))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16, torch.float64])
