@@ -14,6 +14,7 @@ from functools import lru_cache
 from pathlib import Path
 
 import torch
+from torch.utils._device import DeviceContext
 
 LIB_NAME = "libmie_paged.so"
 LIB_PATH = Path(__file__).resolve().parent / LIB_NAME
@@ -272,8 +273,9 @@ def is_rocm_device(t: torch.Tensor) -> bool:
 def plain_inference(x: torch.Tensor) -> bool:
     """True when a library call may stand in for PyTorch operations on x:
     nothing is recorded, traced, transformed or re-dispatched (no gradients,
-    autocast, forward-mode AD, functorch transform, tracing, compilation or
-    dispatch mode), and x is a plain tensor."""
+    autocast, forward-mode AD, functorch transform, tracing, compilation,
+    dispatch or function mode but a default device's), and x is a plain
+    tensor."""
     return (
         not torch.is_grad_enabled()
         and type(x) in (torch.Tensor, torch.nn.Parameter)
@@ -281,6 +283,10 @@ def plain_inference(x: torch.Tensor) -> bool:
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0
         and torch._C._len_torch_dispatch_stack() == 0
+        and all(
+            type(torch._C._get_function_stack_at(i)) is DeviceContext
+            for i in range(torch._C._len_torch_function_stack())
+        )
         and not torch.jit.is_tracing()
         and not torch.compiler.is_compiling()
     )

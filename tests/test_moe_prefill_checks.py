@@ -68,3 +68,21 @@ def test_plain_experts_are_recognised():
         layer = MoEFeedForward(16, 32, 3, 2)
         change(layer)
         assert not layer._experts_are_plain()
+
+
+def test_only_plain_inference_is_stood_in_for():
+    x = torch.randn(2, 4)
+    assert not _native.plain_inference(x)  # gradients on
+
+    class Counting(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        assert _native.plain_inference(x)
+        with torch.device("cpu"):  # a default device changes no operation on x
+            assert _native.plain_inference(x)
+        with Counting():
+            assert not _native.plain_inference(x)
+        with torch.autograd.forward_ad.dual_level():
+            assert not _native.plain_inference(x)
