@@ -381,8 +381,8 @@ int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts, int32_t t
                                   int32_t dtype);
 int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ln_weight, const void* ln_bias, float ln_eps,
                         const void* residual, const void* router_weight, const void* w1, const void* b1,
-                        const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace, int64_t workspace_bytes, int32_t dtype,
-                        void* stream);
+                        const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden,
+                        void* out, void* workspace, int64_t workspace_bytes, int32_t dtype, void* stream);
 
 /*
  * Attention over a prompt at position 0 (CachedAttention.forward,

@@ -585,6 +585,8 @@ __global__ __launch_bounds__(256, 2) void moe_prompt_w2_few(PromptArgs a) {
 // More rows: LDS-staged tiles of 64 x 64, for float32 on the bfloat16 matrix
 // cores (gemm_split.h) and over the rows a tile has, 16 to 64 (1000 tokens,
 // top-2 of 8, FFN 3072: W1 127 -> 98 us, W2 116 -> 89).
+// bfloat16 waits on memory and barriers, hidden by four workgroups per CU: steps
+// of 256 bytes (two per CU) take 53 us a layer for 512 tokens, FFN 2048, these 43.
 template <typename T> struct WideTile {
   using type = mie::gemm::Tile<T, 64, 64, 128, 2, 2>;
 };
@@ -754,8 +756,9 @@ extern "C" int64_t mie_moe_prefill_workspace(int64_t tokens, int32_t num_experts
 
 extern "C" int32_t mie_moe_prefill(const void* x, int64_t tokens, const void* ln_weight, const void* ln_bias,
                                    float ln_eps, const void* residual, const void* router_weight, const void* w1,
-                                   const void* b1, const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim, int32_t hidden, void* out, void* workspace,
-                                   int64_t workspace_bytes, int32_t dtype, void* stream) {
+                                   const void* b1, const void* w2, const void* b2, int32_t num_experts, int32_t top_k, int32_t dim,
+                                   int32_t hidden, void* out, void* workspace, int64_t workspace_bytes, int32_t dtype,
+                                   void* stream) {
   mie::clear_error();
   int32_t rc = check(tokens, num_experts, top_k, dim, hidden, dtype);
   if (rc != MIE_OK) return rc;
