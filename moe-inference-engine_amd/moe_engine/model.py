@@ -498,11 +498,15 @@ class CachedAttention(_TracksReplacement, nn.Module):
         ):
             return False
         pool, dim = alloc.k_pool, x.shape[2]
-        out = self._modules["out_proj"]
+        out = self._modules.get("out_proj")
         params = self._parameters
-        w_in, b_in = params["in_proj_weight"], params["in_proj_bias"]
+        # Pruning, weight norm and parametrizations take the names out of the
+        # registered parameters and compute them: forward then reads them.
+        w_in, b_in = params.get("in_proj_weight"), params.get("in_proj_bias")
         return (
-            type(out) is Linear
+            w_in is not None
+            and "in_proj_bias" in params
+            and type(out) is Linear
             and _plain_module(out)
             and (alloc.num_heads, alloc.head_dim) == (self.num_heads, self.head_dim)
             and self.num_heads * self.head_dim == dim
@@ -927,7 +931,7 @@ class TransformerMoEBlock(nn.Module):
         residual), then the MoE half (fused_moe.prefill likewise).  None when
         the two do not both apply or a module in between is not plain."""
         m = self._modules
-        att, moe, an, mn = m["attention"], m["moe"], m["attn_norm"], m["moe_norm"]
+        att, moe, an, mn = (m.get(name) for name in ("attention", "moe", "attn_norm", "moe_norm"))
         if not (type(att) is CachedAttention and type(moe) is MoEFeedForward and _plain_module(att)
                 and _plain_module(moe) and att.prompt_supported(x, cache, layer_idx)):
             return None
