@@ -270,6 +270,10 @@ def is_rocm_device(t: torch.Tensor) -> bool:
     return t.is_cuda and torch.version.hip is not None
 
 
+# Types whose data_ptr() is the tensor's own memory.
+PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
 def plain_inference(x: torch.Tensor) -> bool:
     """True when a library call may stand in for PyTorch operations on x:
     nothing is recorded, traced, transformed or re-dispatched (no gradients,
@@ -278,7 +282,7 @@ def plain_inference(x: torch.Tensor) -> bool:
     tensor."""
     return (
         not torch.is_grad_enabled()
-        and type(x) in (torch.Tensor, torch.nn.Parameter)
+        and type(x) in PLAIN_TENSORS
         and not torch.is_autocast_enabled()
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0

@@ -243,7 +243,8 @@ def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int
         and dim % vec == 0
         and hidden % vec == 0
         and all(
-            t.shape == shape and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
+            type(t) in _native.PLAIN_TENSORS and t.shape == shape and t.dtype == dtype and t.device == device
+            and t.is_contiguous() and t.data_ptr() % 16 == 0
             for t, shape in (
                 (router_weight, (num_experts, dim)),
                 (w1, (num_experts, hidden, dim)),
@@ -274,10 +275,12 @@ def prefill(x, router_weight, w1_base, b1_base, w2_base, b2_base, *, top_k: int,
     if norm is not None:
         weight, bias, eps = norm
         for t in (weight, bias):
-            if t is not None and (t.shape != (dim,) or not t.is_contiguous() or t.dtype != x.dtype or t.device != x.device):
+            if t is not None and (type(t) not in _native.PLAIN_TENSORS or t.shape != (dim,) or not t.is_contiguous()
+                                  or t.dtype != x.dtype or t.device != x.device):
                 raise ValueError(f"norm parameters must be contiguous [{dim}] vectors like x")
         ln_w, ln_b = weight.data_ptr(), _native.ptr(bias)
-    if residual is not None and (residual.shape != x.shape or not residual.is_contiguous() or residual.dtype != x.dtype
+    if residual is not None and (type(residual) not in _native.PLAIN_TENSORS or residual.shape != x.shape
+                                 or not residual.is_contiguous() or residual.dtype != x.dtype
                                  or residual.device != x.device):
         raise ValueError("the residual must be contiguous and like x")
     out = torch.empty_like(x)

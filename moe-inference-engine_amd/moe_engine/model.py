@@ -78,10 +78,11 @@ def _plain_module(module) -> bool:
 
 
 def _like(t, shape, x) -> bool:
-    """A parameter the kernels can read beside x: this shape, x's dtype and
-    device, contiguous, 16-byte aligned."""
-    return (t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
-            and t.data_ptr() % 16 == 0)
+    """A parameter the kernels can read beside x: a plain tensor (a wrapper
+    subclass has no memory of its own), this shape, x's dtype and device,
+    contiguous, 16-byte aligned."""
+    return (type(t) in _native.PLAIN_TENSORS and t.shape == shape and t.dtype == x.dtype and t.device == x.device
+            and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
 def _aligned(x):
@@ -794,7 +795,7 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
                 if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
                     return False
             for i, t in enumerate((*up._parameters.values(), *down._parameters.values())):  # weight, bias each
-                if t is None or t.data_ptr() != at[i]:
+                if type(t) not in _native.PLAIN_TENSORS or t.data_ptr() != at[i]:
                     return False
                 at[i] += step[i]
         return True

@@ -6,8 +6,8 @@ import pytest
 import torch
 from torch.nn.utils import parametrize, prune
 
-from moe_engine import _native, paged_attention
-from moe_engine.model import BlockAllocator, CachedAttention, ModelConfig, TransformerMoEBlock
+from moe_engine import _native, fused_moe, paged_attention
+from moe_engine.model import BlockAllocator, CachedAttention, ModelConfig, MoEFeedForward, TransformerMoEBlock
 
 DIM, HEADS = 64, 2
 
@@ -90,3 +90,76 @@ def test_a_part_of_the_block_that_is_no_module_keeps_the_pytorch_path(cache, nam
     object.__setattr__(block, name, part)
     with torch.no_grad():
         assert block._prompt(torch.randn(1, 5, DIM), cache, 0) is None
+
+
+class Wrapped(torch.Tensor):
+    """A tensor that holds another one and has no memory of its own, as
+    quantized and distributed tensors do."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, strides=inner.stride(), dtype=inner.dtype,
+                                                   device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        args, kwargs = torch.utils._pytree.tree_map_only(cls, lambda t: t.inner, (args, kwargs or {}))
+        out = func(*args, **kwargs)
+        return cls(out) if func is torch.ops.aten.detach.default else out
+
+
+def replace(module, name, make):
+    owner, _, leaf = name.rpartition(".")
+    owner = module.get_submodule(owner)
+    with torch.no_grad():
+        setattr(owner, leaf, torch.nn.Parameter(make(getattr(owner, leaf).detach()), requires_grad=False))
+
+
+@pytest.mark.parametrize("name", ["in_proj_weight", "in_proj_bias", "out_proj.weight", "out_proj.bias"])
+def test_tensors_without_memory_keep_the_pytorch_path(cache, name):
+    torch.manual_seed(0)
+    att = CachedAttention(DIM, HEADS).eval()
+    x = torch.randn(1, 5, DIM)
+    with torch.no_grad():
+        cache.attention_mode = "gather"
+        want = att(x, cache, 0, 0)
+        cache.attention_mode = "auto"
+        replace(att, name, Wrapped)
+        assert att.get_parameter(name).data_ptr() == 0
+        assert not att.prompt_supported(x, cache, 0)
+        torch.testing.assert_close(att(x, cache, 0, 0), want)
+
+
+@pytest.mark.parametrize("name", ["attn_norm.weight", "attn_norm.bias", "moe_norm.weight", "moe_norm.bias"])
+def test_norms_without_memory_keep_the_pytorch_path(cache, monkeypatch, name):
+    monkeypatch.setattr(MoEFeedForward, "uses_grouped_prefill", lambda *a, **k: True)
+    monkeypatch.setattr(CachedAttention, "_prompt", lambda self, x, *a, **k: x)
+    monkeypatch.setattr(MoEFeedForward, "_forward_grouped", lambda self, x, **k: x)
+    block = TransformerMoEBlock(ModelConfig(num_layers=1, hidden_dim=DIM, num_heads=HEADS, num_experts=2)).eval()
+    x = torch.randn(1, 5, DIM)
+    with torch.no_grad():
+        assert block._prompt(x, cache, 0) is x
+        replace(block, name, Wrapped)
+        assert block._prompt(x, cache, 0) is None
+
+
+def test_moe_weights_without_memory_keep_the_pytorch_path(monkeypatch):
+    monkeypatch.setattr(_native, "is_rocm_device", lambda t: True)
+    layer = MoEFeedForward(16, 32, 3, 2).eval()
+    x, s = torch.randn(1, 4, 16), layer._expert_storage
+    parts = [layer.router.weight, s["w1"], s["b1"], s["w2"], s["b2"]]
+    with torch.no_grad():
+        assert fused_moe.prefill_supported(x, *parts, 2)
+        for i in range(len(parts)):
+            changed = [Wrapped(t.detach()) if i == j else t for j, t in enumerate(parts)]
+            assert not fused_moe.prefill_supported(x, *changed, 2)
+    assert layer._experts_are_plain()
+
+    class Named(torch.Tensor):
+        pass
+
+    replace(layer, "experts.1.net.2.bias", lambda t: t.as_subclass(Named))
+    assert not layer._experts_are_plain()
