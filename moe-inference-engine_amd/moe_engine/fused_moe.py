@@ -40,6 +40,7 @@ HAS_HIP = _native.HAS_HIP
 MAX_EXPERTS = 64
 MAX_TOP_K = 8
 MAX_HIDDEN_DIM = 2048  # the W1 kernel holds x in 8 loads per lane
+MAX_PREFILL_DIM = 1 << 20  # mie_moe_prefill's limit for both widths
 DTYPES = (torch.float32, torch.bfloat16)
 
 
@@ -238,8 +239,8 @@ def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int
         x.shape[-1] == dim
         and 0 < num_experts <= MAX_EXPERTS
         and 0 < top_k <= min(MAX_TOP_K, num_experts)
-        and dim > 0
-        and hidden > 0
+        and 0 < dim <= MAX_PREFILL_DIM
+        and 0 < hidden <= MAX_PREFILL_DIM
         and dim % vec == 0
         and hidden % vec == 0
         and all(

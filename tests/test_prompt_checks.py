@@ -163,3 +163,13 @@ def test_moe_weights_without_memory_keep_the_pytorch_path(monkeypatch):
 
     replace(layer, "experts.1.net.2.bias", lambda t: t.as_subclass(Named))
     assert not layer._experts_are_plain()
+
+
+@pytest.mark.parametrize("dim,hidden", [(1 << 20, 4), ((1 << 20) + 4, 4), (4, 1 << 20), (4, (1 << 20) + 4)])
+def test_supported_widths_are_the_entry_points(monkeypatch, dim, hidden):
+    """A width that the launches refuse is declined, not an error."""
+    monkeypatch.setattr(_native, "is_rocm_device", lambda t: True)
+    parts = [torch.zeros(s) for s in ((1, dim), (1, hidden, dim), (1, hidden), (1, dim, hidden), (1, dim))]
+    taken = fused_moe.prefill_supported(torch.zeros(1, 2, dim), *parts, 1)
+    assert taken == (max(dim, hidden) <= 1 << 20)
+    assert taken == (_native.lib().mie_moe_prefill_workspace(2, 1, 1, dim, hidden, 0) > 0)
