@@ -217,4 +217,13 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, g_met
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&g_module); }
+// abi_version: the header's version these calls were compiled for; bind() is
+// for a library of the same one.
+PyMODINIT_FUNC PyInit__host_calls() {
+  PyObject* m = PyModule_Create(&g_module);
+  if (m && PyModule_AddIntConstant(m, "abi_version", MIE_ABI_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

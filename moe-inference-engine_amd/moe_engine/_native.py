@@ -10,6 +10,7 @@ missing, `lib()` raises and every device entry point of the engine fails loudly.
 """
 
 import ctypes
+import warnings
 from functools import lru_cache
 from pathlib import Path
 
@@ -232,13 +233,19 @@ HAS_HIP = _LIB is not None
 
 def _open_host():
     """The compiled host side of the short calls (csrc/host_calls.cpp), bound
-    to the loaded library's entry points; None without it, and the same calls
-    then go through Python."""
+    to the loaded library's entry points; None without it or when it was built
+    for another ABI version (it calls by address, with the signatures of the
+    header it saw), and the same calls then go through Python."""
     if _LIB is None:
         return None
     try:
         from moe_engine import _host_calls
     except ImportError:
+        return None
+    built = getattr(_host_calls, "abi_version", None)
+    if built != ABI_VERSION:
+        warnings.warn(f"{_host_calls.__file__} was built for ABI version {built}, not {ABI_VERSION}: not used",
+                      RuntimeWarning, stacklevel=2)
         return None
     entry_points = (_LIB.mie_paged_decode, _LIB.mie_paged_decode_append, _LIB.mie_paged_decode_plan, _LIB.mie_kv_gather)
     _host_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in entry_points))

@@ -2,10 +2,14 @@
 the usual form of a call and leaves every other to the Python path, which must
 then answer, or raise, as before."""
 
+import sys
+import types
+
 import numpy as np
 import pytest
 import torch
 
+import moe_engine
 from conftest import print_case
 from moe_engine import _native, kv_ops, paged_attention
 from moe_engine.model import BlockAllocator, ModelConfig
@@ -22,6 +26,21 @@ def test_built_and_declines_what_is_not_a_rocm_tensor():
         assert _native.HOST.decode(*args) is None and _native.HOST.gather(*args) is None
     with pytest.raises((TypeError, ValueError)):
         _native.HOST.bind(0, 0, 0, 0)
+
+
+def test_a_module_built_for_another_abi_is_not_bound(monkeypatch):
+    assert _native.HOST.abi_version == _native.ABI_VERSION == _native.lib().mie_abi_version()
+    bound = []
+    for version in (_native.ABI_VERSION - 1, None, _native.ABI_VERSION):
+        stale = types.SimpleNamespace(abi_version=version, __file__="_host_calls.so", bind=lambda *a: bound.append(a))
+        monkeypatch.setitem(sys.modules, "moe_engine._host_calls", stale)
+        monkeypatch.setattr(moe_engine, "_host_calls", stale, raising=False)
+        if version == _native.ABI_VERSION:
+            assert _native._open_host() is stale and len(bound) == 1
+        else:
+            with pytest.warns(RuntimeWarning, match="ABI version"):
+                assert _native._open_host() is None
+            assert not bound
 
 
 def calls(w):
