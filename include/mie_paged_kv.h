@@ -241,6 +241,18 @@ int32_t mie_paged_decode_plan(int32_t batch, int32_t num_heads, int32_t head_dim
                               int32_t* partition_tokens_out,
                               int64_t* workspace_bytes_out);
 
+/*
+ * The plan for sequences whose lengths the caller knows, the longest being
+ * longest_ctx_len (at most max_ctx_len, which sizes the launch): the
+ * partition_tokens to pass to mie_paged_decode (append = 0) or
+ * mie_paged_decode_append (append = 1), 0 where the automatic choice stands,
+ * and the workspace bytes of that call.  A few rows of more than 320 KB of K
+ * and V each are faster in partitions, which a bound alone does not tell.
+ */
+int32_t mie_paged_decode_plan_known(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_size,
+                                    int32_t max_ctx_len, int32_t longest_ctx_len, int32_t append, int32_t dtype,
+                                    int32_t* partition_tokens_out, int64_t* workspace_bytes_out);
+
 /* 1 if mie_paged_decode is built for (head_dim, dtype), else 0. */
 int32_t mie_paged_decode_supported(int32_t head_dim, int32_t dtype);
 
@@ -579,7 +591,10 @@ int32_t mie_moe_decode_block_acc(const void* x, const void* acc, const void* b_o
  * the five-launch form's split context; a call whose decode needs more than
  * workspace_bytes (see mie_paged_decode_plan at batch 1 and max_ctx_len =
  * position + 1) fails with MIE_ERR_WORKSPACE before anything is launched, and
- * the caller initialises the plan again with a larger workspace.  The plan
+ * the caller initialises the plan again with a larger workspace.  Without
+ * counters the length is known: the partitions of mie_paged_decode_plan_known
+ * (batch 1, both lengths position + 1) are taken where the workspace holds
+ * them.  The plan
  * holds pointers only: the caller keeps every buffer alive while the plan is
  * used, and one plan serves calls in stream order.
  *
@@ -609,7 +624,8 @@ int32_t mie_block_decode(const void* plan, const void* x, const int32_t* counter
 /*
  * The number of launches mie_block_decode issues for `position` (the largest
  * position, with counters): 4 (attention fused with out_proj), 5, or 6 when
- * the decode splits the context and merges its partials.  Negative
+ * the decode splits the context and merges its partials (without counters
+ * also where 5 is given and the workspace serves a known length).  Negative
  * (-MIE_ERR_*) for a bad plan or position.  Issues nothing.
  */
 int32_t mie_block_plan_launches(const void* plan, int32_t position);

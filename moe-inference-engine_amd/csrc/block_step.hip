@@ -208,6 +208,7 @@ struct BlockCall {
   const int32_t* ctx_dev;
   int32_t position, max_ctx;
   bool fused;
+  int32_t part;  // the decode's partition_tokens
   int64_t ws_need;
 };
 
@@ -249,10 +250,24 @@ int32_t check_call(const void* plan, const void* x, const int64_t* token_id, con
   c->ws_need = 0;
   if (c->fused) return MIE_OK;
   // The decode's split-context workspace is checked before anything is
-  // launched, so a call that cannot finish changes nothing.
-  const int32_t rc = mie_paged_decode_plan(1, p.num_heads, p.head_dim, p.block_size, c->max_ctx, p.dtype, 0, nullptr,
-                                           &c->ws_need);
+  // launched, so a call that cannot finish changes nothing.  Without counters
+  // the length is known, and partitions that only a known length is given
+  // (mie_paged_decode_plan_known) are taken where the workspace holds them.
+  c->part = 0;
+  int32_t rc = mie_paged_decode_plan(1, p.num_heads, p.head_dim, p.block_size, c->max_ctx, p.dtype, 0, nullptr,
+                                     &c->ws_need);
   if (rc != MIE_OK) return rc;
+  if (!counters && c->ws_need == 0) {
+    int32_t part = 0;
+    int64_t need = 0;
+    rc = mie_paged_decode_plan_known(1, p.num_heads, p.head_dim, p.block_size, c->max_ctx, c->max_ctx, 0, p.dtype,
+                                     &part, &need);
+    if (rc != MIE_OK) return rc;
+    if (part > 0 && need <= p.workspace_bytes && reinterpret_cast<uintptr_t>(p.workspace) % 16 == 0) {
+      c->part = part;
+      c->ws_need = need;
+    }
+  }
   if (c->ws_need > p.workspace_bytes)
     return mie::fail(MIE_ERR_WORKSPACE, "mie_block_decode: position %d needs a %lld-byte workspace, plan has %lld",
                      position, static_cast<long long>(c->ws_need), static_cast<long long>(p.workspace_bytes));
@@ -280,7 +295,7 @@ int32_t launch_call(const BlockCall& c, void* stream) {
   rc = mie_paged_decode(p.q, row, p.head_dim, p.k_pool, p.v_pool, p.pool_stride_block, p.pool_stride_head,
                         p.num_blocks, p.block_table, p.block_table_len, c.ctx_dev, nullptr, c.max_ctx, c.max_ctx, 1,
                         p.num_heads, p.head_dim, p.block_size, p.scale, p.attn, row, p.head_dim, p.dtype,
-                        c.ws_need ? p.workspace : nullptr, c.ws_need, 0, p.dtype, stream);
+                        c.ws_need ? p.workspace : nullptr, c.ws_need, c.part, p.dtype, stream);
   if (rc != MIE_OK) return rc;
   rc = mie_linear_residual(p.attn, p.w_out, p.b_out, c.x, p.h, p.dim, p.dim, p.dtype, stream);
   if (rc != MIE_OK) return rc;

@@ -12,6 +12,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -23,6 +24,7 @@ namespace {
 decltype(&mie_paged_decode) g_decode;
 decltype(&mie_paged_decode_append) g_decode_append;
 decltype(&mie_paged_decode_plan) g_plan;
+decltype(&mie_paged_decode_plan_known) g_plan_known;
 decltype(&mie_kv_gather) g_gather;
 
 // A plain ROCm tensor: no subclass, no functorch or dispatch wrapper, storage
@@ -92,6 +94,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     scale = PyFloat_AS_DOUBLE(a[8]);
   }
   std::vector<int32_t> host;
+  int64_t longest = 0;
   if (a[7] != Py_None) {
     if (!PyList_CheckExact(a[7]) || PyList_GET_SIZE(a[7]) != batch) Py_RETURN_NONE;
     host.resize(batch);
@@ -99,6 +102,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       int64_t c;
       if (!as_int(PyList_GET_ITEM(a[7], b), c) || c < INT32_MIN || c > INT32_MAX) Py_RETURN_NONE;
       host[b] = static_cast<int32_t>(c);
+      longest = std::max(longest, std::min(c, max_len));
     }
   }
   const at::Tensor *kn = nullptr, *vn = nullptr;
@@ -110,9 +114,11 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Py_RETURN_NONE;
     if (kn->strides() != vn->strides()) Py_RETURN_NONE;
   }
-  int32_t part = 0;
+  int32_t part = static_cast<int32_t>(partition);
   int64_t bytes = 0;
-  int32_t rc = g_plan(batch, heads, dim, block, max_len, code, partition, &part, &bytes);
+  int32_t rc = a[7] != Py_None && partition == 0
+                   ? g_plan_known(batch, heads, dim, block, max_len, longest, kn != nullptr, code, &part, &bytes)
+                   : g_plan(batch, heads, dim, block, max_len, code, partition, nullptr, &bytes);
   if (rc != MIE_OK) return PyLong_FromLong(rc);
   at::Tensor out = at::empty({batch, heads, dim}, q->options().requires_grad(false));
   at::Tensor ws;
@@ -134,11 +140,11 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS
   if (kn) {
     rc = g_decode_append(qp, qt[0], qt[1], kp, vp, kt[1], kt[2], blocks, tab, ts, len, hl, 0, max_len, batch, heads,
-                         dim, block, static_cast<float>(scale), op, heads * dim, dim, code, wsp, bytes, partition, knp,
+                         dim, block, static_cast<float>(scale), op, heads * dim, dim, code, wsp, bytes, part, knp,
                          vnp, nb, nh, code, st);
   } else {
     rc = g_decode(qp, qt[0], qt[1], kp, vp, kt[1], kt[2], blocks, tab, ts, len, hl, 0, max_len, batch, heads, dim,
-                  block, static_cast<float>(scale), op, heads * dim, dim, code, wsp, bytes, partition, code, st);
+                  block, static_cast<float>(scale), op, heads * dim, dim, code, wsp, bytes, part, code, st);
   }
   Py_END_ALLOW_THREADS
   if (rc != MIE_OK) return PyLong_FromLong(rc);
@@ -186,14 +192,14 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(decode, decode_append, plan, gather): the entry points' addresses.
+// bind(decode, decode_append, plan, plan_known, gather): the entry points' addresses.
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  void* p[4];
-  if (n != 4) {
-    PyErr_SetString(PyExc_TypeError, "bind takes four addresses");
+  void* p[5];
+  if (n != 5) {
+    PyErr_SetString(PyExc_TypeError, "bind takes five addresses");
     return nullptr;
   }
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 5; ++i) {
     p[i] = PyLong_AsVoidPtr(a[i]);
     if (!p[i]) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null address");
@@ -203,7 +209,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   g_decode = reinterpret_cast<decltype(g_decode)>(p[0]);
   g_decode_append = reinterpret_cast<decltype(g_decode_append)>(p[1]);
   g_plan = reinterpret_cast<decltype(g_plan)>(p[2]);
-  g_gather = reinterpret_cast<decltype(g_gather)>(p[3]);
+  g_plan_known = reinterpret_cast<decltype(g_plan_known)>(p[3]);
+  g_gather = reinterpret_cast<decltype(g_gather)>(p[4]);
   Py_RETURN_NONE;
 }
 

@@ -76,18 +76,10 @@ constexpr int kMinWaves = 4;
 constexpr int kFlatMaxBatch = 512;
 // Workgroup form: one workgroup of kSplitWaves waves per (sequence, head).
 // Each wave reads its slice as a serial chain of tiles (~2 us per tile when
-// latency-bound) and a row's K and V come in at one CU's rate, so the automatic
-// plan takes this form for at most kWgMaxRows (sequence, head) rows when a row
-// is short (max_ctx <= kWgShortCtx: at most 64 tokens per wave, and at most
-// kWgRowBytes of K and V) or when there are enough rows to fill the GPU with
-// workgroups (rows >= kWgMinRows, max_ctx <= kWgMaxCtx).  The line in bytes,
-// workgroup form against 32-token partitions and their merge (us per call,
-// graph replays): 256 KB rows 5.9 / 7.2 (1 x 512, f32 12 x 64), 7.9 / 6.9 (1 x
-// 1000, bf16 12 x 64), 8.8 / 8.2 (5 x 1000, bf16), 7.4 / 8.7 (1 x 256, f32 6 x
-// 128); 375 KB rows 11.0 / 7.8 (1 x 1000, bf16 8 x 96), 10.2 / 9.4 (5 x 512,
-// f32 8 x 96); 500 KB and more 11.6 / 7.6 (1 x 1000, f32 12 x 64), 17.1 / 11.0
-// (5 x 1000, f32 8 x 96), 20.4 / 11.5 (5 x 1000, f32 6 x 128).  From kWgMinRows
-// rows on the rows fill the CUs: 20.5 / 24.5 (21 x 1000, f32 12 x 64).
+// latency-bound), so the automatic plan takes this form for at most
+// kWgMaxRows (sequence, head) rows when every slice is short (max_ctx <=
+// kWgShortCtx: at most 64 tokens per wave) or when there are enough rows to
+// fill the GPU with workgroups (rows >= kWgMinRows, max_ctx <= kWgMaxCtx).
 // Measured on MI355X (per call, graph replays), workgroup form vs the
 // partition plan: 1 x 96 tokens 3.9 vs 6.8 us, 1 x 512 5.4 vs 7.0, 21 x 1000
 // 13.6 vs 16.3, 16 x 4096 33.5 vs 35.3, 64 x 2048 68.7 vs 73.3, 64 x 4096
@@ -104,10 +96,36 @@ constexpr int kSplitWaves = 16;
 constexpr int kWgTileWords = 8;
 constexpr int kWgOrderMax = 1024;  // batches the workgroup form can dispatch longest first
 constexpr int kWgShortCtx = 1024;
-constexpr int64_t kWgRowBytes = 320 << 10;
 constexpr int kWgMinRows = 128;
 constexpr int kWgMaxRows = 1024;
 constexpr int kWgMaxCtx = 8192;
+// Known lengths (plan_known): the workgroup form reads a row's K and V at one
+// CU's rate, so while fewer than kWgMinRows rows share the GPU, rows above
+// kWgRowBytes go to partitions and their merge.  Workgroup form / partitions,
+// us per call in graph replays on MI355X, every sequence at the full length:
+//   256 KB rows  12 rows 6.9 / 6.9 (bf16 1024 x 64), 7.7 / 6.5 (f32 512 x 64),
+//                60 rows 8.7 / 7.4, 120 rows 9.7 / 8.7
+//   320 KB       12 rows 8.4 / 6.5 (f32 640 x 64), 60 9.9 / 8.2, 96 10.5 / 8.9,
+//                120 10.9 / 10.3
+//   384 KB       12 rows 9.5 / 6.5 (f32 768 x 64), 60 11.2 / 8.5, 96 12.2 / 10.3,
+//                120 12.6 / 10.9, 120 (20 x 6 x 128 bf16) 12.8 / 12.7
+//   512 KB       12 rows 11.3 / 6.6 (f32 1024 x 64), 60 13.9 / 8.9, 120 15.6 / 13.0,
+//                120 (20 x 6 x 128 bf16) 15.9 / 16.4
+//   750 KB       8 rows 15.8 / 6.7 (f32 1000 x 96), 40 18.2 / 10.0, 96 20.2 / 15.4,
+//                120 21.0 / 18.3
+// With the append of several sequences the workgroup form stores the rows
+// itself and partitions take a launch before them (about 2.2 us), so their line
+// rises with the rows and ends at kAppendMaxRows (the same columns):
+//   320 KB       24 rows 8.9 / 8.7, 60 10.4 / 10.6, 96 11.0 / 11.8
+//   384 KB       24 rows 10.3 / 9.2, 60 11.7 / 10.9, 80 12.4 / 12.3, 96 12.7 / 13.2
+//   512 KB       24 rows 12.6 / 9.5, 60 14.4 / 11.5, 96 15.4 / 14.1, 120 16.1 / 16.1
+//   640 KB       120 rows 18.8 / 20.9;  750 KB 96 rows 20.7 / 18.3, 120 21.6 / 21.2
+// A bound on unknown lengths keeps the workgroup form: short contexts under it
+// are the faster ones there (bound 1024, f32 12 x 64, real length 64 3.7 / 6.3,
+// 256 4.7 / 6.4, 512 6.5 / 6.4, 1000 10.9 / 6.5).
+constexpr int64_t kWgRowBytes = 320 << 10;
+constexpr int64_t kAppendRowBytes = 768;  // added to the line for every row
+constexpr int kAppendMaxRows = 96;
 
 constexpr int next_pow2(int x) {
   int p = 1;
@@ -908,6 +926,25 @@ struct Plan {
   bool wg;  // workgroup form (one workgroup per (sequence, head), no merge launch)
 };
 
+constexpr int64_t fast_capacity(int32_t block_size) {  // FAST: <= kWindow blocks
+  return static_cast<int64_t>(kWindow) * block_size;
+}
+
+bool fast_block_size(const KernelShape& ks, int32_t block_size) {
+  return is_pow2(block_size) && block_size % ks.tpl == 0;
+}
+
+// The automatic partition of the partition form, in tokens.
+int64_t auto_partition(const KernelShape& ks, int64_t rows, int32_t block_size, int32_t max_ctx) {
+  const int64_t fast_cap = fast_capacity(block_size);
+  int64_t part = ks.tile;
+  while (part < max_ctx && (rows * ((max_ctx + part - 1) / part) > kTargetItems ||
+                            (max_ctx + part - 1) / part > kMaxParts))
+    part <<= 1;
+  if (fast_block_size(ks, block_size) && part > fast_cap && ks.tile <= fast_cap) part = fast_cap;
+  return part;
+}
+
 int32_t plan(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_size, int32_t max_ctx,
              int32_t dtype, int32_t requested, Plan* out) {
   const KernelShape ks = shape_for(dtype, head_dim);
@@ -918,14 +955,12 @@ int32_t plan(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_s
     return mie::fail(MIE_ERR_INVALID,
                      "mie_paged_decode: bad shape batch=%d heads=%d block_size=%d max_ctx=%d", batch,
                      num_heads, block_size, max_ctx);
-  const bool fast_blocks = is_pow2(block_size) && block_size % ks.tpl == 0;
-  const int64_t fast_cap = static_cast<int64_t>(kWindow) * block_size;  // FAST: <= kWindow blocks
+  const bool fast_blocks = fast_block_size(ks, block_size);
+  const int64_t fast_cap = fast_capacity(block_size);
   const int64_t rows = static_cast<int64_t>(batch) * num_heads;
-  const int64_t row_bytes = static_cast<int64_t>(max_ctx) * head_dim * 2 * mie::elt_size(dtype);
   const bool wg = requested == -1 ||
                   (requested == 0 && rows <= kWgMaxRows &&
-                   ((max_ctx <= kWgShortCtx && row_bytes <= kWgRowBytes) ||
-                    (rows >= kWgMinRows && max_ctx <= kWgMaxCtx)));
+                   (max_ctx <= kWgShortCtx || (rows >= kWgMinRows && max_ctx <= kWgMaxCtx)));
   if (requested < -1)
     return mie::fail(MIE_ERR_INVALID, "mie_paged_decode: partition_tokens %d (0 = automatic, -1 = workgroup form)",
                      requested);
@@ -954,11 +989,7 @@ int32_t plan(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_s
                        requested, ks.tile);
     part = requested;
   } else {
-    part = ks.tile;
-    while (part < max_ctx && (rows * ((max_ctx + part - 1) / part) > kTargetItems ||
-                              (max_ctx + part - 1) / part > kMaxParts))
-      part <<= 1;
-    if (fast_blocks && part > fast_cap && ks.tile <= fast_cap) part = fast_cap;
+    part = auto_partition(ks, rows, block_size, max_ctx);
   }
   if (part > (int64_t{1} << 30)) part = int64_t{1} << 30;
   const int64_t max_parts = max_ctx > 0 ? (max_ctx + part - 1) / part : 1;
@@ -969,6 +1000,24 @@ int32_t plan(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_s
   out->fast = fast_blocks && part <= fast_cap;
   out->wg = false;
   return MIE_OK;
+}
+
+// The plan for lengths the caller knows, the longest of them `longest`: the
+// automatic plan, or the partitions to request in its place (*requested; see
+// kWgRowBytes).
+int32_t plan_known(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t block_size, int32_t max_ctx,
+                   int32_t longest, bool append, int32_t dtype, int32_t* requested, Plan* out) {
+  *requested = 0;
+  const int32_t rc = plan(batch, num_heads, head_dim, block_size, max_ctx, dtype, 0, out);
+  if (rc != MIE_OK || !out->wg) return rc;
+  const int64_t rows = static_cast<int64_t>(batch) * num_heads;
+  const int64_t row_bytes = static_cast<int64_t>(longest) * head_dim * 2 * mie::elt_size(dtype);
+  const bool appends = append && batch > 1;
+  if ((appends ? rows > kAppendMaxRows : rows >= kWgMinRows) ||
+      row_bytes <= kWgRowBytes + (appends ? kAppendRowBytes * rows : 0))
+    return rc;
+  *requested = static_cast<int32_t>(auto_partition(shape_for(dtype, head_dim), rows, block_size, max_ctx));
+  return plan(batch, num_heads, head_dim, block_size, max_ctx, dtype, *requested, out);
 }
 
 // wg: the workgroup form; else flat_items > 0: the flat work list with that
@@ -1041,6 +1090,23 @@ extern "C" int32_t mie_paged_decode_plan(int32_t batch, int32_t num_heads, int32
   const int32_t rc = plan(batch, num_heads, head_dim, block_size, max_ctx_len, dtype, partition_tokens, &p);
   if (rc != MIE_OK) return rc;
   if (partition_tokens_out) *partition_tokens_out = p.part;
+  if (workspace_bytes_out) *workspace_bytes_out = p.ws_bytes;
+  return MIE_OK;
+}
+
+extern "C" int32_t mie_paged_decode_plan_known(int32_t batch, int32_t num_heads, int32_t head_dim,
+                                               int32_t block_size, int32_t max_ctx_len, int32_t longest_ctx_len,
+                                               int32_t append, int32_t dtype, int32_t* partition_tokens_out,
+                                               int64_t* workspace_bytes_out) {
+  if (longest_ctx_len < 0 || longest_ctx_len > max_ctx_len)
+    return mie::fail(MIE_ERR_INVALID, "mie_paged_decode_plan_known: longest length %d outside [0, max_ctx_len=%d]",
+                     longest_ctx_len, max_ctx_len);
+  Plan p;
+  int32_t requested = 0;
+  const int32_t rc = plan_known(batch, num_heads, head_dim, block_size, max_ctx_len, longest_ctx_len, append != 0,
+                                dtype, &requested, &p);
+  if (rc != MIE_OK) return rc;
+  if (partition_tokens_out) *partition_tokens_out = requested;
   if (workspace_bytes_out) *workspace_bytes_out = p.ws_bytes;
   return MIE_OK;
 }

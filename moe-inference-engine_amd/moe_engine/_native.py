@@ -100,6 +100,11 @@ _SIGNATURES = {
         _i32,
         [_i32, _i32, _i32, _i32, _i32, _i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i64)],
     ),
+    "mie_paged_decode_plan_known": (
+        _i32,
+        [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32,  # batch, heads, head_dim, block_size, max, longest, append, dtype
+         ctypes.POINTER(_i32), ctypes.POINTER(_i64)],
+    ),
     "mie_paged_decode_supported": (_i32, [_i32, _i32]),
     "mie_qkv_append": (
         _i32,
@@ -247,7 +252,8 @@ def _open_host():
         warnings.warn(f"{_host_calls.__file__} was built for ABI version {built}, not {ABI_VERSION}: not used",
                       RuntimeWarning, stacklevel=2)
         return None
-    entry_points = (_LIB.mie_paged_decode, _LIB.mie_paged_decode_append, _LIB.mie_paged_decode_plan, _LIB.mie_kv_gather)
+    entry_points = (_LIB.mie_paged_decode, _LIB.mie_paged_decode_append, _LIB.mie_paged_decode_plan,
+                    _LIB.mie_paged_decode_plan_known, _LIB.mie_kv_gather)
     _host_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in entry_points))
     return _host_calls
 
@@ -342,5 +348,21 @@ def decode_plan(batch, num_heads, head_dim, block_size, max_ctx_len, dtype, part
             ctypes.byref(part), ctypes.byref(ws),
         ),
         "mie_paged_decode_plan",
+    )
+    return part.value, ws.value
+
+
+@lru_cache(maxsize=1024)
+def decode_plan_known(batch, num_heads, head_dim, block_size, max_ctx_len, longest, append, dtype):
+    """(partition_tokens, workspace_bytes) for lengths known on the host, the
+    longest of them `longest`: what to request of the decode (0 = automatic)."""
+    part = _i32(0)
+    ws = _i64(0)
+    check(
+        lib().mie_paged_decode_plan_known(
+            batch, num_heads, head_dim, block_size, max_ctx_len, longest, append, dtype_code(dtype),
+            ctypes.byref(part), ctypes.byref(ws),
+        ),
+        "mie_paged_decode_plan_known",
     )
     return part.value, ws.value

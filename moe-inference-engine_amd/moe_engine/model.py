@@ -1071,6 +1071,14 @@ class TransformerMoEBlock(nn.Module):
                                                        x.data_ptr()), "mie_block_plan_set_embedding")
 
         init(None)
+        if lib.mie_block_plan_launches(plan, 0) != 4:
+            # Without the fused attention, contexts the decode keeps in one
+            # launch under a bound are split where the length is known (eager
+            # steps), if the plan's workspace holds the partials.
+            need = max(_native.decode_plan_known(1, heads, head_dim, block_size, n, n, False, dtype)[1]
+                       for n in range(64, 1025, 64))
+            if need:
+                init(torch.empty(need, dtype=torch.uint8, device=device))
 
         def run(fn, arg, cache, position, stream):
             """One call of the plan.  A longer context splits into partitions:

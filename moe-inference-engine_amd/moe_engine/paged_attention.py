@@ -108,10 +108,11 @@ def decode_layer(
             raise ValueError("block tables must be [batch, max_blocks] with unit inner stride")
         bt_stride = block_tables.stride(0)
     host_lens = None
+    longest = None  # of the lengths, where the host knows them
     if context_lens is None:
         if context_len is None:
             raise ValueError("pass context_len or context_lens")
-        max_context_len = int(context_len)
+        longest = max_context_len = int(context_len)
         ctx_ptr = 0
     else:
         if max_context_len is None:
@@ -125,6 +126,7 @@ def decode_layer(
             if len(context_lens_host) != batch:
                 raise ValueError("context_lens_host must hold one length per sequence")
             host_lens = (ctypes.c_int32 * batch)(*(int(c) for c in context_lens_host))
+            longest = min(max((0, *host_lens)), int(max_context_len))
     if out_dtype is None:
         out_dtype = q.dtype if out is None else out.dtype
     if out is None:
@@ -133,9 +135,15 @@ def decode_layer(
         raise ValueError("out must be [batch, heads, head_dim] with unit inner stride")
     if scale is None:
         scale = 1.0 / math.sqrt(head_dim)
-    _, ws_bytes = _native.decode_plan(
-        batch, heads, head_dim, block_size, int(max_context_len), q.dtype, int(partition_tokens)
-    )
+    partition_tokens = int(partition_tokens)
+    if longest is not None and longest >= 0 and partition_tokens == 0:
+        partition_tokens, ws_bytes = _native.decode_plan_known(
+            batch, heads, head_dim, block_size, int(max_context_len), longest, k_new is not None, q.dtype
+        )
+    else:
+        _, ws_bytes = _native.decode_plan(
+            batch, heads, head_dim, block_size, int(max_context_len), q.dtype, partition_tokens
+        )
     ws = _workspace(ws_bytes, q.device)
     if k_new is not None or v_new is not None:
         if k_new is None or v_new is None:
@@ -154,7 +162,7 @@ def decode_layer(
                 batch, heads, head_dim, block_size,
                 float(scale),
                 out.data_ptr(), out.stride(0), out.stride(1), _native.dtype_code(out.dtype),
-                _native.ptr(ws), ws_bytes, int(partition_tokens),
+                _native.ptr(ws), ws_bytes, partition_tokens,
                 k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1),
                 _native.dtype_code(q.dtype), _native.stream_of(q),
             ),
@@ -170,7 +178,7 @@ def decode_layer(
             batch, heads, head_dim, block_size,
             float(scale),
             out.data_ptr(), out.stride(0), out.stride(1), _native.dtype_code(out.dtype),
-            _native.ptr(ws), ws_bytes, int(partition_tokens),
+            _native.ptr(ws), ws_bytes, partition_tokens,
             _native.dtype_code(q.dtype), _native.stream_of(q),
         ),
         "mie_paged_decode",
@@ -215,8 +223,8 @@ def decode(q: torch.Tensor, cache, layer_idx: int, context_len: int) -> torch.Te
         # Lean path for the engine's own calls: the launch constants are the
         # allocator's, the plan is cached, one C call.
         layer_bytes, sblk, shead, code = launch
-        part, ws_bytes = _native.decode_plan(
-            1, num_heads, head_dim, allocator.block_size, context_len, q.dtype, 0
+        part, ws_bytes = _native.decode_plan_known(
+            1, num_heads, head_dim, allocator.block_size, context_len, context_len, False, q.dtype
         )
         out = torch.empty((1, num_heads, 1, head_dim), dtype=q.dtype, device=q.device)
         ws = _workspace(ws_bytes, q.device)
@@ -229,7 +237,7 @@ def decode(q: torch.Tensor, cache, layer_idx: int, context_len: int) -> torch.Te
             1, num_heads, head_dim, allocator.block_size,
             1.0 / math.sqrt(head_dim),
             out.data_ptr(), num_heads * head_dim, head_dim, code,
-            _native.ptr(ws), ws_bytes, 0,
+            _native.ptr(ws), ws_bytes, part,
             code, _native.stream_of(q),
         )
         if rc:

@@ -63,6 +63,52 @@ def test_decode_plan_rejects_bad_partition_and_unbuilt_shapes():
         _native.decode_plan(1, 12, 64, 16, 4096, torch.bfloat16, -2)
 
 
+@pytest.mark.parametrize("heads,head_dim", [(12, 64), (8, 96), (6, 128), (1, 256), (64, 8)])
+@pytest.mark.parametrize("batch", [1, 2, 5, 16])
+def test_a_bound_up_to_1024_tokens_needs_no_workspace(batch, heads, head_dim):
+    """The automatic plan knows a bound only; callers rely on 0 bytes there."""
+    import torch
+
+    for dtype in (torch.float32, torch.bfloat16):
+        for bound in (1, 427, 1000, 1024):
+            part, ws = _native.decode_plan(batch, heads, head_dim, 16, bound, dtype, 0)
+            assert part >= bound and ws == 0
+
+
+def test_known_lengths_take_partitions_where_rows_are_few_and_large():
+    import torch
+
+    known = lambda *a: _native.decode_plan_known(*a)  # noqa: E731
+    f32, bf16 = torch.float32, torch.bfloat16
+    # 320 KB of K and V per row: 640 tokens of 64 float32 values.
+    assert known(1, 12, 64, 16, 640, 640, False, f32) == (0, 0)
+    part, ws = known(1, 12, 64, 16, 641, 641, False, f32)
+    assert part > 0 and ws == _native.decode_plan(1, 12, 64, 16, 641, f32, part)[1] > 0
+    # The longest length decides, the bound sizes the workspace.
+    assert known(1, 12, 64, 16, 1024, 640, False, f32) == (0, 0)
+    part, ws = known(1, 12, 64, 16, 1024, 641, False, f32)
+    assert part > 0 and ws == _native.decode_plan(1, 12, 64, 16, 1024, f32, part)[1]
+    assert known(1, 12, 64, 16, 1024, 1024, False, bf16) == (0, 0)
+    assert known(1, 8, 96, 16, 1024, 1024, False, bf16)[0] > 0
+    # From 128 rows on the rows fill the GPU.
+    assert known(10, 12, 64, 16, 1000, 1000, False, f32)[0] > 0
+    assert known(11, 12, 64, 16, 1000, 1000, False, f32) == (0, 0)
+    # With the append of a batch the workgroup form saves a launch: the line
+    # rises by 768 bytes a row and ends at 96 rows.  One sequence is not a batch.
+    assert known(1, 12, 64, 16, 641, 641, True, f32)[0] > 0
+    assert known(2, 12, 64, 16, 676, 676, True, f32) == (0, 0)
+    assert known(2, 12, 64, 16, 677, 677, True, f32)[0] > 0
+    assert known(8, 12, 64, 16, 784, 784, True, f32) == (0, 0)
+    assert known(8, 12, 64, 16, 785, 785, True, f32)[0] > 0
+    assert known(9, 12, 64, 16, 1024, 1024, True, f32) == (0, 0)
+    # Past 1024 tokens the automatic plan stands, whatever it is.
+    for shape in ((1, 12, 64, 16, 2048), (64, 12, 64, 16, 8192)):
+        assert known(*shape, shape[-1], True, bf16) == (0, _native.decode_plan(*shape, bf16, 0)[1])
+    for longest in (-1, 11):
+        with pytest.raises((RuntimeError, ValueError), match="longest"):
+            known(1, 12, 64, 16, 10, longest, False, f32)
+
+
 def test_decode_plan_workgroup_form_needs_no_workspace():
     import torch
 
