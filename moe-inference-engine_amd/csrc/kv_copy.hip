@@ -107,10 +107,20 @@ struct GatherArgs {
 // grid = (ceil(length * vecs_per_row / (PER * kCopyThreads)), num_heads, 2 [K, V]).
 // A thread moves PER vectors, kCopyThreads apart, all their table reads and
 // then all their loads in flight together: with one vector a wave spends its
-// life in one dependent chain (table, load, store).  The pool is read once
-// (non-temporal); the output is for the attention that follows and is stored
-// through the caches.  8192 tokens x 12 heads x 64 bf16 (50 MB moved) on
-// MI355X: 12.95 -> 11.66 us.
+// life in one dependent chain (table, load, store).  With several the pool is
+// read around the caches (non-temporal), which pays where K and V of a call
+// are tens of MB; with one they are small and through the caches is faster.
+// Graph replays over 12 layers on MI355X, 12 heads x 64 bf16, us per layer
+// into one destination / into one per layer:
+//                1 vector      1, non-temporal   2              4
+//   1024 tokens  2.75 / 2.74    2.86 / 2.92      3.11 /  3.05   3.13 /  3.13
+//   2048         3.66 / 3.65    3.92 / 3.92      4.11 /  4.12   4.25 /  4.26
+//   4096         5.56 / 6.69    6.44 / 6.38      5.81 /  5.84   6.04 /  6.06
+//   8192        10.54 / 12.12  10.63 / 11.15    10.35 / 10.87   9.80 / 10.10
+//  16384        17.79 / 20.72  18.16 / 19.68    18.78 / 19.21  17.35 / 18.98
+// (a replay finds pools of up to 4096 tokens in the last-level cache; with it
+// emptied before each call 4096 tokens take 9.2, 9.0, 8.4 and 8.7, 8192 13.1,
+// 13.4, 13.4 and 13.0.)
 template <int VB, int PER>
 __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
   using T = typename Raw<VB>::T;
@@ -137,8 +147,9 @@ __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
     const uint32_t t = min(tok[p], static_cast<uint32_t>(a.length) - 1u);
     const uint32_t slot = t - a.bs.div(t) * a.bs.d;
     const bool ok = phys[p] >= 0 && phys[p] < a.num_blocks;
-    v[p] = load_once<T>(pool + (ok ? phys[p] : 0) * a.pool_sblk + static_cast<int64_t>(slot) * a.row_bytes +
-                        static_cast<int64_t>(vec) * VB);
+    const char* src = pool + (ok ? phys[p] : 0) * a.pool_sblk + static_cast<int64_t>(slot) * a.row_bytes +
+                      static_cast<int64_t>(vec) * VB;
+    v[p] = PER > 1 ? load_once<T>(src) : *reinterpret_cast<const T*>(src);
     if (!ok) tok[p] = 0xffffffffu;
   }
 #pragma unroll
@@ -150,11 +161,11 @@ __global__ __launch_bounds__(kCopyThreads) void kv_gather_kernel(GatherArgs a) {
 }
 
 template <int VB>
-void launch_gather(const GatherArgs& a, dim3 grid, bool four, hipStream_t st) {
-  if (four) {
-    kv_gather_kernel<VB, 4><<<grid, kCopyThreads, 0, st>>>(a);
-  } else {
-    kv_gather_kernel<VB, 1><<<grid, kCopyThreads, 0, st>>>(a);
+void launch_gather(const GatherArgs& a, dim3 grid, int per, hipStream_t st) {
+  switch (per) {
+    case 4: kv_gather_kernel<VB, 4><<<grid, kCopyThreads, 0, st>>>(a); break;
+    case 2: kv_gather_kernel<VB, 2><<<grid, kCopyThreads, 0, st>>>(a); break;
+    default: kv_gather_kernel<VB, 1><<<grid, kCopyThreads, 0, st>>>(a); break;
   }
 }
 
@@ -300,16 +311,21 @@ extern "C" int32_t mie_kv_gather(const void* k_pool, const void* v_pool, int64_t
     return mie::fail(MIE_ERR_INVALID, "mie_kv_gather: length * row vectors exceeds 2^31");
 
   // Four vectors per thread where that still makes 1024 workgroups (four per
-  // CU); the last workgroup's indices stay in FastDiv's range.
-  const int64_t wide = (total + 4 * kCopyThreads - 1) / (4 * kCopyThreads);
-  const bool four = wide * num_heads * 2 >= 1024 && total < (int64_t{1} << 31) - 4 * kCopyThreads;
-  const dim3 grid(static_cast<uint32_t>(four ? wide : (total + kCopyThreads - 1) / kCopyThreads), num_heads, 2);
+  // CU; 12 heads x 64 bf16 from 5377 tokens on), or two where that makes 1152
+  // (from 3009 on; at 2700 tokens one takes 4.3 us, two 4.75, at 3000 both
+  // 5.0); the last workgroup's indices stay in FastDiv's range.
+  auto groups = [&](int per) { return (total + per * kCopyThreads - 1) / (per * kCopyThreads); };
+  auto fills = [&](int per, int64_t least) {
+    return groups(per) * num_heads * 2 >= least && total < (int64_t{1} << 31) - per * kCopyThreads;
+  };
+  const int per = fills(4, 1024) ? 4 : fills(2, 1152) ? 2 : 1;
+  const dim3 grid(static_cast<uint32_t>(groups(per)), num_heads, 2);
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (vb) {
-    case 16: launch_gather<16>(a, grid, four, st); break;
-    case 8: launch_gather<8>(a, grid, four, st); break;
-    case 4: launch_gather<4>(a, grid, four, st); break;
-    default: launch_gather<2>(a, grid, four, st); break;
+    case 16: launch_gather<16>(a, grid, per, st); break;
+    case 8: launch_gather<8>(a, grid, per, st); break;
+    case 4: launch_gather<4>(a, grid, per, st); break;
+    default: launch_gather<2>(a, grid, per, st); break;
   }
   return mie::check_launch("mie_kv_gather");
 }

@@ -178,3 +178,19 @@ def test_config3_append_and_gather_round_trip(context):
         gk, gv = kv_ops.gather(k_pool, v_pool, layer, table_dev, context + 1)
         assert torch.equal(gk[0].view(torch.int16), truth_k[layer].view(torch.int16))
         assert torch.equal(gv[0].view(torch.int16), truth_v[layer].view(torch.int16))
+
+
+@pytest.mark.parametrize("heads,head_dim,dtype,length", [
+    (12, 64, torch.bfloat16, 3008), (12, 64, torch.bfloat16, 3009), (12, 64, torch.bfloat16, 5376),
+    (12, 64, torch.bfloat16, 5377), (512, 8, torch.float32, 255), (512, 8, torch.float32, 257),
+    (512, 8, torch.float32, 513), (1, 256, torch.float64, 4097)])
+def test_gather_at_the_switches_between_vectors_per_thread(heads, head_dim, dtype, length):
+    """One, two and four vectors per thread, on both sides of the switches and
+    with tails; exact against the indexed rebuild."""
+    blocks = -(-length // 16) + 2
+    pools = [torch.randn(1, blocks, heads, 16, head_dim, device="cuda").to(dtype) for _ in range(2)]
+    table = torch.randperm(blocks)[: -(-length // 16)].to(torch.int32).to("cuda")
+    print_case("gather switches", heads, head_dim, dtype, length)
+    got = kv_ops.gather(*pools, 0, table, length)
+    for g, p in zip(got, pools):
+        assert torch.equal(g[0], p[0, table.long()].transpose(0, 1).reshape(heads, -1, head_dim)[:, :length])
