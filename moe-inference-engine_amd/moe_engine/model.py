@@ -71,6 +71,29 @@ _GLOBAL_MODULE_HOOKS = (nn.modules.module._global_forward_hooks, nn.modules.modu
 _PROMPT_MAX_TOKENS = 1 << 19
 
 
+def _prompt_attention_pays(tokens: int, dim: int, dtype: torch.dtype) -> bool:
+    """Whether the HIP prompt attention beats library products around
+    PyTorch's attention, whose ten host operations take about 78 us however
+    short the prompt.  Its 16-query tiles read K and V more often than a long
+    prompt or a wide model affords in bfloat16; in float32 the crossing comes
+    with the attention itself.  Few tokens of very wide layers are the
+    weights' reads, where the library's products are the faster ones.
+
+    Measured on MI355X, us per layer, HIP / PyTorch:
+      bfloat16, operations 8 T d^2 + 2 T^2 d: 12 x 64 1024 tokens (6.4e9) 42 /
+      80, 1792 (13e9) 68 / 81, 2048 (16e9) 89 / 90, 4096 240 / 162; 24 x 32 1792
+      (13e9) 74 / 78, 2048 (16e9) 87 / 81; 16 x 64 1280 (14e9) 68 / 79, 1536
+      (18e9) 81 / 80; 32 x 64 384 (13e9) 53 / 80, 640 (23e9) 84 / 80; 32 x 128
+      16 50 / 79, 192 (26e9) 90 / 83; 64 x 128 16 128 / 121.
+      float32, 2 T^2 d: 12 x 64 16384 tokens (4.1e11) 5315 / 6198, 32768
+      (1.6e12) 22964 / 21876; 6 x 128 16384 6337 / 6498; 32 x 128 4096 (1.4e11)
+      5054 / 6051, 8192 (5.5e11) 14290 / 14059; 32 x 64 16 tokens 36 / 78; 32 x
+      128 16 104 / 80, 64 134 / 107, 256 290 / 293."""
+    if dtype == torch.float32:
+        return 2 * tokens * tokens * dim <= 5 * 10**11 and (dim <= 3072 or tokens >= 256)
+    return 8 * tokens * dim * dim + 2 * tokens * tokens * dim <= 15 * 10**9 and dim <= 4096
+
+
 def _plain_module(module) -> bool:
     """Whether calling the module runs its class's forward and nothing else."""
     return not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
@@ -480,11 +503,12 @@ class CachedAttention(_TracksReplacement, nn.Module):
         )
 
     def prompt_supported(self, x, cache, layer_idx) -> bool:
-        """Whether a prompt x at position 0 can take the HIP prompt attention
+        """Whether a prompt x at position 0 takes the HIP prompt attention
         (paged_attention.prefill): a paged cache on a ROCm device in a mode
         that may run the direct kernels, one float32 or bfloat16 sequence whose
-        projections match the pools, unmodified modules, and nothing recorded
-        or transformed (_native.plain_inference)."""
+        projections match the pools, sizes it is faster for
+        (_prompt_attention_pays), unmodified modules, and nothing recorded or
+        transformed (_native.plain_inference)."""
         alloc = getattr(cache, "allocator", None)
         if (
             alloc is None
@@ -495,6 +519,7 @@ class CachedAttention(_TracksReplacement, nn.Module):
             or x.dim() != 3
             or x.shape[0] != 1
             or not 0 < x.shape[1] <= _PROMPT_MAX_TOKENS
+            or not _prompt_attention_pays(x.shape[1], x.shape[2], x.dtype)
             or not _native.plain_inference(x)
         ):
             return False

@@ -173,3 +173,23 @@ def test_supported_widths_are_the_entry_points(monkeypatch, dim, hidden):
     taken = fused_moe.prefill_supported(torch.zeros(1, 2, dim), *parts, 1)
     assert taken == (max(dim, hidden) <= 1 << 20)
     assert taken == (_native.lib().mie_moe_prefill_workspace(2, 1, 1, dim, hidden, 0) > 0)
+
+
+@pytest.mark.parametrize("heads,head_dim,dtype,tokens,taken", [
+    (12, 64, torch.bfloat16, 1024, True), (12, 64, torch.bfloat16, 1900, True), (12, 64, torch.bfloat16, 2048, False),
+    (24, 32, torch.bfloat16, 2048, False), (4, 32, torch.bfloat16, 8192, False), (16, 64, torch.bfloat16, 1536, False),
+    (32, 64, torch.bfloat16, 384, True), (32, 64, torch.bfloat16, 640, False), (64, 128, torch.bfloat16, 16, False),
+    (12, 64, torch.float32, 16384, True), (12, 64, torch.float32, 32768, False), (32, 64, torch.float32, 2, True),
+])
+def test_prompts_take_the_launches_where_they_are_faster(cache, heads, head_dim, dtype, tokens, taken):
+    dim = heads * head_dim
+    config = ModelConfig(num_layers=1, hidden_dim=dim, num_heads=heads)
+    allocator = BlockAllocator(config, 1, 16, "cpu", dtype, "auto")
+    allocator._launch = cache.allocator._launch
+    with torch.device("meta"):
+        att = CachedAttention(dim, heads).to(dtype)
+    # Parameters of the right shape without their memory filled in.
+    att = att.to_empty(device="cpu")
+    with torch.no_grad():
+        x = torch.empty(1, tokens, dim, dtype=dtype)
+        assert att.prompt_supported(x, allocator.new_cache(), 0) is taken
