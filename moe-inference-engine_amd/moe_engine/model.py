@@ -762,6 +762,19 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
     # Prefill of at most this many tokens runs dense-masked on the GPU.
     DENSE_PREFILL_MAX_TOKENS = 512
 
+    # bfloat16 prompts of more operations (the selected experts' 4 T k d h) per
+    # expert than this run as library products, whose host waits (about 135 us
+    # an expert) are small by then.  Measured on MI355X, us per layer, grouped
+    # kernels / per-expert PyTorch: 768 x 3072, 8 experts, top-2, 32768 tokens
+    # (7.7e10 per expert) 1717 / 2038, 65536 3227 / 2855; 2048 x 8192 4096 (6.9e10)
+    # 1292 / 1650, 8192 2445 / 2222; 4096 x 14336 1500 (8.8e10) 1766 / 1964, 3000
+    # 3100 / 2529; 4 experts, 768 x 3072, 16384 (7.7e10) 851 / 950, 32768 1636 /
+    # 1432; one expert, 768 x 2048, 4096 (2.6e10) 93 / 208, 16384 (1.0e11) 366 /
+    # 333; 64 experts, top-6, 2048 x 1408, 32768 (3.5e10) 8436 / 12243.  float32:
+    # faster up to 65536 tokens and 4096 x 14336, all sizes measured but one
+    # (4096 x 14336, 32 tokens: 798 / 761).
+    GROUPED_PREFILL_BF16_OPS = 80 * 10**9
+
     def uses_dense_prefill(self, x: torch.Tensor, *, decode: bool) -> bool:
         """Multi-token (or mode 'auto'/'direct' prefill) float32 input on a
         ROCm device with the canonical layout takes _forward_dense; everything
@@ -827,7 +840,7 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
 
     def uses_grouped_prefill(self, x: torch.Tensor, *, decode: bool) -> bool:
         """Prompts at inference take the grouped HIP kernels (fused_moe.prefill)
-        where these apply: float32 or bfloat16 on a ROCm device with the
+        where these apply and are faster (GROUPED_PREFILL_BF16_OPS): float32 or bfloat16 on a ROCm device with the
         canonical layout.  Gradients, autocast, forward-mode AD, functorch
         transforms, tracing and dispatch modes keep the PyTorch paths, and so
         do experts whose modules were changed, where those would run them
@@ -838,6 +851,9 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
             self.mode != "reference"
             and not (decode and tokens == 1)
             and tokens >= 1
+            and (x.dtype != torch.bfloat16
+                 or 4 * tokens * self.top_k * self.dim * self.hidden_dim
+                 <= self.GROUPED_PREFILL_BF16_OPS * self.num_experts)
             and _native.plain_inference(x)
             and fused_moe.prefill_supported(x, self.router.weight, s["w1"], s["b1"], s["w2"], s["b2"], self.top_k)
             and s["w1"].shape[0] == self.num_experts

@@ -193,3 +193,16 @@ def test_prompts_take_the_launches_where_they_are_faster(cache, heads, head_dim,
     with torch.no_grad():
         x = torch.empty(1, tokens, dim, dtype=dtype)
         assert att.prompt_supported(x, allocator.new_cache(), 0) is taken
+
+
+@pytest.mark.parametrize("experts,top_k,dtype,tokens,taken", [
+    (1, 1, torch.bfloat16, 39062500, True), (1, 1, torch.bfloat16, 39062501, False),
+    (8, 2, torch.bfloat16, 156250000, True), (8, 2, torch.bfloat16, 156250001, False),
+    (8, 2, torch.float32, 156250001, True)])
+def test_moe_prompts_take_the_launches_where_they_are_faster(monkeypatch, experts, top_k, dtype, tokens, taken):
+    """16 x 32 experts: 80e9 operations per expert, 4 T k 16 x 32."""
+    monkeypatch.setattr(_native, "is_rocm_device", lambda t: True)
+    layer = MoEFeedForward(16, 32, experts, top_k).to(dtype).eval()
+    with torch.no_grad():
+        x = torch.zeros(1, 1, 16, dtype=dtype).expand(1, tokens, 16)
+        assert layer.uses_grouped_prefill(x, decode=False) is taken
