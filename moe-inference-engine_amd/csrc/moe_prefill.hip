@@ -607,7 +607,10 @@ struct Plan {
 Plan make_plan(int32_t tokens, int32_t E, int32_t top_k, int32_t dim, int32_t hidden, int elt) {
   Plan p;
   const int64_t slots = static_cast<int64_t>(tokens) * top_k;
-  p.few = slots <= 20 * static_cast<int64_t>(E);
+  // float32 sums of fewer than 16 products stay in float32 instructions too:
+  // what the split leaves out of a product (gemm_split.h) is only made up for by
+  // the longer sums' own rounding.
+  p.few = slots <= 20 * static_cast<int64_t>(E) || (elt == 4 && std::min(dim, hidden) < 16);
   const int bn = p.few ? 32 : 64, kb = p.few ? 1024 : 128;
   p.rows = p.few ? E : static_cast<int32_t>(slots / 64 + std::min<int64_t>(E, slots));
   // W2 has few column tiles, so its K is split.  bfloat16 and few rows wait on

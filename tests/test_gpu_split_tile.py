@@ -110,3 +110,38 @@ def test_infinities_are_float32s():
         for got, want in ((keys, k), (values, v)):
             assert torch.equal(got[0, :, 399].reshape(-1).double(), want)  # infinities of the same signs
             assert got[0, :, :399].isfinite().all()
+
+
+@pytest.mark.parametrize("rows", [21, 64, 200])
+@pytest.mark.parametrize("dim", [4, 8, 12])
+def test_short_sums_are_float32s(rows, dim):
+    """Sums of fewer than 16 products keep each product whole.  One value per
+    row and column product, the GELU of values above 16 is the value, and W2
+    picks one of them: the output is the float32 product, bit for bit."""
+    layer = one_expert(dim, 16)
+    up, _, down = layer.experts[0].net
+    x = torch.zeros(1, rows, dim, device="cuda")
+    at = torch.arange(rows, device="cuda") % dim
+    value = torch.rand(rows, device="cuda") * 4 + 4
+    with torch.no_grad():
+        x[0, torch.arange(rows, device="cuda"), at] = value
+        up.weight.copy_(torch.rand(16, dim, device="cuda") * 4 + 4)
+        up.bias.zero_()
+        down.weight.copy_(torch.eye(16, device="cuda")[:dim])
+        down.bias.zero_()
+        print_case("short sums", rows, dim)
+        assert layer.uses_grouped_prefill(x, decode=False)
+        got = layer(x)[0]
+        assert torch.equal(got, value[:, None] * up.weight[:dim, at].t())
+        # A short second product: one hidden value in 4 or 8.
+        layer = one_expert(32, dim)
+        up, _, down = layer.experts[0].net
+        x = torch.zeros(1, rows, 32, device="cuda")
+        x[..., 0] = 16 + torch.arange(rows, device="cuda")  # whole numbers: the first product is exact
+        up.weight.zero_()
+        up.weight[dim - 1, 0] = 1
+        up.bias.zero_()
+        down.weight.copy_(torch.rand(32, dim, device="cuda") + 1)
+        down.bias.zero_()
+        got = layer(x)[0]
+        assert torch.equal(got, x[0, :, :1] * down.weight[:, dim - 1])
