@@ -212,7 +212,18 @@ int32_t mie_paged_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,
  * or partitions of one sequence, the decode kernel stores the rows and takes
  * the new token's score and value from the rows it loaded, without reading
  * them back; otherwise the append runs as its own launch before the decode, on
- * the same stream.  A sequence with ctx_b = 0 gets no append and a zero output; a new
+ * the same stream.
+ *
+ * The block that a sequence's new token goes to must be that sequence's own:
+ * no other sequence of the call may have it among the blocks it attends to.
+ * Blocks that hold earlier tokens only may be shared.  In the workgroup form
+ * another sequence's workgroup would read such a block while this one's
+ * stores into it, in no order.  Sequences that do share it (the last tokens
+ * of one sequence at several lengths) are appended by mie_kv_append and then
+ * attended by mie_paged_decode, or, with a batch of two and more, by this
+ * entry with partition_tokens > 0, where the append is always its own launch.
+ *
+ * A sequence with ctx_b = 0 gets no append and a zero output; a new
  * token whose block id is outside the pool is not stored and its output is
  * NaN.  Other arguments and limits as mie_paged_decode.
  */

@@ -1239,10 +1239,11 @@ int32_t decode_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h, const
   if (k_new) {
     if (p.wg || (flat_items > 0 && batch == 1)) {
       // The decode kernel stores the rows and attends to the new token itself
-      // (1 x 2048 bf16: two launches instead of three).  In partitions for one
-      // sequence only: several may name the same blocks (the last tokens of one
-      // sequence at several lengths), and each must then see what the others
-      // append.
+      // (1 x 2048 bf16: two launches instead of three).  With several sequences
+      // in the workgroup form each owns the block its token goes to (the
+      // entry's contract); partitions requested for several keep the append in
+      // a launch before them, so there they may share it (the last tokens of
+      // one sequence at several lengths).
       a.k_new = static_cast<const char*>(k_new);
       a.v_new = static_cast<const char*>(v_new);
       a.new_sb = new_stride_b;

@@ -76,7 +76,11 @@ def decode_layer(
     With k_new / v_new ([B, H, D], the pools' dtype) the step's append is
     fused in: each sequence's new token is its last context token, stored at
     position ctx_b - 1 through the table and attended to (mie_paged_decode_append;
-    no launch of its own in the workgroup form or for one sequence).
+    no launch of its own in the workgroup form or for one sequence).  The block
+    that token goes to must be the sequence's own: sequences that share it (the
+    last tokens of one sequence at several lengths) are appended by
+    kv_ops.append and then decoded, or given partition_tokens > 0, where the
+    append of several sequences is a launch before the decode.
     """
     lib = _native.lib()
     if q.dim() != 3:

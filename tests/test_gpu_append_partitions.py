@@ -89,6 +89,40 @@ def test_rows_of_one_sequence_see_each_others_tokens():
         assert torch.equal(rows, new.transpose(0, 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens", [[698, 699, 700], [15, 17, 16], [700, 700]])
+def test_rows_that_share_their_last_blocks_in_both_documented_ways(lens, dtype):
+    """Rows of one sequence at several lengths: appended by their own launch and
+    then decoded in every form, and by the fused entry with partitions
+    requested.  Oracle: float64 attention over the pools with every row's token
+    in (for two rows of one length, the same token)."""
+    w = make_workload([max(lens)], num_heads=12, head_dim=64, block_size=16, dtype=dtype, seed=5)
+    rows = len(lens)
+    tables = w.block_tables.expand(rows, -1).contiguous()
+    q, k_new, v_new = (torch.randn(rows, 12, 64, device="cuda").to(dtype) for _ in range(3))
+    if len(set(lens)) == 1:
+        k_new, v_new = (t[:1].expand(rows, -1, -1).contiguous() for t in (k_new, v_new))
+    context = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    pools = [t.clone() for t in (w.k_pool, w.v_pool)]
+    print_case("shared last block", lens, dtype)
+    kv_ops.append(*pools, 0, k_new[:, :, None], v_new[:, :, None], tables, positions=context - 1)
+    k, v = (p[0, tables[0].long()].transpose(0, 1).reshape(12, -1, 64).double() for p in pools)
+    want = torch.stack([
+        (torch.softmax((k[:, :n] * q[b].double()[:, None]).sum(-1) / 8, -1)[..., None] * v[:, :n]).sum(1)
+        for b, n in enumerate(lens)])
+    # float32 sums of N(0, 1) values, as the decode tests' 1e-5; bfloat16 adds the output's rounding, 2^-9 of
+    # values below 4.
+    limit = 1e-5 if dtype == torch.float32 else 1e-2
+    for part in (0, -1, 256):
+        got = paged_attention.decode_batched(q, *pools, 0, tables, context, max(lens), partition_tokens=part,
+                                             context_lens_host=lens)
+        assert (got.double() - want).abs().max().item() <= limit
+    got = paged_attention.decode_batched(q, w.k_pool, w.v_pool, 0, tables, context, max(lens), partition_tokens=256,
+                                         context_lens_host=lens, k_new=k_new, v_new=v_new)
+    assert (got.double() - want).abs().max().item() <= limit
+    assert torch.equal(w.k_pool, pools[0]) and torch.equal(w.v_pool, pools[1])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16, torch.float64])
 @pytest.mark.parametrize("heads,head_dim,block_size,length", [(12, 64, 16, 8192), (12, 64, 16, 4097), (40, 24, 7, 3001),
                                                               (12, 64, 16, 1)])
