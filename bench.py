@@ -12,7 +12,8 @@ layer over the whole batch: the batched append of each sequence's new token
 full contexts - one mie_paged_decode_append launch (`--unfused`: the append
 launch, then the decode launch).  Inputs are resident in HBM before timing.
 
-Printed: ONE JSON line.  `value` is algorithmic bytes (attention + append) per
+Printed: ONE JSON line, short enough to be read back from the end of a log
+(LINE_LIMIT).  `value` is algorithmic bytes (attention + append) per
 step over the measured step time, in GB/s.  `roofline` is the dominant
 launch: its algorithmic bytes (attention + append fused; attention alone with
 `--unfused`) over its average duration from HIP events recorded on the launch
@@ -20,9 +21,10 @@ stream: one event pair around the timed loop of back-to-back fused launches
 (region / steps), or events around every attention call with `--unfused`.
 `cpu_baseline` times the oracle's gather + scaled_dot_product_attention path
 (the reference's CPU path) on a bounded sample of the same workload.
-`secondary` carries the per-token end-to-end decode latency (config 1, and
-its shape in bfloat16) and the single-layer, append/gather and long-context
-figures (configs 2, 3, 5).
+`per_token_decode_ms` is the metric's second half, the end-to-end decode
+latency (config 1).  The secondary figures (each round of config 1, its shape
+in bfloat16, the single-layer, append/gather and long-context workloads of
+configs 2, 3, 5) go to stderr, one line `[bench] secondary.<name> <JSON>` each.
 """
 
 import argparse
@@ -41,6 +43,7 @@ PEAK_HBM_GBS = 8000.0  # MI355X HBM3E
 SECONDARY_NAMES = ("launch_floor", "round_latency", "north_star_64x8192", "config2_single_layer", "config3_append_gather",
                    "config5_long_context", "fused_moe_decode", "config1_e2e_decode", "config1_context_sweep",
                    "config1_attention_micro", "config1_bf16_decode")
+LINE_LIMIT = 4000  # characters of the printed line
 TRAFFIC_FILE = ROOT / "profiles" / "paged_decode_config4_traffic.json"
 
 
@@ -773,6 +776,13 @@ def main():
             torch.cuda.empty_cache()
         add_floor_fractions(secondary)
 
+    for name, figures in secondary.items():
+        log(f"secondary.{name}", json.dumps(figures))
+    print(result_line(args, main_res, cpu, secondary, total_tokens), flush=True)
+
+
+def result_line(args, main_res, cpu, secondary, total_tokens) -> str:
+    """The printed JSON line."""
     line = {
         "metric": METRIC,
         "value": round(main_res["value"], 2),
@@ -804,16 +814,15 @@ def main():
         "cpu_baseline": cpu,
         "per_token_decode_ms": per_token_decode_ms(secondary.get("config1_e2e_decode"),
                                                    secondary.get("config1_context_sweep")),
-        "secondary": secondary,
     }
-    print(json.dumps(line), flush=True)
+    return json.dumps(line)
 
 
 def per_token_decode_ms(e2e, sweep=None):
     """The metric's second half: BASELINE config 1's median greedy decode
     latency per token for each system, from the config1_e2e_decode secondary
     (None when it did not run), with the paging-cost intervals of the e2e
-    rounds and of the context sweep at every context."""
+    rounds and the context sweep's medians."""
     if not e2e or "summary" not in e2e:
         return None
     out = {system: s["decode_median_ms"] for system, s in e2e["summary"].items()}
@@ -835,13 +844,8 @@ def per_token_decode_ms(e2e, sweep=None):
         out["parity"] = {k: parity[k] for k in ("engine_cache", "max_abs_logit_diff", "max_rel_logit_diff",
                                                 "greedy_tokens_compared", "first_greedy_mismatch",
                                                 "tokens_equal_reference_engine") if k in parity}
-    if sweep and "paging_cost_ms" in sweep:
-        out["context_sweep"] = {
-            "median_step_ms": sweep["median_step_ms"],
-            "paging_cost_ms": sweep["paging_cost_ms"],
-            "rounds": sweep["rounds"],
-            "placement_sampled": sweep["placement_sampled"],
-        }
+    if sweep and "median_step_ms" in sweep:
+        out["context_sweep"] = {"median_step_ms": sweep["median_step_ms"], "rounds": sweep.get("rounds")}
     out["rounds"] = e2e.get("rounds")
     out["placement_sampled"] = e2e.get("placement_sampled")
     out["workload"] = ("BASELINE config 1: 12 layers, d 768, 12 x 64 heads, top-2 of 8, FFN 2048, vocab 50257, "
