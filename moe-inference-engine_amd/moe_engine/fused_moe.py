@@ -235,6 +235,7 @@ def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int
     num_experts, dim = router_weight.shape
     hidden = w1.shape[1]
     vec = 16 // x.element_size()
+    plain = _native.PLAIN_TENSORS
     return (
         x.shape[-1] == dim
         and 0 < num_experts <= MAX_EXPERTS
@@ -244,8 +245,8 @@ def prefill_supported(x: torch.Tensor, router_weight, w1, b1, w2, b2, top_k: int
         and dim % vec == 0
         and hidden % vec == 0
         and all(
-            type(t) in _native.PLAIN_TENSORS and t.shape == shape and t.dtype == dtype and t.device == device
-            and t.is_contiguous() and t.data_ptr() % 16 == 0
+            t.shape == shape and t.dtype is dtype and t.device == device and t.is_contiguous() and type(t) in plain
+            and t.data_ptr() % 16 == 0
             for t, shape in (
                 (router_weight, (num_experts, dim)),
                 (w1, (num_experts, hidden, dim)),

@@ -100,11 +100,14 @@ def _plain_module(module) -> bool:
                 or any(_GLOBAL_MODULE_HOOKS))
 
 
-def _like(t, shape, x) -> bool:
-    """A parameter the kernels can read beside x: a plain tensor (a wrapper
-    subclass has no memory of its own), this shape, x's dtype and device,
-    contiguous, 16-byte aligned."""
-    return (type(t) in _native.PLAIN_TENSORS and t.shape == shape and t.dtype == x.dtype and t.device == x.device
+_PLAIN_TENSORS = _native.PLAIN_TENSORS
+
+
+def _like(t, shape, dtype, device) -> bool:
+    """A parameter the kernels can read beside an activation of this dtype and
+    device: a plain tensor (a wrapper subclass has no memory of its own), this
+    shape, contiguous, 16-byte aligned."""
+    return (type(t) in _PLAIN_TENSORS and t.shape == shape and t.dtype is dtype and t.device == device
             and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
@@ -523,7 +526,7 @@ class CachedAttention(_TracksReplacement, nn.Module):
             or not _native.plain_inference(x)
         ):
             return False
-        pool, dim = alloc.k_pool, x.shape[2]
+        pool, dim, dtype, device = alloc.k_pool, x.shape[2], x.dtype, x.device
         out = self._modules.get("out_proj")
         params = self._parameters
         # Pruning, weight norm and parametrizations take the names out of the
@@ -537,13 +540,13 @@ class CachedAttention(_TracksReplacement, nn.Module):
             and (alloc.num_heads, alloc.head_dim) == (self.num_heads, self.head_dim)
             and self.num_heads * self.head_dim == dim
             and 0 <= layer_idx < pool.shape[0]
-            and x.dtype == pool.dtype
-            and x.device == pool.device
-            and _like(w_in, (3 * dim, dim), x)
-            and (b_in is None or _like(b_in, (3 * dim,), x))
-            and _like(out.weight, (dim, dim), x)
-            and (out.bias is None or _like(out.bias, (dim,), x))
-            and paged_attention.prefill_supported(self.num_heads, self.head_dim, x.dtype)
+            and dtype is pool.dtype
+            and device == pool.device
+            and _like(w_in, (3 * dim, dim), dtype, device)
+            and (b_in is None or _like(b_in, (3 * dim,), dtype, device))
+            and _like(out.weight, (dim, dim), dtype, device)
+            and (out.bias is None or _like(out.bias, (dim,), dtype, device))
+            and paged_attention.prefill_supported(self.num_heads, self.head_dim, dtype)
         )
 
     def _prompt(self, x, cache, layer_idx, norm=None, residual=None):
@@ -819,6 +822,7 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
         if any(_GLOBAL_MODULE_HOOKS):
             return False
         s = self._expert_storage
+        parameter = nn.Parameter  # registered tensors that are plain ones
         # Addresses of the next expert's parameters, and the steps between experts.
         at = [s[name].data_ptr() for name in ("w1", "b1", "w2", "b2")]
         step = [s[name].stride(0) * s[name].element_size() for name in ("w1", "b1", "w2", "b2")]
@@ -830,10 +834,11 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
             if type(up) is not Linear or type(act) is not nn.GELU or type(down) is not Linear or act.approximate != "none":
                 return False
             for m in (expert, net, up, act, down):
-                if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                own = m.__dict__
+                if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
                     return False
             for i, t in enumerate((*up._parameters.values(), *down._parameters.values())):  # weight, bias each
-                if type(t) not in _native.PLAIN_TENSORS or t.data_ptr() != at[i]:
+                if type(t) is not parameter or t.data_ptr() != at[i]:
                     return False
                 at[i] += step[i]
         return True
@@ -977,11 +982,11 @@ class TransformerMoEBlock(nn.Module):
         if not (type(att) is CachedAttention and type(moe) is MoEFeedForward and _plain_module(att)
                 and _plain_module(moe) and att.prompt_supported(x, cache, layer_idx)):
             return None
-        dim = x.shape[2]
+        dim, dtype, device = x.shape[2], x.dtype, x.device
         for norm in (an, mn):
             if not (type(norm) is LayerNorm and _plain_module(norm) and tuple(norm.normalized_shape) == (dim,)
-                    and norm.weight is not None and _like(norm.weight, (dim,), x)
-                    and (norm.bias is None or _like(norm.bias, (dim,), x))):
+                    and norm.weight is not None and _like(norm.weight, (dim,), dtype, device)
+                    and (norm.bias is None or _like(norm.bias, (dim,), dtype, device))):
                 return None
         if not moe.uses_grouped_prefill(x, decode=False):
             return None
