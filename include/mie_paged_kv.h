@@ -396,7 +396,9 @@ int32_t mie_moe_decode_block(const void* x, const void* ln_weight, const void* l
  * x and out [tokens, dim], the weights in canonical
  * layouts as for mie_moe_decode, all 16-byte aligned; dim and hidden multiples
  * of 4 (float32) or 8 (bfloat16), at most 64 experts and top_k 8.  out must
- * not alias x.  Only experts that a token selected are read.  workspace holds
+ * not alias x.  With more than about 20 rows per expert only the experts that
+ * a token selected are read; with fewer the first 2048 bytes of every expert's
+ * rows may be too.  workspace holds
  * mie_moe_prefill_workspace bytes (negative: the shape is not supported);
  * nothing in it needs clearing.  Four launches per 4096 tokens.
  */

@@ -27,7 +27,10 @@
 //   3. moe_prompt_w2: partial sums of W2_e h over one K split.
 //   4. moe_prompt_combine: the splits' sum, bias, weight and expert-order sum.
 // The work follows the routing: top_k / E of what running every expert on
-// every token takes, at any skew, and an expert without tokens is not read.
+// every token takes, at any skew.  Row tiles (many rows per expert) do not read
+// an expert without tokens; the few-rows form has the first two windows (2048
+// bytes) of every expert's rows of W1, and of its share of W2's, in flight
+// before the routing is known.
 //
 // Bounds: at few tokens the experts' bytes (768 x 2048 x 8 float32: 101 MB),
 // at many the matrix cores (float32 instructions: 153 TFLOP/s; the split form

@@ -448,11 +448,27 @@ void launch_direct(const LinearArgs& a, hipStream_t st) {
 // workgroups over the 256 CUs takes `first`, each further one, overlapping,
 // `more` (us at K 768 with the epilogue; every tile scales with K alike).  Split tiles
 // win from about 320 x 2304 on; below, the small tile's rounds are few and the
-// shortest (300 tokens: a layer in 35 us with it, 37 with 48x64 split).  Measured on MI355X, us, 32x32 / 64x48 in float32
-// instructions, then split 32x64 / 48x64 / 64x64 / 64x128, products alone: 1000 x 2304 44 / 42
-// - 40 / 31 / 33 / 39; 1000 x 768 16 / 16 - 16 / 17 / 18 / 25; 333 x 2304 20 / 26
-// - 16 / 17 / 17 / 27; 2048 x 3072 103 / 99 - 86 / 77 / 63 / 60; 62 x 2304 8 / 16
-// - 13 / 16 / 17 / 24.
+// shortest (300 tokens: a layer in 35 us with it, 37 with 48x64 split).
+//
+// Measured on MI355X, us, products alone at K 768 (graph replays); float32:
+//   rows x n (32x32 tiles)  direct 16x16  32x16  32x32 | split 32x64  48x64  64x64  64x128
+//     32 x 2304    (72)         7.8   6.7    8.1        13.3   17.4   18.2   25.4
+//    128 x 768     (96)         7.9   6.7    7.9        13.3   17.6   18.6   26.1
+//     48 x 2304   (144)         8.0  10.0    8.1        13.3   17.5   18.4   25.9
+//     62 x 2304   (144)        10.4  10.7    8.1        13.3   17.7   18.5   26.2
+//     96 x 2304   (216)        13.5  11.0    8.2        13.4   17.7   18.7   26.3
+//    300 x 768    (240)        13.2  10.9    8.2        13.4   17.7   18.7   26.2
+//    333 x 2304   (792)        35.1  29.7   20.0        16.9   18.0   19.0   28.9
+//   1000 x 768    (768)        34.0  26.9   16.5        17.1   18.5   19.5   26.7
+//   1000 x 2304  (2304)        97.1  74.3   42.5        41.5   31.0   33.5   39.5
+//   2048 x 3072  (6144)           -     -    103          86     77     63     60
+// bfloat16, the last three columns 32x32, 32x64, 64x48 staged:
+//     32 x 2304    (72)         4.7   4.2   |  4.5   6.0   7.2
+//    128 x 768     (96)         4.7   4.2   |  4.5   6.0   7.2
+//     62 x 2304   (144)         6.1   5.9   |  4.6   6.1   7.3
+//    300 x 768    (240)         7.5   6.1   |  4.6   6.1   7.3
+//    333 x 2304   (792)        19.0  16.7   |  8.2   7.9   9.2
+//   1000 x 2304  (2304)        50.8  41.2   | 15.8  13.8  15.3
 //
 // bfloat16: the staged tile whose last round wastes least - rounds x tile area;
 // on a tie the smallest tile while it makes at most 512 workgroups (more of

@@ -8,8 +8,10 @@ attention's two of at most 1100, so 4 * sqrt(1100) * 2^-24 = 7.9e-6; in
 bfloat16 at most four stored values round by 2^-9 on the way (q or k or v,
 the attention's output, the projection's, the residual sum), and rounded
 scores move the softmax by as much again: 8 * 2^-9 / 2 = 7.8e-3.  Lengths sit
-at the edges of the kernels' tiles (16 and 32 queries, 32 keys per wave, 128
-per workgroup step, 256 for the switch to 32 queries) and of blocks.
+at the edges of the attention's tiles (16 queries, 32 keys per wave, 128 per
+workgroup step), of the projections' forms (12 x 64: QKV leaves the direct tiles
+after 32 tokens, the output projection takes larger direct tiles from 65 and
+leaves them after 160) and of blocks.
 """
 
 import math
@@ -68,6 +70,7 @@ def attention(dim, heads, dtype, seed=0):
         (12, 64, 16, 1), (12, 64, 16, 15), (12, 64, 16, 17), (12, 64, 16, 62), (12, 64, 16, 129),
         (12, 64, 16, 256), (12, 64, 16, 257), (12, 64, 16, 1024), (8, 96, 16, 33), (8, 96, 16, 300),
         (2, 32, 7, 100), (3, 32, 16, 513), (4, 128, 32, 65), (8, 128, 32, 1000), (1, 64, 1, 31),
+        (12, 64, 16, 32), (12, 64, 16, 33), (12, 64, 16, 64), (12, 64, 16, 65), (12, 64, 16, 160), (12, 64, 16, 161),
     ],
 )
 def test_prompt_matches_float64(heads, head_dim, block_size, tokens, dtype):
