@@ -103,16 +103,20 @@ constexpr int kWgMaxCtx = 8192;
 // CU's rate, so while fewer than kWgMinRows rows share the GPU, rows above
 // kWgRowBytes go to partitions and their merge.  Workgroup form / partitions,
 // us per call in graph replays on MI355X, every sequence at the full length:
-//   256 KB rows  12 rows 6.9 / 6.9 (bf16 1024 x 64), 7.7 / 6.5 (f32 512 x 64),
-//                60 rows 8.7 / 7.4, 120 rows 9.7 / 8.7
+//   192 KB rows  12 rows 6.2 / 6.9 (bf16 768 x 64), 6.4 / 6.5 (f32 384 x 64),
+//                60 7.2 / 7.3, 120 7.8 / 8.4
+//   256 KB       12 rows 6.9 / 6.9 (bf16 1024 x 64), 7.7 / 6.5 (f32 512 x 64),
+//                60 8.7 / 7.4, 120 9.7 / 8.7, 120 (20 x 6 x 128 f32) 9.5 / 11.0
 //   320 KB       12 rows 8.4 / 6.5 (f32 640 x 64), 60 9.9 / 8.2, 96 10.5 / 8.9,
-//                120 10.9 / 10.3
+//                120 10.9 / 10.3, 120 (20 x 6 x 128 bf16) 11.2 / 12.1
 //   384 KB       12 rows 9.5 / 6.5 (f32 768 x 64), 60 11.2 / 8.5, 96 12.2 / 10.3,
 //                120 12.6 / 10.9, 120 (20 x 6 x 128 bf16) 12.8 / 12.7
 //   512 KB       12 rows 11.3 / 6.6 (f32 1024 x 64), 60 13.9 / 8.9, 120 15.6 / 13.0,
 //                120 (20 x 6 x 128 bf16) 15.9 / 16.4
 //   750 KB       8 rows 15.8 / 6.7 (f32 1000 x 96), 40 18.2 / 10.0, 96 20.2 / 15.4,
 //                120 21.0 / 18.3
+// One line for all row counts: a few rows gain from about 240 KB on, 90 to 127
+// rows of many sequences lose up to 1.5 us below 320 KB.
 // With the append of several sequences the workgroup form stores the rows
 // itself and partitions take a launch before them (about 2.2 us), so their line
 // rises with the rows and ends at kAppendMaxRows (the same columns):
