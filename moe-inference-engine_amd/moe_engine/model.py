@@ -819,34 +819,43 @@ class MoEFeedForward(_TracksReplacement, nn.Module):
         """Whether running the experts' modules would compute exactly what the
         canonical storages describe: unmodified Expert modules without hooks,
         whose parameters are the storages' slices."""
-        if any(_GLOBAL_MODULE_HOOKS):
-            return False
+        experts = self.experts._modules
         s = self._expert_storage
-        parameter = nn.Parameter  # registered tensors that are plain ones
+        if any(_GLOBAL_MODULE_HOOKS) or len(experts) != s["w1"].shape[0]:
+            return False
+        linear, gelu, sequential, parameter = Linear, nn.GELU, nn.Sequential, nn.Parameter
         # Addresses of the next expert's parameters, and the steps between experts.
-        at = [s[name].data_ptr() for name in ("w1", "b1", "w2", "b2")]
-        step = [s[name].stride(0) * s[name].element_size() for name in ("w1", "b1", "w2", "b2")]
-        for expert in self.experts._modules.values():
+        at_w1, at_b1, at_w2, at_b2 = (s[name].data_ptr() for name in ("w1", "b1", "w2", "b2"))
+        step_w1, step_b1, step_w2, step_b2 = (
+            s[name].stride(0) * s[name].element_size() for name in ("w1", "b1", "w2", "b2"))
+        for expert in experts.values():
             net = expert._modules.get("net")
-            if type(expert) is not Expert or type(net) is not nn.Sequential or len(net._modules) != 3:
+            if type(expert) is not Expert or type(net) is not sequential or len(net._modules) != 3:
                 return False
             up, act, down = net._modules.values()
-            if type(up) is not Linear or type(act) is not nn.GELU or type(down) is not Linear or act.approximate != "none":
+            if type(up) is not linear or type(act) is not gelu or type(down) is not linear or act.approximate != "none":
                 return False
             for m in (expert, net, up, act, down):
                 own = m.__dict__
                 if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
                     return False
-            for i, t in enumerate((*up._parameters.values(), *down._parameters.values())):  # weight, bias each
-                if type(t) is not parameter or t.data_ptr() != at[i]:
-                    return False
-                at[i] += step[i]
+            # By name: a Linear may have further parameters that its forward does not read.
+            w1, b1 = up._parameters.get("weight"), up._parameters.get("bias")
+            w2, b2 = down._parameters.get("weight"), down._parameters.get("bias")
+            if not (type(w1) is type(b1) is type(w2) is type(b2) is parameter
+                    and w1.data_ptr() == at_w1 and b1.data_ptr() == at_b1
+                    and w2.data_ptr() == at_w2 and b2.data_ptr() == at_b2):
+                return False
+            at_w1 += step_w1
+            at_b1 += step_b1
+            at_w2 += step_w2
+            at_b2 += step_b2
         return True
 
     def uses_grouped_prefill(self, x: torch.Tensor, *, decode: bool) -> bool:
         """Prompts at inference take the grouped HIP kernels (fused_moe.prefill)
-        where these apply and are faster (GROUPED_PREFILL_BF16_OPS): float32 or bfloat16 on a ROCm device with the
-        canonical layout.  Gradients, autocast, forward-mode AD, functorch
+        where these apply and are faster (GROUPED_PREFILL_BF16_OPS): float32
+        or bfloat16 on a ROCm device with the canonical layout.  Gradients, autocast, forward-mode AD, functorch
         transforms, tracing and dispatch modes keep the PyTorch paths, and so
         do experts whose modules were changed, where those would run them
         (_forward_dense reads the storages too)."""

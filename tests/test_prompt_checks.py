@@ -206,3 +206,20 @@ def test_moe_prompts_take_the_launches_where_they_are_faster(monkeypatch, expert
     with torch.no_grad():
         x = torch.zeros(1, 1, 16, dtype=dtype).expand(1, tokens, 16)
         assert layer.uses_grouped_prefill(x, decode=False) is taken
+
+
+def test_experts_with_further_parameters_and_fewer_experts():
+    """A parameter a Linear's forward does not read changes nothing; a bias by
+    another name, a storage with more experts than the layer has, do."""
+    layer = MoEFeedForward(16, 32, 3, 2)
+    layer.experts[1].net[2].register_parameter("scale", torch.nn.Parameter(torch.ones(16)))
+    assert layer._experts_are_plain()
+    layer.experts[2].net[0].register_parameter("scale", torch.nn.Parameter(torch.ones(16)))
+    assert layer._experts_are_plain()
+    bias = layer.experts[0].net[0].bias
+    layer.experts[0].net[0].bias = None
+    layer.experts[0].net[0].register_parameter("shift", bias)
+    assert not layer._experts_are_plain()
+    layer = MoEFeedForward(16, 32, 3, 2)
+    del layer.experts[2]
+    assert not layer._experts_are_plain()
