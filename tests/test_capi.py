@@ -104,6 +104,15 @@ def test_known_lengths_take_partitions_where_rows_are_few_and_large():
     # Past 1024 tokens the automatic plan stands, whatever it is.
     for shape in ((1, 12, 64, 16, 2048), (64, 12, 64, 16, 8192)):
         assert known(*shape, shape[-1], True, bf16) == (0, _native.decode_plan(*shape, bf16, 0)[1])
+    # What it returns can be requested, for every built shape.
+    for head_dim in (4, 8, 16, 32, 64, 96, 128, 256):
+        for dtype in (f32, bf16):
+            for heads in (1, 7, 40):
+                for block_size in (1, 7, 16, 64):
+                    part, ws = known(1, heads, head_dim, block_size, 1024, 1024, True, dtype)
+                    large = 1024 * head_dim * 2 * dtype.itemsize > 320 << 10
+                    assert (part > 0) == large
+                    assert ws == _native.decode_plan(1, heads, head_dim, block_size, 1024, dtype, part)[1]
     for longest in (-1, 11):
         with pytest.raises((RuntimeError, ValueError), match="longest"):
             known(1, 12, 64, 16, 10, longest, False, f32)
